@@ -50,10 +50,12 @@ enum {
     RLN_ERR_MEMORY = -7          /* device allocation failed */
 };
 
-/* Precision of the squared-difference (diff2) kernels. */
+/* Precision of the squared-difference (diff2) kernels. Both run the coarse cross term Re(P conj(CTF*s*X_t)) on the
+ * FP32 matrix units with FP32 accumulation, the particle's own power in FP64; RLN_PREC_SPLIT_BF16 allows BF16 hi+lo
+ * products for it, which the FP32 contraction is at least as fast as. */
 enum {
-    RLN_PREC_PLAIN_FP32 = 0,     /* direct sum of |CTF*s*P - X_t|^2 in FP32 (fallback path) */
-    RLN_PREC_SPLIT_BF16 = 1      /* coarse cross term Re(P conj(CTF*s*X_t)) on MFMA, BF16 hi+lo, FP32 accumulation */
+    RLN_PREC_PLAIN_FP32 = 0,
+    RLN_PREC_SPLIT_BF16 = 1
 };
 
 /* Options of one E-step run; names follow MlOptimiser / MlModel / HealpixSampling members. */

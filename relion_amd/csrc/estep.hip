@@ -188,15 +188,15 @@ struct Engine {
     bool model_set = false;
     bool coarse_valid = false;
     // constant tables
-    DevBuf d_frames_c, d_frames_f, d_proj_c;
-    DevBuf d_pf, d_zero_row;                        // split-BF16 coarse projections (FP32 complex), a zero row
-    DevBuf d_ehi, d_elo;                            // split-BF16 translation phases [NT][Kp/2]
-    DevBuf d_wc, d_ctf2, d_ynorm;                   // split-BF16 particle rows per chunk (group layout)
-    DevBuf d_grp, d_exg;                            // pixel groups (row, x0); x phases with rows padded to xs4
-    int Kp = 0;                                     // contraction length: 8 * groups, multiple of 32
-    int G = 0, xs4 = 0;                             // pixel groups with weight; coarse row length padded to 4
+    DevBuf d_frames_c, d_frames_f;
+    // coarse pass (k_coarse_lattice): projections and a zero row, particle rows per chunk, the pixel layout's groups
+    // and row pairs, phases of the lattice's y and x shifts and its columns
+    DevBuf d_pf, d_zero_row, d_wc, d_ctf2, d_ynorm, d_grp, d_pairs_c, d_ytab, d_xtab, d_cols, d_tile_of;
+    int Kc = 0;                                     // complex slots per projection
+    int n_pairs_c = 0, n_xsteps = 0;                // row pairs; steps of the longest row
+    int mshift = 0, col_tiles = 1;                  // positive shifts of the lattice; column tiles
     DevBuf d_q_c, d_q_f, d_minv_w, d_mresol, d_xa_shell;
-    DevBuf d_ex_c, d_ey_c, d_ex_f, d_ey_f, d_tr_ix, d_tr_iy, d_over_x, d_over_y;
+    DevBuf d_ex_f, d_ey_f, d_tr_ix, d_tr_iy, d_over_x, d_over_y;
     DevBuf d_vols, d_bp_ptrs;
     std::vector<double> over_x, over_y;  // [NT*4] pixels
     // coarse translations on their lattice: distinct x and y values (Angstrom) and each translation's indices
@@ -209,7 +209,7 @@ struct Engine {
     DevBuf d_meta_f, d_meta_d, d_meta_ll;
     DevBuf d_or_off, d_or_cnt, d_or_proj, d_or_prior, d_or_frame, d_or_class, d_or_dir, d_tr_prior;
     DevBuf d_oc_off;  // per-particle offsets of per-orientation state
-    DevBuf d_ctfq, d_yq, d_tiles;
+    DevBuf d_tiles;
     DevBuf d_diff2, d_weight, d_mask, d_stats_c, d_stats_f;
     DevBuf d_npairs, d_njobs, d_nchunks, d_pair_off, d_job_off, d_chunk_off, d_pairs, d_jobs, d_chunk_job,
         d_chunk_first;
@@ -359,6 +359,95 @@ int launch_check(const char *what) {
 
 }  // namespace
 
+// Columns of the coarse kernel's x contraction (kernels.h): the lattice's x shifts on the 16 lanes of each column tile,
+// and the column tile of every translation. A lattice of at most 256 translations, the points of a disc, has at most 9
+// positive shifts on an axis.
+static int lattice_columns(Engine &e) {
+    const int m = ((int)e.tr_ux.size() - 1) / 2;
+    if ((int)e.tr_ux.size() != 2 * m + 1 || e.tr_uy.size() != e.tr_ux.size() || m > 9)
+        RLN_FAIL(RLN_ERR_ARG, "unexpected translation lattice of %d x %d shifts", (int)e.tr_ux.size(),
+                 (int)e.tr_uy.size());
+    e.mshift = m;
+    e.col_tiles = m > rlnk::kColShift ? 2 : 1;
+    // translation index of (column, ty = 0) and the column's half height
+    std::vector<rlnk::CoarseColumn> by_ix(2 * m + 1, rlnk::CoarseColumn{0, -1});
+    for (int t = 0; t < e.NT; ++t) {
+        rlnk::CoarseColumn &c = by_ix[e.tr_cix[t]];
+        const int iy = e.tr_ciy[t] - m;
+        if (iy == 0) c.t0 = t;
+        c.half = std::max(c.half, iy);
+    }
+    std::vector<rlnk::CoarseColumn> cols(16 * e.col_tiles + 1, rlnk::CoarseColumn{0, -1});
+    std::vector<int> tile_of(e.NT, 0);
+    for (int ct = 0; ct < e.col_tiles; ++ct)
+        for (int n = 0; n < 16; ++n) {
+            const int k = rlnk::kColShift * ct + (n & 7) + 1;
+            if (k <= m) cols[16 * ct + n] = by_ix[n < 8 ? m + k : m - k];
+        }
+    if (m == rlnk::kColShift)
+        cols[16] = by_ix[m];
+    else
+        cols[16 * (e.col_tiles - 1) + 7] = by_ix[m];
+    for (int t = 0; t < e.NT; ++t) {
+        const int ix = std::abs(e.tr_cix[t] - m);
+        tile_of[t] = ix == 0 ? e.col_tiles - 1 : (ix - 1) / rlnk::kColShift;
+    }
+    RLN_TRY(upload(e.d_cols, cols, e.stream));
+    return upload(e.d_tile_of, tile_of, e.stream);
+}
+
+// Pixel layout of the coarse contraction and its phase tables (kernels.h), from the coarse sqrt(Minvsigma2 / 2).
+static int coarse_layout(Engine &e, const std::vector<float> &qc) {
+    const int s = e.igc.s, xs = e.igc.xs, m = e.mshift;
+    const double N = e.cfg.ori_size, px = e.cfg.pixel_size;
+    std::vector<int2> grp, pairs;
+    std::vector<float> ytab;
+    e.n_xsteps = 0;
+    // cos and -sin of 2 pi k shift / N, the phase reduced in turns before the trigonometry
+    auto phase = [&](double k, double shift) {
+        double turns = -k * shift / N;
+        turns -= std::nearbyint(turns);
+        return make_float2((float)cos(2. * kPi * turns), (float)sin(2. * kPi * turns));
+    };
+    for (int y = 0; y <= s / 2; ++y) {
+        const bool minus = y > 0 && s - y >= xs;
+        int xmax = -1;
+        for (int x = 0; x < xs; ++x)
+            if (qc[(size_t)y * xs + x] != 0.f || (minus && qc[(size_t)(s - y) * xs + x] != 0.f)) xmax = x;
+        const int steps = (xmax + 8) / 8;
+        if (steps == 0) continue;
+        for (int j = 0; j < steps; ++j) {
+            grp.push_back(make_int2(y, 8 * j));
+            grp.push_back(make_int2(minus ? s - y : -1, 8 * j));
+        }
+        pairs.push_back(make_int2(steps, minus ? 1 : 0));
+        for (int k = 0; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).x);
+        for (int k = 1; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).y);
+        e.n_xsteps = std::max(e.n_xsteps, steps);
+    }
+    e.n_pairs_c = (int)pairs.size();
+    e.Kc = 8 * (int)grp.size();
+    std::vector<float2> xtab((size_t)e.col_tiles * e.n_xsteps * 64);
+    for (int ct = 0; ct < e.col_tiles; ++ct)
+        for (int j = 0; j < e.n_xsteps; ++j)
+            for (int l = 0; l < 64; ++l) {
+                const int n = l & 15, x = 8 * j + 2 * (l >> 4), k = rlnk::kColShift * ct + (n & 7) + 1;
+                float2 v = make_float2(0.f, 0.f);
+                if (k <= m) {
+                    const float2 p0 = phase(x, e.tr_ux[m + k] / px), p1 = phase(x + 1, e.tr_ux[m + k] / px);
+                    v = n < 8 ? make_float2(p0.x, p1.x) : make_float2(p0.y, p1.y);
+                } else if (n == 7 && ct == e.col_tiles - 1) {
+                    v = make_float2(1.f, 1.f);  // tx = 0
+                }
+                xtab[((size_t)ct * e.n_xsteps + j) * 64 + l] = v;
+            }
+    RLN_TRY(upload(e.d_grp, grp, e.stream));
+    RLN_TRY(upload(e.d_pairs_c, pairs, e.stream));
+    RLN_TRY(upload(e.d_ytab, ytab, e.stream));
+    RLN_TRY(upload(e.d_xtab, xtab, e.stream));
+    return upload(e.d_zero_row, std::vector<float2>(std::max(e.Kc, 1), make_float2(0.f, 0.f)), e.stream);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Engine setup
 // ------------------------------------------------------------------------------------------------
@@ -416,12 +505,7 @@ static int engine_init(Engine &e, const rln_estep_config &cfg) {
         }
     RLN_TRY(upload(e.d_frames_c, fc, e.stream));
     RLN_TRY(upload(e.d_frames_f, ff, e.stream));
-    // translations: coarse phase rows per translation, fine rows per distinct sub-shift
-    std::vector<double> cx(e.NT), cy(e.NT);
-    for (int t = 0; t < e.NT; ++t) {
-        cx[t] = e.grid.tx[t] / cfg.pixel_size;
-        cy[t] = e.grid.ty[t] / cfg.pixel_size;
-    }
+    // translations: the coarse lattice, fine phase rows per distinct sub-shift
     {
         std::map<double, int> mx, my;
         for (int t = 0; t < e.NT; ++t) {
@@ -445,11 +529,8 @@ static int engine_init(Engine &e, const rln_estep_config &cfg) {
             e.tr_ciy[t] = my[e.grid.ty[t]];
         }
     }
+    RLN_TRY(lattice_columns(e));
     std::vector<float2> rows;
-    phase_rows(cx, e.sc, false, cfg.ori_size, rows);
-    RLN_TRY(upload(e.d_ex_c, rows, e.stream));
-    phase_rows(cy, e.sc, true, cfg.ori_size, rows);
-    RLN_TRY(upload(e.d_ey_c, rows, e.stream));
     e.over_x.resize((size_t)e.NT * 4);
     e.over_y.resize((size_t)e.NT * 4);
     for (int t = 0; t < e.NT; ++t) e.grid.oversampled_translations(t, &e.over_x[t * 4], &e.over_y[t * 4]);
@@ -493,17 +574,6 @@ static int engine_init(Engine &e, const rln_estep_config &cfg) {
         e.n_wsum_pix = (int)wp.size();
         RLN_TRY(upload(e.d_wsum_pix, banded_lists(wp, e.igf.s, e.igf.xs), e.stream));
     }
-    if (cfg.precision == RLN_PREC_SPLIT_BF16 && e.NT > 256)
-        RLN_FAIL(RLN_ERR_ARG, "split-BF16 coarse pass supports at most 256 translations (%d)", e.NT);
-    if (cfg.precision == RLN_PREC_SPLIT_BF16) {
-        // x phases of the coarse translations with rows padded to a multiple of 4 (zeros past xs)
-        e.xs4 = 4 * ((e.igc.xs + 3) / 4);
-        phase_rows(cx, e.sc, false, cfg.ori_size, rows);
-        std::vector<float2> rows4((size_t)e.NT * e.xs4, make_float2(0.f, 0.f));
-        for (int t = 0; t < e.NT; ++t)
-            for (int x = 0; x < e.igc.xs; ++x) rows4[(size_t)t * e.xs4 + x] = rows[(size_t)t * e.igc.xs + x];
-        RLN_TRY(upload(e.d_exg, rows4, e.stream));
-    }
     HIP_TRY(hipStreamSynchronize(e.stream));
     return RLN_OK;
 }
@@ -527,31 +597,7 @@ static int engine_model_tables(Engine &e) {
     std::vector<float> qc, qf, mw;
     q_of(e.sc, qc, nullptr);
     q_of(e.sf, qf, &mw);
-    if (cfg.precision == RLN_PREC_SPLIT_BF16) {
-        // pixel groups of the split pass: per row, x = 0 .. last pixel with non-zero Minvsigma2, in fours
-        std::vector<int2> grp;
-        for (int i = 0; i < e.igc.s; ++i) {
-            int xmax = -1;
-            for (int x = 0; x < e.igc.xs; ++x)
-                if (qc[(size_t)i * e.igc.xs + x] != 0.f) xmax = x;
-            for (int x0 = 0; x0 <= xmax; x0 += 4) grp.push_back(make_int2(i, x0));
-        }
-        e.G = (int)grp.size();
-        const int ng = 4 * ((e.G + 3) / 4);
-        grp.resize(std::max(ng, 4), make_int2(0, 0));
-        e.Kp = 8 * (int)grp.size();
-        RLN_TRY(upload(e.d_grp, grp, e.stream));
-        std::vector<float2> z(e.Kp / 2, make_float2(0.f, 0.f));
-        RLN_TRY(upload(e.d_zero_row, z, e.stream));
-        const long long ne = (long long)e.NT * (e.Kp / 2);
-        RLN_TRY(e.d_ehi.ensure(sizeof(unsigned int) * (size_t)ne));
-        RLN_TRY(e.d_elo.ensure(sizeof(unsigned int) * (size_t)ne));
-        hipLaunchKernelGGL(rlnk::k_phase_split, dim3((unsigned)((ne + rlnk::kBlock - 1) / rlnk::kBlock)),
-                           dim3(rlnk::kBlock), 0, e.stream, e.d_exg.as<const float2>(), e.xs4,
-                           e.d_ey_c.as<const float2>(), e.igc.s, e.d_grp.as<const int2>(), e.Kp / 2, e.NT,
-                           e.d_ehi.as<unsigned int>(), e.d_elo.as<unsigned int>());
-        HIP_TRY(hipGetLastError());
-    }
+    RLN_TRY(coarse_layout(e, qc));
     RLN_TRY(upload(e.d_q_c, qc, e.stream));
     RLN_TRY(upload(e.d_q_f, qf, e.stream));
     // fine pixels gathered per fine orientation: non-zero Minvsigma2 inside the projection radius
@@ -593,21 +639,12 @@ static int engine_coarse_projections(Engine &e) {
     for (int k = 0; k < e.K; ++k)
         if (e.proj_version[k] != e.proj[k]->version) stale = true;
     if (!stale) return RLN_OK;
-    if (e.cfg.precision == RLN_PREC_SPLIT_BF16) {
-        const size_t rows = (size_t)e.K * e.n_or;
-        RLN_TRY(e.d_pf.ensure(rows * (e.Kp / 2) * sizeof(float2)));
-        dim3 grid(e.K * e.n_or, (e.Kp / 2 + rlnk::kBlock - 1) / rlnk::kBlock);
-        hipLaunchKernelGGL(rlnk::k_project_grid_split, grid, dim3(rlnk::kBlock), 0, e.stream,
-                           e.d_vols.as<const float4 *const>(), e.vg, e.d_frames_c.as<const rlnk::Frame>(), e.n_or,
-                           e.igc, e.d_grp.as<const int2>(), e.G, e.Kp, e.d_pf.as<float2>());
-        RLN_TRY(launch_check("k_project_grid_split"));
-    } else {
-        const size_t n = (size_t)e.K * e.n_or * e.igc.P;
-        RLN_TRY(e.d_proj_c.ensure(n * sizeof(float2)));
-        dim3 grid(e.K * e.n_or, (e.igc.P + rlnk::kBlock - 1) / rlnk::kBlock);
+    RLN_TRY(e.d_pf.ensure((size_t)e.K * e.n_or * e.Kc * sizeof(float2)));
+    if (e.Kc > 0) {
+        dim3 grid(e.K * e.n_or, (e.Kc + rlnk::kBlock - 1) / rlnk::kBlock);
         hipLaunchKernelGGL(rlnk::k_project_grid, grid, dim3(rlnk::kBlock), 0, e.stream,
                            e.d_vols.as<const float4 *const>(), e.vg, e.d_frames_c.as<const rlnk::Frame>(), e.n_or,
-                           e.igc, e.d_proj_c.as<float2>());
+                           e.igc, e.d_grp.as<const int2>(), e.Kc, e.d_pf.as<float2>());
         RLN_TRY(launch_check("k_project_grid"));
     }
     for (int k = 0; k < e.K; ++k) e.proj_version[k] = e.proj[k]->version;
@@ -1257,31 +1294,44 @@ static int run_fine_stage(Engine &e, const FineLaunch &L0) {
     return RLN_OK;
 }
 
-template <int NTT>
-static void launch_mfma_t(Engine &e, unsigned n_tiles, const float *xi2, const long long *d2off) {
-    hipLaunchKernelGGL(rlnk::k_coarse_mfma<NTT>, dim3((n_tiles + rlnk::kMfG - 1) / rlnk::kMfG),
-                       dim3(rlnk::kMfBlock), 0, e.stream, e.d_tiles.as<const rlnk::CoarseTile>(), (int)n_tiles,
-                       e.d_or_off.as<const int>(), e.d_or_cnt.as<const int>(),
-                       e.d_or_proj.as<const int>(), e.d_pf.as<const float2>(), e.d_wc.as<const float2>(), e.d_ctf2.as<const float>(), e.d_ynorm.as<const double>(),
-                       e.d_ehi.as<const unsigned int>(), e.d_elo.as<const unsigned int>(), xi2, d2off, e.NT, e.Kp,
-                       e.d_zero_row.as<const float2>(), e.d_diff2.as<float>(), e.d_wpart.as<rlnk::WPart>());
-}
-
-static int launch_coarse_mfma(Engine &e, unsigned n_tiles, const float *xi2, const long long *d2off) {
-    const int ntt = (e.NT + 15) / 16;
-    switch (ntt) {
-#define RLN_MFMA_CASE(N)                          \
-    case N:                                       \
-        launch_mfma_t<N>(e, n_tiles, xi2, d2off); \
+static int launch_coarse(Engine &e, unsigned n_tiles, const float *xi2, const long long *d2off) {
+    rlnk::CoarseArgs a{};
+    a.tiles = e.d_tiles.as<const rlnk::CoarseTile>();
+    a.or_off = e.d_or_off.as<const int>();
+    a.or_cnt = e.d_or_cnt.as<const int>();
+    a.or_proj = e.d_or_proj.as<const int>();
+    a.pf = e.d_pf.as<const float2>();
+    a.zero_row = e.d_zero_row.as<const float2>();
+    a.w = e.d_wc.as<const float2>();
+    a.ctf2 = e.d_ctf2.as<const float>();
+    a.ynorm = e.d_ynorm.as<const double>();
+    a.xi2half = xi2;
+    a.d2_off = d2off;
+    a.pairs = e.d_pairs_c.as<const int2>();
+    a.ytab = e.d_ytab.as<const float>();
+    a.xtab = e.d_xtab.as<const float2>();
+    a.cols = e.d_cols.as<const rlnk::CoarseColumn>();
+    a.tile_of = e.col_tiles > 1 ? e.d_tile_of.as<const int>() : nullptr;
+    a.n_pairs = e.n_pairs_c;
+    a.n_xsteps = e.n_xsteps;
+    a.NT = e.NT;
+    a.Kc = e.Kc;
+    a.diff2 = e.d_diff2.as<float>();
+    a.part = e.d_wpart.as<rlnk::WPart>();
+    const dim3 grid(n_tiles, e.col_tiles);
+    const size_t lds = sizeof(float2) * 64 * e.n_xsteps;
+    switch (e.mshift) {
+#define RLN_COARSE_CASE(M)                                                                               \
+    case M:                                                                                              \
+        hipLaunchKernelGGL(rlnk::k_coarse_lattice<M>, grid, dim3(rlnk::kBlock), lds, e.stream, a);       \
         break;
-        RLN_MFMA_CASE(1) RLN_MFMA_CASE(2) RLN_MFMA_CASE(3) RLN_MFMA_CASE(4) RLN_MFMA_CASE(5) RLN_MFMA_CASE(6)
-        RLN_MFMA_CASE(7) RLN_MFMA_CASE(8) RLN_MFMA_CASE(9) RLN_MFMA_CASE(10) RLN_MFMA_CASE(11) RLN_MFMA_CASE(12)
-        RLN_MFMA_CASE(13) RLN_MFMA_CASE(14) RLN_MFMA_CASE(15) RLN_MFMA_CASE(16)
-#undef RLN_MFMA_CASE
+        RLN_COARSE_CASE(0) RLN_COARSE_CASE(1) RLN_COARSE_CASE(2) RLN_COARSE_CASE(3) RLN_COARSE_CASE(4)
+        RLN_COARSE_CASE(5) RLN_COARSE_CASE(6) RLN_COARSE_CASE(7) RLN_COARSE_CASE(8) RLN_COARSE_CASE(9)
+#undef RLN_COARSE_CASE
         default:
-            RLN_FAIL(RLN_ERR_ARG, "split-BF16 coarse pass supports at most 256 translations (%d)", e.NT);
+            RLN_FAIL(RLN_ERR_ARG, "translation lattice of %d shifts on an axis", 2 * e.mshift + 1);
     }
-    return launch_check("k_coarse_mfma");
+    return launch_check("k_coarse_lattice");
 }
 
 // The host lists of a chunk (h) are built beforehand, for the chunk after the first on a second host thread
@@ -1348,47 +1398,26 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     const double *d_prior = d_old + 2 * cB;
     const double *d_xi2d = d_old + 4 * cB;  // highres_Xi2 / 2 in FP64
 
-    // coarse: scaled images, shifted images
-    const bool split = cfg.precision == RLN_PREC_SPLIT_BF16;
-    if (split) {
-        const size_t nc = (size_t)B * (e.Kp / 2);
-        RLN_TRY(e.d_wc.ensure(nc * sizeof(float2)));
-        RLN_TRY(e.d_ctf2.ensure(nc * sizeof(float)));
-        RLN_TRY(e.d_ynorm.ensure(sizeof(double) * B));
-        HIP_TRY(hipMemsetAsync(e.d_ynorm.ptr, 0, sizeof(double) * B, st));
-        const int nthr = std::max(e.Kp / 2, (int)Pc);
-        hipLaunchKernelGGL(rlnk::k_prep_coarse_split, dim3((nthr + rlnk::kBlock - 1) / rlnk::kBlock, B),
-                           dim3(rlnk::kBlock), 0, st, dX, dC, d_scale, e.sf, (int)Pf, e.igc, e.d_q_c.as<const float>(),
-                           e.d_grp.as<const int2>(), e.G, e.Kp, cfg.do_ctf_correction, e.d_wc.as<float2>(),
-                           e.d_ctf2.as<float>(), e.d_ynorm.as<double>());
-        RLN_TRY(launch_check("k_prep_coarse_split"));
-    } else {
-        RLN_TRY(e.d_ctfq.ensure(sizeof(float) * Pc * B));
-        RLN_TRY(e.d_yq.ensure(sizeof(float2) * Pc * NT * B));
-        hipLaunchKernelGGL(rlnk::k_prep_coarse, dim3((Pc + rlnk::kBlock - 1) / rlnk::kBlock, NT, B),
-                           dim3(rlnk::kBlock), 0, st, dX, dC, d_scale, e.sf, (int)Pf, e.igc,
-                           e.d_q_c.as<const float>(), e.d_ex_c.as<const float2>(), e.d_ey_c.as<const float2>(), NT,
-                           cfg.do_ctf_correction, e.d_ctfq.as<float>(), e.d_yq.as<float2>());
-        RLN_TRY(launch_check("k_prep_coarse"));
-    }
+    // coarse: particle rows in the contraction's layout
+    const size_t nc = (size_t)B * e.Kc;
+    RLN_TRY(e.d_wc.ensure(nc * sizeof(float2)));
+    RLN_TRY(e.d_ctf2.ensure(nc * sizeof(float)));
+    RLN_TRY(e.d_ynorm.ensure(sizeof(double) * B));
+    HIP_TRY(hipMemsetAsync(e.d_ynorm.ptr, 0, sizeof(double) * B, st));
+    hipLaunchKernelGGL(rlnk::k_prep_coarse, dim3((std::max(e.Kc, (int)Pc) + rlnk::kBlock - 1) / rlnk::kBlock, B),
+                       dim3(rlnk::kBlock), 0, st, dX, dC, d_scale, e.sf, (int)Pf, e.igc, e.d_q_c.as<const float>(),
+                       e.d_grp.as<const int2>(), e.Kc, cfg.do_ctf_correction, e.d_wc.as<float2>(),
+                       e.d_ctf2.as<float>(), e.d_ynorm.as<double>());
+    RLN_TRY(launch_check("k_prep_coarse"));
     HIP_TRY(hipEventRecord(e.ev[kStCoarse], st));
     RLN_TRY(e.d_diff2.ensure(sizeof(float) * std::max<long long>(1, h.total_entries)));
     RLN_TRY(e.d_weight.ensure(sizeof(double) * std::max<long long>(1, h.total_entries)));
     RLN_TRY(e.d_mask.ensure(std::max<long long>(1, h.total_entries)));
-    // per-particle selection state; the split coarse kernel folds the minimum diff2 into it as it writes
+    // per-particle selection state; the coarse kernel folds the minimum diff2 into it as it writes
     const unsigned gB = (unsigned)((B + rlnk::kBlock - 1) / rlnk::kBlock);
     RLN_TRY(e.d_wpart.ensure(sizeof(rlnk::WPart) * B));
     hipLaunchKernelGGL(rlnk::k_wpart_init, dim3(gB), dim3(rlnk::kBlock), 0, st, e.d_wpart.as<rlnk::WPart>(), B);
-    if (split && !h.tiles.empty()) {
-        RLN_TRY(launch_coarse_mfma(e, (unsigned)h.tiles.size(), d_xi2, d_d2off.as<const long long>()));
-    } else if (!h.tiles.empty()) {
-        hipLaunchKernelGGL(rlnk::k_coarse_diff2, dim3((unsigned)h.tiles.size(), (NT + rlnk::kCoTT - 1) / rlnk::kCoTT),
-                           dim3(rlnk::kBlock), 0, st, e.d_tiles.as<const rlnk::CoarseTile>(), e.d_or_off.as<const int>(),
-                           e.d_or_cnt.as<const int>(), e.d_or_proj.as<const int>(), e.d_proj_c.as<const float2>(),
-                           e.d_ctfq.as<const float>(), e.d_yq.as<const float2>(), d_xi2, d_d2off.as<const long long>(),
-                           NT, (int)Pc, e.d_diff2.as<float>());
-        RLN_TRY(launch_check("k_coarse_diff2"));
-    }
+    if (!h.tiles.empty()) RLN_TRY(launch_coarse(e, (unsigned)h.tiles.size(), d_xi2, d_d2off.as<const long long>()));
     HIP_TRY(hipEventRecord(e.ev[kStCoarseW], st));
     RLN_TRY(e.d_stats_c.ensure(sizeof(rlnk::PassStats) * B));
     rlnk::WeightArgs wa{};
@@ -1426,7 +1455,6 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         rlnk::WPart *wp = e.d_wpart.as<rlnk::WPart>();
         unsigned int *hc = e.d_hcnt.as<unsigned int>();
         double *hs = e.d_hsum.as<double>();
-        if (!split) hipLaunchKernelGGL(rlnk::k_wseg_min, dim3(nseg), dim3(rlnk::kBlock), 0, st, wa, sg, wp);
         hipLaunchKernelGGL(rlnk::k_wseg_exp, dim3(nseg), dim3(rlnk::kBlock), 0, st, wa, sg, wp, hc, hs);
         hipLaunchKernelGGL(rlnk::k_wsel_start, dim3(gB), dim3(rlnk::kBlock), 0, st, wa, wp, B);
         for (int shift = 56; shift >= 0; shift -= 8) {
@@ -1982,13 +2010,13 @@ extern "C" int rln_estep_destroy(rln_estep *e) {
     if (!e) return RLN_OK;
     (void)hipSetDevice(e->device);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
-    rln::DevBuf *bufs[] = {&e->d_frames_c, &e->d_frames_f, &e->d_proj_c, &e->d_pf, &e->d_ehi, &e->d_elo,
-                           &e->d_zero_row, &e->d_wc, &e->d_grp, &e->d_exg, &e->d_ctf2, &e->d_ynorm, &e->d_q_c, &e->d_q_f, &e->d_minv_w,
-                           &e->d_mresol, &e->d_xa_shell, &e->d_ex_c, &e->d_ey_c, &e->d_ex_f, &e->d_ey_f,
+    rln::DevBuf *bufs[] = {&e->d_frames_c, &e->d_frames_f, &e->d_pf, &e->d_zero_row, &e->d_wc, &e->d_ctf2, &e->d_ynorm,
+                           &e->d_grp, &e->d_pairs_c, &e->d_ytab, &e->d_xtab, &e->d_cols, &e->d_tile_of, &e->d_q_c,
+                           &e->d_q_f, &e->d_minv_w, &e->d_mresol, &e->d_xa_shell, &e->d_ex_f, &e->d_ey_f,
                            &e->d_tr_ix, &e->d_tr_iy, &e->d_over_x, &e->d_over_y, &e->d_vols, &e->d_bp_ptrs,
                            &e->d_fimg, &e->d_fimgn, &e->d_fctf, &e->d_meta_f, &e->d_meta_d, &e->d_meta_ll,
                            &e->d_or_off, &e->d_oc_off, &e->d_or_cnt, &e->d_or_proj, &e->d_or_prior, &e->d_or_frame,
-                           &e->d_or_class, &e->d_or_dir, &e->d_tr_prior, &e->d_ctfq, &e->d_yq, &e->d_tiles,
+                           &e->d_or_class, &e->d_or_dir, &e->d_tr_prior, &e->d_tiles,
                            &e->d_diff2, &e->d_weight, &e->d_mask, &e->d_stats_c, &e->d_stats_f, &e->d_npairs,
                            &e->d_njobs, &e->d_nchunks, &e->d_pair_off, &e->d_job_off, &e->d_chunk_off, &e->d_pairs,
                            &e->d_jobs, &e->d_job_order, &e->d_chunk_job, &e->d_chunk_first, &e->d_fdiff2, &e->d_fbase, &e->d_fweight,
@@ -2180,9 +2208,8 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
     // chunk boundaries from a device-memory budget for the coarse intermediates (13 bytes per coarse pose:
     // diff2, FP64 weight, mask), with per-particle pose counts: the explicit list, the whole grid, or a fraction
     // of it for local searches
-    const size_t Pc = e->igc.P, Pf = e->igf.P;
-    const bool split = e->cfg.precision == RLN_PREC_SPLIT_BF16;
-    const double fixed = (split ? 6.0 * e->Kp : 8.0 * Pc * e->NT) + 20.0 * Pf + 64.0 * 1024;
+    const size_t Pf = e->igf.P;
+    const double fixed = 12.0 * e->Kc + 20.0 * Pf + 64.0 * 1024;
     const double budget = 24.0e9;
     std::vector<int> starts;
     {

@@ -85,159 +85,16 @@ inline unsigned fold_blocks(const VolGeom &g, int layers = -1) {
 // Coarse pass
 // --------------------------------------------------------------------------------------------------
 
-// Projections of every coarse orientation of every class at the coarse size:
-// proj[(k*n_or + o)*P + p] (class-major). One thread per pixel, grid (K*n_or, ceil(P/256)).
-__global__ void __launch_bounds__(kBlock) k_project_grid(const float4 *const *__restrict__ vols, VolGeom vg,
-                                                         const Frame *__restrict__ frames, int n_or, ImgGeom ig,
-                                                         float2 *__restrict__ proj) {
-    const int p = blockIdx.y * kBlock + threadIdx.x;
-    const int ko = blockIdx.x;
-    if (p >= ig.P) return;
-    const int k = ko / n_or, o = ko - k * n_or;
-    int x, y;
-    pixel_xy(p, ig.s, ig.xs, x, y);
-    float2 v = make_float2(0.f, 0.f);
-    if (x * x + y * y <= ig.proj_r2_max) v = project_pixel(vols[k], vg, frames[o], x, y);
-    proj[(size_t)ko * ig.P + p] = v;
-}
-
-// Windowed, sqrt(Minvsigma2/2)-scaled images of the coarse pass for B particles:
-//   ctfq[b][p] = q_p * ctf_b(p) * scale_b  and  yq[b][t][p] = q_p * X_b(p) * exp(-2 pi i (x tx + y ty)/N),
-// with the phase factored as ex[t][x] * ey[t][i]. X and ctf are read from the fine-size input (window of
-// src/fftw.h:809-857). grid (ceil(P/256), NT, B).
-__global__ void __launch_bounds__(kBlock) k_prep_coarse(const float2 *__restrict__ fimg, const float *__restrict__ fctf,
-                                                        const float *__restrict__ scale, int sf, int Pf, ImgGeom ig,
-                                                        const float *__restrict__ q, const float2 *__restrict__ ex,
-                                                        const float2 *__restrict__ ey, int NT, int do_ctf,
-                                                        float *__restrict__ ctfq, float2 *__restrict__ yq) {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    const int t = blockIdx.y, b = blockIdx.z;
-    if (p >= ig.P) return;
-    const int i = p / ig.xs, x = p - i * ig.xs;
-    const int y = (i < ig.xs) ? i : i - ig.s;
-    const int isrc = (y < 0) ? y + sf : y;
-    const size_t src = (size_t)b * Pf + (size_t)isrc * (sf / 2 + 1) + x;
-    const float qp = q[p];
-    const float2 X = fimg[src];
-    const float2 ph = cmul(ex[(size_t)t * ig.xs + x], ey[(size_t)t * ig.s + i]);
-    const float2 v = cmul(make_float2(X.x * qp, X.y * qp), ph);
-    yq[((size_t)b * NT + t) * ig.P + p] = v;
-    if (t == 0) ctfq[(size_t)b * ig.P + p] = qp * (do_ctf ? fctf[src] : 1.f) * scale[b];
-}
-
-// Tile of the coarse squared differences: TO orientations x TT translations of one particle.
-constexpr int kCoTO = 64, kCoTT = 64, kCoCP = 32;
+// Orientations of one block of the coarse kernel (16 per wave).
+constexpr int kCoTO = 64;
 
 struct CoarseTile {
     int b;        // particle within the batch
     int o_begin;  // first orientation (within the particle's list)
 };
 
-// diff2[b][o][t] = highres_Xi2/2 + sum_p |ctfq_b(p) * P_o(p) - yq_b,t(p)|^2 (getAllSquaredDifferences,
-// src/ml_optimiser.cpp:7430-7442). Orientations whose prior or class prior is zero are marked -999 (never
-// computed, as in the reference's exp_Mweight initialisation, :7155). grid (n_tiles, ceil(NT/TT)).
-__global__ void __launch_bounds__(kBlock) k_coarse_diff2(const CoarseTile *__restrict__ tiles,
-                                                         const int *__restrict__ or_off, const int *__restrict__ or_cnt,
-                                                         const int *__restrict__ or_proj, const float2 *__restrict__ proj,
-                                                         const float *__restrict__ ctfq, const float2 *__restrict__ yq,
-                                                         const float *__restrict__ xi2half, const long long *__restrict__ d2_off,
-                                                         int NT, int P, float *__restrict__ diff2) {
-    __shared__ float2 As[kCoCP][kCoTO];
-    __shared__ float2 Ys[kCoCP][kCoTT];
-    __shared__ int og_s[kCoTO];
-    const CoarseTile tile = tiles[blockIdx.x];
-    const int b = tile.b;
-    const int n_o = or_cnt[b];
-    const int t_begin = blockIdx.y * kCoTT;
-    const int tid = threadIdx.x;
-    const int to = tid >> 4, tt = tid & 15;
-    if (tid < kCoTO) {
-        const int o = tile.o_begin + tid;
-        og_s[tid] = (o < n_o) ? or_proj[or_off[b] + o] : -1;
-    }
-    __syncthreads();
-    const float *cq = ctfq + (size_t)b * P;
-    const float2 *yb = yq + (size_t)b * NT * P;
-    float tot[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) tot[i][j] = 0.f;
-    for (int p0 = 0; p0 < P; p0 += kCoCP) {
-        // stage c*P for TO orientations (coalesced along p)
-        for (int idx = tid; idx < kCoCP * kCoTO; idx += kBlock) {
-            const int oo = idx / kCoCP, pp = idx - oo * kCoCP;
-            const int p = p0 + pp;
-            float2 v = make_float2(0.f, 0.f);
-            const int og = og_s[oo];
-            if (og >= 0 && p < P) {
-                const float2 pr = proj[(size_t)og * P + p];
-                const float c = cq[p];
-                v = make_float2(c * pr.x, c * pr.y);
-            }
-            As[pp][oo] = v;
-        }
-        for (int idx = tid; idx < kCoCP * kCoTT; idx += kBlock) {
-            const int tq = idx / kCoCP, pp = idx - tq * kCoCP;
-            const int p = p0 + pp, t = t_begin + tq;
-            Ys[pp][tq] = (t < NT && p < P) ? yb[(size_t)t * P + p] : make_float2(0.f, 0.f);
-        }
-        __syncthreads();
-        float acc[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-#pragma unroll 4
-        for (int pp = 0; pp < kCoCP; ++pp) {
-            float2 a[4], y[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[pp][to + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) y[j] = Ys[pp][tt + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float dr = a[i].x - y[j].x, di = a[i].y - y[j].y;
-                    acc[i][j] = fmaf(dr, dr, acc[i][j]);
-                    acc[i][j] = fmaf(di, di, acc[i][j]);
-                }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) tot[i][j] += acc[i][j];
-        __syncthreads();
-    }
-    const float base = xi2half[b];
-    float *out = diff2 + d2_off[b];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int oo = to + 16 * i;
-        const int o = tile.o_begin + oo;
-        if (o >= n_o) continue;
-        const bool skip = og_s[oo] < 0 || or_proj[or_off[b] + o] < 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int t = t_begin + tt + 16 * j;
-            if (t < NT) out[(size_t)o * NT + t] = skip ? -999.f : base + tot[i][j];
-        }
-    }
-}
-
-// --------------------------------------------------------------------------------------------------
-// Split-BF16 coarse pass on MFMA.
-// diff2(o,t) = Xi2/2 + sum_p c_p^2 |P_o(p)|^2 + sum_p |y_t(p)|^2 - 2 sum_p Re(P_o(p) conj(c_p y_t(p))),
-// with y_t(p) = q_p X(p) exp(-2 pi i (x tx + y ty)/N) (|y_t|^2 does not depend on t) and c_p = q_p ctf_p s.
-// The cross term is a real contraction over k = 2p + {re, im} of A[o][k] (the projection, shared by all
-// particles) and B[t][k] = c_p y_t(p); both are split x = hi + lo in BF16 and the products hi*hi + hi*lo +
-// lo*hi are accumulated in FP32 by v_mfma_f32_16x16x32_bf16.
-// --------------------------------------------------------------------------------------------------
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float floatx2_t __attribute__((ext_vector_type(2)));
 
 // round-to-nearest-even FP32 -> BF16 bit pattern
 __device__ __forceinline__ unsigned short f2bf(float x) {
@@ -245,16 +102,11 @@ __device__ __forceinline__ unsigned short f2bf(float x) {
     u += 0x7fffu + ((u >> 16) & 1u);
     return (unsigned short)(u >> 16);
 }
-__device__ __forceinline__ float bf2f(unsigned short h) { return __uint_as_float((unsigned int)h << 16); }
-__device__ __forceinline__ void split_bf16(float x, unsigned short &hi, unsigned short &lo) {
-    hi = f2bf(x);
-    lo = f2bf(x - bf2f(hi));
-}
 __device__ __forceinline__ bf16x8_t load_bf16x8(const unsigned short *p) {
     return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(p));
 }
 
-// Lane layout of v_mfma_f32_16x16x32_bf16 used below (checked by k_selftest_mfma): lane l supplies row l%16 of
+// Lane layout of v_mfma_f32_16x16x32_bf16 (checked by k_selftest_mfma): lane l supplies row l%16 of
 // A and column l%16 of B, each with the 8 consecutive k = 8*(l/16) .. 8*(l/16)+7; it receives D rows
 // 4*(l/16) .. 4*(l/16)+3 of column l%16.
 __global__ void k_selftest_mfma(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ D) {
@@ -269,52 +121,52 @@ __global__ void k_selftest_mfma(const float *__restrict__ A, const float *__rest
     for (int j = 0; j < 4; ++j) D[(4 * (l / 16) + j) * 16 + l % 16] = acc[j];
 }
 
-// Contraction layout of the split-BF16 pass: pixel groups of 4 consecutive x in one row. Group g = (row i, x0)
-// holds pixels (i, x0 .. x0+3) at k = 8g + 2j + {re, im}; the groups cover, row by row, x = 0 up to the last
-// pixel whose Minvsigma2 is non-zero, so rows and corners that carry no weight are not contracted. Kp = 8 *
-// (groups rounded up to a multiple of 4); slots past the last group and pixels with x >= xs hold zeros.
+// --------------------------------------------------------------------------------------------------
+// Coarse squared differences (getAllSquaredDifferences, src/ml_optimiser.cpp:7430-7442):
+//   diff2(o,t) = Xi2/2 + sum_p |c_p P_o(p) - y_t(p)|^2,  y_t(p) = q_p X(p) E_t(p),  c_p = q_p ctf_p s,
+// with E_t(x, y) = exp(-2 pi i (x tx + y ty) / N) and |y_t| = |q X|, expanded to
+//   Xi2/2 + sum |q X|^2 (FP64, per particle) + sum c^2 |P|^2 (per orientation) - 2 cross(o,t),
+//   cross(o,t) = sum_p Re(conj(A_o(p)) E_t(p)),  A = P conj(w),  w = c q X.
+// The translations lie on a lattice, so E factors into an x and a y phase and the cross term into two short
+// contractions instead of one over all pixels for every translation: with A = a + i b, cx + i sx the x phase of tx and
+// cy + i sy the y phase of ty,
+//   U(y,tx) = sum_x a cx + b sx,  V(y,tx) = sum_x b cx - a sx,  cross = sum_y cy U + sy V.
+// Opposite shifts share their sums (cos is even, sin odd): the x contraction is the real matrix product of the rows a
+// and b with the columns cos(tx), sin(tx), tx > 0, on the FP32 matrix units; rows y and -y are added and subtracted
+// before the y contraction, which runs in registers on each lane's tx.
+//
+// Pixel layout of that contraction: per row pair (y, -y), y = 0 .. s/2, steps of 16 complex slots: 8 consecutive x of
+// row y, then the same 8 of row -y (zeros where there is no such row); a pair has steps up to its last pixel whose
+// Minvsigma2 is non-zero, so rows and corners that carry no weight are not contracted. grp holds (row, x0) of every 8
+// slots (row -1: none). Kc = 16 * steps complex slots per projection.
+// --------------------------------------------------------------------------------------------------
 
-// hi + lo split of two floats with the hardware round-to-nearest-even conversion; hi and lo are packed pairs
-__device__ __forceinline__ void split2_bf16(float a, float b, unsigned int &hi, unsigned int &lo) {
-    const bf16x2_t h = __builtin_convertvector((floatx2_t){a, b}, bf16x2_t);
-    hi = __builtin_bit_cast(unsigned int, h);
-    const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xffff0000u);
-    lo = __builtin_bit_cast(unsigned int, __builtin_convertvector((floatx2_t){ra, rb}, bf16x2_t));
-}
-
-// Projection tables of the split pass in the group layout: FP32 complex pf [K*n_or][Kp/2] (the coarse kernel
-// multiplies them by the particle and splits them in BF16). grid (K*n_or, ceil(Kp/2/256)).
-__global__ void __launch_bounds__(kBlock) k_project_grid_split(const float4 *const *__restrict__ vols, VolGeom vg,
-                                                               const Frame *__restrict__ frames, int n_or, ImgGeom ig,
-                                                               const int2 *__restrict__ grp, int G, int Kp,
-                                                               float2 *__restrict__ pf) {
-    const int idx = blockIdx.y * kBlock + threadIdx.x;  // complex slot 4g + j
+// Projections of every coarse orientation of every class in that layout: FP32 complex pf [K*n_or][Kc].
+// grid (K*n_or, ceil(Kc/256)).
+__global__ void __launch_bounds__(kBlock) k_project_grid(const float4 *const *__restrict__ vols, VolGeom vg,
+                                                         const Frame *__restrict__ frames, int n_or, ImgGeom ig,
+                                                         const int2 *__restrict__ grp, int Kc, float2 *__restrict__ pf) {
+    const int idx = blockIdx.y * kBlock + threadIdx.x;  // complex slot 8g + j
     const int ko = blockIdx.x;
-    if (2 * idx >= Kp) return;
-    const int g = idx >> 2, j = idx & 3;
+    if (idx >= Kc) return;
+    const int2 gr = grp[idx >> 3];
+    const int x = gr.y + (idx & 7), i = gr.x;
+    const int y = (i < ig.xs) ? i : i - ig.s;
     float2 v = make_float2(0.f, 0.f);
-    if (g < G) {
-        const int2 gr = grp[g];
-        const int x = gr.y + j, i = gr.x;
-        const int y = (i < ig.xs) ? i : i - ig.s;
-        if (x < ig.xs && x * x + y * y <= ig.proj_r2_max) {
-            const int k = ko / n_or, o = ko - k * n_or;
-            v = project_pixel(vols[k], vg, frames[o], x, y);
-        }
+    if (i >= 0 && x < ig.xs && x * x + y * y <= ig.proj_r2_max) {
+        const int k = ko / n_or, o = ko - k * n_or;
+        v = project_pixel(vols[k], vg, frames[o], x, y);
     }
-    pf[(size_t)ko * (Kp / 2) + idx] = v;
+    pf[(size_t)ko * Kc + idx] = v;
 }
 
-// Particle side of the split pass, in the group layout: w[b][4g+j] = c_p q_p X(p) with c_p = q_p ctf_p s (the
-// translation phase is the coarse kernel's B operand), ctf2[b][4g+j] = c_p^2, and ynorm[b] = sum_p |q_p X(p)|^2
-// over all pixels (FP64). grid (ceil(max(Kp/2, P)/256), B).
-__global__ void __launch_bounds__(kBlock) k_prep_coarse_split(const float2 *__restrict__ fimg,
-                                                              const float *__restrict__ fctf,
-                                                              const float *__restrict__ scale, int sf, int Pf,
-                                                              ImgGeom ig, const float *__restrict__ q,
-                                                              const int2 *__restrict__ grp, int G, int Kp, int do_ctf,
-                                                              float2 *__restrict__ w, float *__restrict__ ctf2,
-                                                              double *__restrict__ ynorm) {
+// Particle side in that layout: w[b][slot] = c_p q_p X(p), ctf2[b][slot] = c_p^2, and ynorm[b] = sum_p |q_p X(p)|^2
+// over all pixels (FP64). grid (ceil(max(Kc, P)/256), B).
+__global__ void __launch_bounds__(kBlock) k_prep_coarse(const float2 *__restrict__ fimg, const float *__restrict__ fctf,
+                                                        const float *__restrict__ scale, int sf, int Pf, ImgGeom ig,
+                                                        const float *__restrict__ q, const int2 *__restrict__ grp,
+                                                        int Kc, int do_ctf, float2 *__restrict__ w,
+                                                        float *__restrict__ ctf2, double *__restrict__ ynorm) {
     __shared__ double red[kBlock / 64];
     const int idx = blockIdx.x * kBlock + threadIdx.x;
     const int b = blockIdx.y;
@@ -324,24 +176,21 @@ __global__ void __launch_bounds__(kBlock) k_prep_coarse_split(const float2 *__re
         const int isrc = (y < 0) ? y + sf : y;
         return (size_t)b * Pf + (size_t)isrc * (sf / 2 + 1) + x;
     };
-    if (idx < Kp / 2) {
-        const int g = idx >> 2, j = idx & 3;
+    if (idx < Kc) {
+        const int2 gr = grp[idx >> 3];
+        const int x = gr.y + (idx & 7), i = gr.x;
         float2 v = make_float2(0.f, 0.f);
         float c2 = 0.f;
-        if (g < G) {
-            const int2 gr = grp[g];
-            const int x = gr.y + j, i = gr.x;
-            if (x < ig.xs) {
-                const size_t src = src_of(i, x);
-                const float qp = q[i * ig.xs + x];
-                const float c = qp * (do_ctf ? fctf[src] : 1.f) * sc;
-                const float2 X = fimg[src];
-                v = make_float2(c * qp * X.x, c * qp * X.y);
-                c2 = c * c;
-            }
+        if (i >= 0 && x < ig.xs) {
+            const size_t src = src_of(i, x);
+            const float qp = q[i * ig.xs + x];
+            const float c = qp * (do_ctf ? fctf[src] : 1.f) * sc;
+            const float2 X = fimg[src];
+            v = make_float2(c * qp * X.x, c * qp * X.y);
+            c2 = c * c;
         }
-        w[(size_t)b * (Kp / 2) + idx] = v;
-        ctf2[(size_t)b * (Kp / 2) + idx] = c2;
+        w[(size_t)b * Kc + idx] = v;
+        ctf2[(size_t)b * Kc + idx] = c2;
     }
     float yn = 0.f;
     if (idx < ig.P) {
@@ -360,26 +209,8 @@ __global__ void __launch_bounds__(kBlock) k_prep_coarse_split(const float2 *__re
     }
 }
 
-// Translation operand of the split pass, the same for every particle: the phase E[t][4g + m] = ex[t][x0 + m] *
-// ey[t][row] of every complex slot of pixel group g = (row, x0) (rows of exg padded with zeros past xs), split
-// into BF16 hi and lo (re, im) pairs. grid (ceil(NT * Kc / 256)).
-__global__ void __launch_bounds__(kBlock) k_phase_split(const float2 *__restrict__ exg, int xs4,
-                                                        const float2 *__restrict__ ey, int s,
-                                                        const int2 *__restrict__ grp, int Kc, int NT,
-                                                        unsigned int *__restrict__ ehi, unsigned int *__restrict__ elo) {
-    const long long idx = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (idx >= (long long)NT * Kc) return;
-    const int t = (int)(idx / Kc), c = (int)(idx - (long long)t * Kc);
-    const int2 gr = grp[c >> 2];
-    const float2 v = cmul(exg[(size_t)t * xs4 + gr.y + (c & 3)], ey[(size_t)t * s + gr.x]);
-    unsigned int h, l;
-    split2_bf16(v.x, v.y, h, l);
-    ehi[idx] = h;
-    elo[idx] = l;
-}
-
-// Per-particle state of the coarse weights and significance selection (k_wpart_init .. k_wsel_stats); the
-// split coarse kernel already folds its minimum diff2 into mn_bits.
+// Per-particle state of the coarse weights and significance selection (k_wpart_init .. k_wsel_stats); the coarse
+// kernel already folds its minimum diff2 into mn_bits.
 struct WPart {
     unsigned int mn_bits;   // min diff2 (non-negative float bits)
     int status;
@@ -395,176 +226,216 @@ struct WPart {
     long long n_above;      // entries >= thr
 };
 
-constexpr int kMfO = 64;    // orientations per tile (4 MFMA row tiles)
-constexpr int kMfG = 1;     // tiles per block, each with its own 4 waves
-constexpr int kMfBlock = 256 * kMfG;
+// Columns of the x contraction: 16 lanes hold one signed x shift each, tx = +(n + 1) on lane n < 8 (matrix column
+// cos) and -(n - 7) on lane n >= 8 (column sin), counted from kColShift * tile; where a tile
+// has fewer than 8 positive shifts, lane 7 is tx = 0 (in the last tile) and lane 15 unused.
+struct CoarseColumn {
+    int t0;    // translation index of (tx, ty = 0)
+    int half;  // ty = -half .. half exist, -1: no column
+};
+constexpr int kColShift = 8;
 
-// One block per two coarse tiles (64 orientations of one particle each, possibly different particles) and all
-// translations. The cross term sum_p Re(conj(P_o(p)) w(p) E_t(p)) is a real dot product of (re, im) pairs
-// between A[o][p] = P_o(p) conj(w(p)), formed while a group stages its tile's projection rows (64 rows a K step)
-// and split in BF16, and B[t][p] = E_t(p), the particle-independent phase table split once per model
-// (k_phase_split) and read straight into the MFMA operands: the two groups read the same B fragments, the second
-// from the cache. Wave w of a group owns translation tiles w, w+4, w+8, ... and the group's four orientation
-// tiles; row tiles past the tile's orientations are skipped. grid (ceil(n_tiles / 2)).
-template <int NTT>  // translation tiles of 16 in the block (16*NTT >= NT)
-__global__ void __launch_bounds__(kMfBlock, 3) k_coarse_mfma(const CoarseTile *__restrict__ tiles, int n_tiles,
-                                                          const int *__restrict__ or_off,
-                                                          const int *__restrict__ or_cnt,
-                                                          const int *__restrict__ or_proj,
-                                                          const float2 *__restrict__ pf,
-                                                          const float2 *__restrict__ w,
-                                                          const float *__restrict__ ctf2,
-                                                          const double *__restrict__ ynorm,
-                                                          const unsigned int *__restrict__ ehi,
-                                                          const unsigned int *__restrict__ elo,
-                                                          const float *__restrict__ xi2half,
-                                                          const long long *__restrict__ d2_off, int NT, int Kp,
-                                                          const float2 *__restrict__ zero_row,
-                                                          float *__restrict__ diff2, WPart *__restrict__ part) {
-    constexpr int kTW = (NTT + 3) / 4;  // translation tiles per wave
-    constexpr int kAStride = 40;        // bf16 per staged A row (32 + 8 padding against bank conflicts)
-    __shared__ int og_s[kMfG][kMfO];
-    __shared__ float a_norm[kMfG][kMfO];
-    // A operand of one K step (hi and lo planes of the block's 128 rows), double buffered
-    __shared__ __align__(16) unsigned short s_a[2][2][kMfG * kMfO * kAStride];
+struct CoarseArgs {
+    const CoarseTile *tiles;
+    const int *or_off, *or_cnt, *or_proj;
+    const float2 *pf;         // projections [K*n_or][Kc]
+    const float2 *zero_row;   // [Kc] zeros
+    const float2 *w;          // [b][Kc]
+    const float *ctf2;        // [b][Kc]
+    const double *ynorm;
+    const float *xi2half;
+    const long long *d2_off;
+    const int2 *pairs;        // row pairs: (steps, 1 with a row -y)
+    const float *ytab;        // per row pair: cos(2 pi y ty / N) for ty = 0 .. M, -sin for ty = 1 .. M
+    const float2 *xtab;       // [column tile][step of a row][lane]: the two x phases of the lane's column
+    const CoarseColumn *cols; // [column tile][16], then the tx = 0 column of M == 8
+    const int *tile_of;       // column tile of each translation, null with one tile
+    int n_pairs, n_xsteps;
+    int NT, Kc;
+    float *diff2;
+    WPart *part;
+};
+
+// Value of the lane 8 further in its row of 16 lanes.
+__device__ __forceinline__ float dpp_ror8(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
+}
+
+// One block per tile of 64 orientations of one particle, 16 per wave, all translations of one column tile; M: number
+// of positive shifts of the lattice. Each lane loads its row's projection values (lane l: orientation l % 16, x pairs
+// 2 (l / 16) of every 8) and forms A in registers, so that the operands of the x contraction
+// (v_mfma_f32_16x16x4_f32: lane l supplies row or column l % 16 at k = l / 16 and receives rows 4 (l / 16) .. + 3 of
+// column l % 16) need neither LDS nor barriers; the column operand is the same for every row, particle and
+// orientation. The results leave through LDS so that whole rows are stored.
+// The lattice form needs 4 (2 M) + 4 (2 M + 1)^2 / s flops per pixel and orientation where the direct cross term needs
+// 4 NT (113 translations, coarse size 54: 57 against 452), which is why FP32 matrix products here are faster than BF16
+// hi+lo products of the direct form, and 6 to 11 times faster than direct squared differences on the vector units.
+// Measured (box 128, 36,864 orientations x 113 translations): 101 particles 81 -> 7.3 ms against direct FP32 squared
+// differences; 151 particles and 4 classes 63.6 -> 44 ms against BF16 hi+lo.
+// grid (tiles, column tiles), dynamic LDS: xtab of the column tile.
+template <int M>
+__global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
+    constexpr bool kZero = M == kColShift;  // the tx = 0 column has no lane: summed beside the others
+    constexpr int kY = 2 * M + 1;
+    __shared__ float s_out[kBlock / 64][4][256];
+    extern __shared__ float2 s_x[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int grp = wave >> 2, wv = wave & 3, gtid = tid & 255;
-    const int ti = kMfG * blockIdx.x + grp;
-    const bool has = ti < n_tiles;
-    const CoarseTile tile = has ? tiles[ti] : CoarseTile{0, 0};
+    const int n = lane & 15, g = lane >> 4;
+    const CoarseTile tile = a.tiles[blockIdx.x];
     const int b = tile.b;
-    const int n_o = has ? or_cnt[b] : 0;
-    const int n_rows = has ? min(kMfO, n_o - tile.o_begin) : 0;  // valid orientations of the tile
-    const int Kc = Kp / 2;  // complex slots per row
-    if (gtid < kMfO) og_s[grp][gtid] = gtid < n_rows ? or_proj[or_off[b] + tile.o_begin + gtid] : -1;
+    const int n_o = a.or_cnt[b];
+    const int o0 = tile.o_begin + 16 * wave;
+    const int n_rows = max(0, min(16, n_o - o0));
+    const int og = n < n_rows ? a.or_proj[a.or_off[b] + o0 + n] : -1;
+    for (int i = tid; i < a.n_xsteps * 64; i += kBlock) s_x[i] = a.xtab[(size_t)blockIdx.y * a.n_xsteps * 64 + i];
     __syncthreads();
-    floatx4_t acc[4][kTW];
+    const float4 *pr = reinterpret_cast<const float4 *>(og >= 0 ? a.pf + (size_t)og * a.Kc : a.zero_row) + g;
+    const float4 *wr = reinterpret_cast<const float4 *>(a.w + (size_t)b * a.Kc) + g;
+    const float2 *cr = reinterpret_cast<const float2 *>(a.ctf2 + (size_t)b * a.Kc) + g;
+    const float sgn = n < 8 ? 1.f : -1.f;
+    float cc[M + 1][4], cs[M + 1][4];  // cos and sin parts per |ty| of this lane's 4 rows (cs[0] unused)
+    float zc[M + 1], zs[M + 1];        // the tx = 0 column, this lane's share of row n
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int k = 0; k <= M; ++k) {
 #pragma unroll
-        for (int j = 0; j < kTW; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    const int r16 = lane & 15, gq = lane >> 4;
-    const int row_tiles = (n_rows + 15) >> 4;  // row tiles of this wave's group with orientations (uniform)
-    // staging: thread gtid of a group forms the 4 complex slots 16 ks + 4 sq of its tile's row gtid / 4 in K step
-    // ks (8 bf16 of hi and of lo), its projection values loaded one K step ahead
-    const int srow = gtid >> 2, sq = gtid & 3, arow = grp * kMfO + srow;
-    const float4 *st_p;
-    {
-        const int og = og_s[grp][srow];
-        st_p = reinterpret_cast<const float4 *>(og >= 0 ? pf + (size_t)og * Kc : zero_row);
+        for (int r = 0; r < 4; ++r) cc[k][r] = cs[k][r] = 0.f;
+        zc[k] = zs[k] = 0.f;
     }
-    const float4 *wrow = reinterpret_cast<const float4 *>(w + (size_t)b * Kc);
-    const float4 *c2row = reinterpret_cast<const float4 *>(ctf2 + (size_t)b * Kc);
-    float an = 0.f;  // this thread's part of sum_p c_p^2 |P_o(p)|^2 over its row's slots
-    auto stage = [&](float4 p0, float4 p1, int ks, int to) {
-        const float4 w0 = wrow[8 * ks + 2 * sq], w1 = wrow[8 * ks + 2 * sq + 1];
-        const float4 c2 = c2row[4 * ks + sq];
-        an = fmaf(p0.x * p0.x + p0.y * p0.y, c2.x, an);
-        an = fmaf(p0.z * p0.z + p0.w * p0.w, c2.y, an);
-        an = fmaf(p1.x * p1.x + p1.y * p1.y, c2.z, an);
-        an = fmaf(p1.z * p1.z + p1.w * p1.w, c2.w, an);
-        const float2 pv[4] = {make_float2(p0.x, p0.y), make_float2(p0.z, p0.w), make_float2(p1.x, p1.y),
-                              make_float2(p1.z, p1.w)};
-        const float2 wq[4] = {make_float2(w0.x, w0.y), make_float2(w0.z, w0.w), make_float2(w1.x, w1.y),
-                              make_float2(w1.z, w1.w)};
-        unsigned int hh[4], ll[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {  // P conj(w)
-            const float re = pv[m].x * wq[m].x + pv[m].y * wq[m].y;
-            const float im = pv[m].y * wq[m].x - pv[m].x * wq[m].y;
-            split2_bf16(re, im, hh[m], ll[m]);
-        }
-        *reinterpret_cast<uint4 *>(&s_a[to][0][arow * kAStride + 8 * sq]) = make_uint4(hh[0], hh[1], hh[2], hh[3]);
-        *reinterpret_cast<uint4 *>(&s_a[to][1][arow * kAStride + 8 * sq]) = make_uint4(ll[0], ll[1], ll[2], ll[3]);
+    float an = 0.f;  // this lane's share of sum_p c_p^2 |P_o(p)|^2 of row n
+    float4 pp, pm, wp, wm;
+    float2 cp, cm;
+    auto load = [&](int st) {  // step st of the layout: 8 float4 of complex pairs, 4 of row y and 4 of row -y
+        pp = pr[8 * st];
+        pm = pr[8 * st + 4];
+        wp = wr[8 * st];
+        wm = wr[8 * st + 4];
+        cp = cr[8 * st];
+        cm = cr[8 * st + 4];
     };
-    int tt[kTW];
-#pragma unroll
-    for (int j = 0; j < kTW; ++j) {
-        const int t = 16 * (wv + 4 * j) + r16;
-        tt[j] = ((wv + 4 * j) < NTT && t < NT) ? t : -1;
-    }
-    // projection values of kPre K steps in flight: register set d holds step ks with ks % kPre == d
-    constexpr int kPre = 3;
-    const int nK = Kp / 32;
-    float4 pa[kPre][2];
-#pragma unroll
-    for (int d = 0; d < kPre; ++d) {
-        pa[d][0] = d < nK ? st_p[8 * d + 2 * sq] : make_float4(0.f, 0.f, 0.f, 0.f);
-        pa[d][1] = d < nK ? st_p[8 * d + 2 * sq + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    stage(pa[0][0], pa[0][1], 0, 0);
-    __syncthreads();
-    for (int ks0 = 0; ks0 < nK; ks0 += kPre) {
-#pragma unroll
-        for (int d = 0; d < kPre; ++d) {
-            const int ks = ks0 + d, buf = ks & 1;
-            if (ks >= nK) break;    // uniform over the block
-            if (ks + kPre < nK) {  // set d was staged at the end of step ks - 1: reload it for step ks + kPre
-                pa[d][0] = st_p[8 * (ks + kPre) + 2 * sq];
-                pa[d][1] = st_p[8 * (ks + kPre) + 2 * sq + 1];
-            }
-
-            if (row_tiles > 0) {
-                bf16x8_t ah[4], al[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int row = grp * kMfO + 16 * i + r16;
-                    ah[i] = __builtin_bit_cast(
-                        bf16x8_t, *reinterpret_cast<const uint4 *>(&s_a[buf][0][row * kAStride + 8 * gq]));
-                    al[i] = __builtin_bit_cast(
-                        bf16x8_t, *reinterpret_cast<const uint4 *>(&s_a[buf][1][row * kAStride + 8 * gq]));
+    auto norm = [&](const float4 &p, const float2 &c2) {
+        an = fmaf(p.x * p.x + p.y * p.y, c2.x, an);
+        an = fmaf(p.z * p.z + p.w * p.w, c2.y, an);
+    };
+    const int n_steps = a.Kc / 16;
+    if (n_rows > 0 && n_steps > 0) {
+        int st = 0;
+        load(0);
+        for (int k = 0; k < a.n_pairs; ++k) {
+            const int2 pd = a.pairs[k];
+            floatx4_t da = {0.f, 0.f, 0.f, 0.f}, db = da, ea = da, eb = da;
+            float zpa = 0.f, zpb = 0.f, zma = 0.f, zmb = 0.f;
+            for (int j = 0; j < pd.x; ++j) {
+                const float4 p = pp, w = wp, pn = pm, wn = wm;
+                const float2 c = cp, cn = cm;
+                st += 1;
+                if (st < n_steps) load(st);
+                const float2 x = s_x[64 * j + lane];
+                // A = P conj(w)
+                const float a0 = p.x * w.x + p.y * w.y, b0 = p.y * w.x - p.x * w.y;
+                const float a1 = p.z * w.z + p.w * w.w, b1 = p.w * w.z - p.z * w.w;
+                da = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, x.x, da, 0, 0, 0);
+                db = __builtin_amdgcn_mfma_f32_16x16x4f32(b0, x.x, db, 0, 0, 0);
+                da = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, x.y, da, 0, 0, 0);
+                db = __builtin_amdgcn_mfma_f32_16x16x4f32(b1, x.y, db, 0, 0, 0);
+                norm(p, c);
+                if (kZero) {
+                    zpa += a0 + a1;
+                    zpb += b0 + b1;
                 }
-                const int slot = 16 * ks + 4 * gq;  // this lane's 4 complex slots of the B fragment
-#pragma unroll
-                for (int j = 0; j < kTW; ++j) {
-                    if (wv + 4 * j >= NTT) continue;
-                    uint4 hv = make_uint4(0u, 0u, 0u, 0u), lv = hv;
-                    if (tt[j] >= 0) {
-                        hv = *reinterpret_cast<const uint4 *>(ehi + (size_t)tt[j] * Kc + slot);
-                        lv = *reinterpret_cast<const uint4 *>(elo + (size_t)tt[j] * Kc + slot);
-                    }
-                    const bf16x8_t bh = __builtin_bit_cast(bf16x8_t, hv);
-                    const bf16x8_t bl = __builtin_bit_cast(bf16x8_t, lv);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (i >= row_tiles) continue;
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh, acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl, acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, acc[i][j], 0, 0, 0);
+                if (pd.y) {
+                    const float a2 = pn.x * wn.x + pn.y * wn.y, b2 = pn.y * wn.x - pn.x * wn.y;
+                    const float a3 = pn.z * wn.z + pn.w * wn.w, b3 = pn.w * wn.z - pn.z * wn.w;
+                    ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, x.x, ea, 0, 0, 0);
+                    eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b2, x.x, eb, 0, 0, 0);
+                    ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a3, x.y, ea, 0, 0, 0);
+                    eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b3, x.y, eb, 0, 0, 0);
+                    norm(pn, cn);
+                    if (kZero) {
+                        zma += a2 + a3;
+                        zmb += b2 + b3;
                     }
                 }
             }
-            // the other buffer was last read in the previous step, before the barrier that ended it
-            if (ks + 1 < nK) stage(pa[(d + 1) % kPre][0], pa[(d + 1) % kPre][1], ks + 1, buf ^ 1);
-            __syncthreads();
-        }
-    }
-    an += __shfl_xor(an, 1);  // the 4 threads of a row are consecutive lanes
-    an += __shfl_xor(an, 2);
-    if (sq == 0) a_norm[grp][srow] = an;
-    __syncthreads();
-    if (!has) return;
-    const float base = xi2half[b] + (float)ynorm[b];
-    float *out = diff2 + d2_off[b];
-    float mn = 3.0e38f;  // minimum of the non-negative values written, for the weights' exponent offset
-#pragma unroll
-    for (int j = 0; j < kTW; ++j) {
-        if (tt[j] < 0) continue;
-        const int t = tt[j];  // D column
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
+            const float *yt = a.ytab + (size_t)k * kY;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int oo = 16 * i + gq * 4 + r;  // D row within the tile
-                if (oo >= n_rows) continue;
-                const float v = og_s[grp][oo] < 0 ? -999.f : base + a_norm[grp][oo] - 2.f * acc[i][j][r];
-                out[(size_t)(tile.o_begin + oo) * NT + t] = v;
+                // cos lanes (+tx): U = Sa + Sb', V = Tb - Ta'; sin lanes (-tx): U = Sa' - Sb, V = Tb' + Ta, primes
+                // from the partner lane, S and T the sum and difference of rows y and -y
+                const float su = n < 8 ? da[r] + ea[r] : db[r] + eb[r];
+                const float sv = n < 8 ? db[r] - eb[r] : da[r] - ea[r];
+                const float U = fmaf(sgn, su, dpp_ror8(su)), V = fmaf(-sgn, dpp_ror8(sv), sv);
+                cc[0][r] += yt[0] * U;
+#pragma unroll
+                for (int m = 1; m <= M; ++m) {
+                    cc[m][r] = fmaf(yt[m], U, cc[m][r]);
+                    cs[m][r] = fmaf(yt[M + m], V, cs[m][r]);
+                }
+            }
+            if (kZero) {
+                const float U = zpa + zma, V = zpb - zmb;
+                zc[0] += yt[0] * U;
+#pragma unroll
+                for (int m = 1; m <= M; ++m) {
+                    zc[m] = fmaf(yt[m], U, zc[m]);
+                    zs[m] = fmaf(yt[M + m], V, zs[m]);
+                }
+            }
+        }
+    }
+    an += __shfl_xor(an, 16);  // the four lanes of row n
+    an += __shfl_xor(an, 32);
+    if (kZero) {
+#pragma unroll
+        for (int m = 0; m <= M; ++m) {
+            zc[m] += __shfl_xor(zc[m], 16);
+            zc[m] += __shfl_xor(zc[m], 32);
+            zs[m] += __shfl_xor(zs[m], 16);
+            zs[m] += __shfl_xor(zs[m], 32);
+        }
+    }
+    const double base = (double)a.xi2half[b] + a.ynorm[b];
+    const CoarseColumn col = a.cols[16 * blockIdx.y + n];
+    CoarseColumn zcol{0, -1};
+    if (kZero) zcol = a.cols[16 * gridDim.y];
+    float *out = a.diff2 + a.d2_off[b];
+    float mn = 3.0e38f;  // minimum of the non-negative values written, for the weights' exponent offset
+    auto value = [&](float norm2, float cross) {
+        const float v = (float)(base + (double)(norm2 - 2.f * cross));
+        return v < 0.f ? 0.f : v;  // rounding of a match without noise; NaN stays
+    };
+    float (*so)[256] = s_out[wave];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        // rows 4 g + r of the four lane groups; row n of the zero column's lanes is one of them when n % 4 == r
+        const float nr = __shfl(an, 4 * g + r);
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m <= M; ++m) {
+            if (m <= col.half) {
+                so[g][col.t0 + m] = value(nr, cc[m][r] + cs[m][r]);
+                if (m > 0) so[g][col.t0 - m] = value(nr, cc[m][r] - cs[m][r]);
+            }
+            if (kZero && g == 0 && (n & 3) == r && m <= zcol.half) {
+                so[n >> 2][zcol.t0 + m] = value(an, zc[m] + zs[m]);
+                if (m > 0) so[n >> 2][zcol.t0 - m] = value(an, zc[m] - zs[m]);
+            }
+        }
+        __syncthreads();
+        for (int gg = 0; gg < 4; ++gg) {
+            const int row = 4 * gg + r;
+            if (row >= n_rows) break;
+            const bool off = __shfl(og, row) < 0;  // orientation or class without prior: never evaluated
+            for (int t = lane; t < a.NT; t += 64) {
+                if (a.tile_of && a.tile_of[t] != (int)blockIdx.y) continue;
+                const float v = off ? -999.f : so[gg][t];
+                out[(size_t)(o0 + row) * a.NT + t] = v;
                 if (v >= 0.f) mn = fminf(mn, v);
             }
+        }
     }
     for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o));
     // sign bit cleared: -0 orders as +0 among the unsigned bit patterns of non-negative floats
-    if (lane == 0 && mn < 3.0e38f) atomicMin(&part[b].mn_bits, __float_as_uint(mn) & 0x7fffffffu);
+    if (lane == 0 && mn < 3.0e38f) atomicMin(&a.part[b].mn_bits, __float_as_uint(mn) & 0x7fffffffu);
 }
 
 // --------------------------------------------------------------------------------------------------
@@ -1071,25 +942,6 @@ __global__ void __launch_bounds__(kBlock) k_wpart_init(WPart *__restrict__ part,
     WPart p{};
     p.mn_bits = 0x7f800000u;  // +inf
     part[b] = p;
-}
-
-__global__ void __launch_bounds__(kBlock) k_wseg_min(WeightArgs a, const WSeg *__restrict__ segs,
-                                                     WPart *__restrict__ part) {
-    __shared__ float red[kBlock / 64];
-    const WSeg sg = segs[blockIdx.x];
-    const float *d2 = a.diff2 + a.d2_off[sg.b];
-    float mn = 3.0e38f;
-    for (long long e = sg.begin + threadIdx.x; e < sg.end; e += kBlock) {
-        const float v = d2[e];
-        if (v >= 0.f) mn = fminf(mn, v);
-    }
-    for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mn;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kBlock / 64; ++w) mn = fminf(mn, red[w]);
-        if (mn < 3.0e38f) atomicMin(&part[sg.b].mn_bits, __float_as_uint(mn) & 0x7fffffffu);
-    }
 }
 
 // Weights of one segment, their sum, and the first radix pass of the selection (the top byte of every positive
