@@ -190,10 +190,10 @@ struct Engine {
     // constant tables
     DevBuf d_frames_c, d_frames_f;
     // coarse pass (k_coarse_lattice): projections and a zero row, particle rows per chunk, the pixel layout's groups
-    // and row pairs, phases of the lattice's y and x shifts and its columns
-    DevBuf d_pf, d_zero_row, d_wc, d_ctf2, d_ynorm, d_grp, d_pairs_c, d_ytab, d_xtab, d_cols, d_tile_of;
+    // and steps, phases of the lattice's y and x shifts and its columns
+    DevBuf d_pf, d_zero_row, d_wc, d_ctf2, d_ynorm, d_grp, d_steps, d_ytab, d_xtab, d_cols, d_tile_of;
     int Kc = 0;                                     // complex slots per projection
-    int n_pairs_c = 0, n_xsteps = 0;                // row pairs; steps of the longest row
+    int n_steps = 0, n_xsteps = 0;                  // steps of the layout; steps of the longest row
     int mshift = 0, col_tiles = 1;                  // positive shifts of the lattice; column tiles
     DevBuf d_q_c, d_q_f, d_minv_w, d_mresol, d_xa_shell;
     DevBuf d_ex_f, d_ey_f, d_tr_ix, d_tr_iy, d_over_x, d_over_y;
@@ -400,7 +400,7 @@ static int lattice_columns(Engine &e) {
 static int coarse_layout(Engine &e, const std::vector<float> &qc) {
     const int s = e.igc.s, xs = e.igc.xs, m = e.mshift;
     const double N = e.cfg.ori_size, px = e.cfg.pixel_size;
-    std::vector<int2> grp, pairs;
+    std::vector<int2> grp, steps;
     std::vector<float> ytab;
     e.n_xsteps = 0;
     // cos and -sin of 2 pi k shift / N, the phase reduced in turns before the trigonometry
@@ -414,18 +414,22 @@ static int coarse_layout(Engine &e, const std::vector<float> &qc) {
         int xmax = -1;
         for (int x = 0; x < xs; ++x)
             if (qc[(size_t)y * xs + x] != 0.f || (minus && qc[(size_t)(s - y) * xs + x] != 0.f)) xmax = x;
-        const int steps = (xmax + 8) / 8;
-        if (steps == 0) continue;
-        for (int j = 0; j < steps; ++j) {
+        const int n = (xmax + 8) / 8;
+        if (n == 0) continue;
+        for (int j = 0; j < n; ++j) {
             grp.push_back(make_int2(y, 8 * j));
             grp.push_back(make_int2(minus ? s - y : -1, 8 * j));
+            steps.push_back(make_int2(64 * j, (minus ? rlnk::kStepMinus : 0) | (j + 1 == n ? rlnk::kStepEnd : 0)));
         }
-        pairs.push_back(make_int2(steps, minus ? 1 : 0));
         for (int k = 0; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).x);
         for (int k = 1; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).y);
-        e.n_xsteps = std::max(e.n_xsteps, steps);
+        e.n_xsteps = std::max(e.n_xsteps, n);
     }
-    e.n_pairs_c = (int)pairs.size();
+    if (steps.size() & 1) {
+        grp.insert(grp.end(), 2, make_int2(-1, 0));
+        steps.push_back(make_int2(0, 0));
+    }
+    e.n_steps = (int)steps.size();
     e.Kc = 8 * (int)grp.size();
     std::vector<float2> xtab((size_t)e.col_tiles * e.n_xsteps * 64);
     for (int ct = 0; ct < e.col_tiles; ++ct)
@@ -442,7 +446,7 @@ static int coarse_layout(Engine &e, const std::vector<float> &qc) {
                 xtab[((size_t)ct * e.n_xsteps + j) * 64 + l] = v;
             }
     RLN_TRY(upload(e.d_grp, grp, e.stream));
-    RLN_TRY(upload(e.d_pairs_c, pairs, e.stream));
+    RLN_TRY(upload(e.d_steps, steps, e.stream));
     RLN_TRY(upload(e.d_ytab, ytab, e.stream));
     RLN_TRY(upload(e.d_xtab, xtab, e.stream));
     return upload(e.d_zero_row, std::vector<float2>(std::max(e.Kc, 1), make_float2(0.f, 0.f)), e.stream);
@@ -1307,12 +1311,12 @@ static int launch_coarse(Engine &e, unsigned n_tiles, const float *xi2, const lo
     a.ynorm = e.d_ynorm.as<const double>();
     a.xi2half = xi2;
     a.d2_off = d2off;
-    a.pairs = e.d_pairs_c.as<const int2>();
+    a.steps = e.d_steps.as<const int2>();
     a.ytab = e.d_ytab.as<const float>();
     a.xtab = e.d_xtab.as<const float2>();
     a.cols = e.d_cols.as<const rlnk::CoarseColumn>();
     a.tile_of = e.col_tiles > 1 ? e.d_tile_of.as<const int>() : nullptr;
-    a.n_pairs = e.n_pairs_c;
+    a.n_steps = e.n_steps;
     a.n_xsteps = e.n_xsteps;
     a.NT = e.NT;
     a.Kc = e.Kc;
@@ -2011,7 +2015,7 @@ extern "C" int rln_estep_destroy(rln_estep *e) {
     (void)hipSetDevice(e->device);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     rln::DevBuf *bufs[] = {&e->d_frames_c, &e->d_frames_f, &e->d_pf, &e->d_zero_row, &e->d_wc, &e->d_ctf2, &e->d_ynorm,
-                           &e->d_grp, &e->d_pairs_c, &e->d_ytab, &e->d_xtab, &e->d_cols, &e->d_tile_of, &e->d_q_c,
+                           &e->d_grp, &e->d_steps, &e->d_ytab, &e->d_xtab, &e->d_cols, &e->d_tile_of, &e->d_q_c,
                            &e->d_q_f, &e->d_minv_w, &e->d_mresol, &e->d_xa_shell, &e->d_ex_f, &e->d_ey_f,
                            &e->d_tr_ix, &e->d_tr_iy, &e->d_over_x, &e->d_over_y, &e->d_vols, &e->d_bp_ptrs,
                            &e->d_fimg, &e->d_fimgn, &e->d_fctf, &e->d_meta_f, &e->d_meta_d, &e->d_meta_ll,

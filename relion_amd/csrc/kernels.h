@@ -137,8 +137,8 @@ __global__ void k_selftest_mfma(const float *__restrict__ A, const float *__rest
 //
 // Pixel layout of that contraction: per row pair (y, -y), y = 0 .. s/2, steps of 16 complex slots: 8 consecutive x of
 // row y, then the same 8 of row -y (zeros where there is no such row); a pair has steps up to its last pixel whose
-// Minvsigma2 is non-zero, so rows and corners that carry no weight are not contracted. grp holds (row, x0) of every 8
-// slots (row -1: none). Kc = 16 * steps complex slots per projection.
+// Minvsigma2 is non-zero, so rows and corners that carry no weight are not contracted. An empty step makes their number
+// even. grp holds (row, x0) of every 8 slots (row -1: zeros). Kc = 16 * steps complex slots per projection.
 // --------------------------------------------------------------------------------------------------
 
 // Projections of every coarse orientation of every class in that layout: FP32 complex pf [K*n_or][Kc].
@@ -234,6 +234,8 @@ struct CoarseColumn {
     int half;  // ty = -half .. half exist, -1: no column
 };
 constexpr int kColShift = 8;
+constexpr int kStepMinus = 1, kStepEnd = 2;  // the step has a row -y; it is the last of its row pair
+constexpr int kStepChunk = 64;               // steps whose particle rows are staged in LDS at a time (even)
 
 struct CoarseArgs {
     const CoarseTile *tiles;
@@ -245,16 +247,21 @@ struct CoarseArgs {
     const double *ynorm;
     const float *xi2half;
     const long long *d2_off;
-    const int2 *pairs;        // row pairs: (steps, 1 with a row -y)
+    const int2 *steps;        // [n_steps] (offset of the step's x phases in xtab, flags: kStepMinus | kStepEnd)
     const float *ytab;        // per row pair: cos(2 pi y ty / N) for ty = 0 .. M, -sin for ty = 1 .. M
     const float2 *xtab;       // [column tile][step of a row][lane]: the two x phases of the lane's column
     const CoarseColumn *cols; // [column tile][16], then the tx = 0 column of M == 8
     const int *tile_of;       // column tile of each translation, null with one tile
-    int n_pairs, n_xsteps;
+    int n_steps, n_xsteps;    // n_steps even
     int NT, Kc;
     float *diff2;
     WPart *part;
 };
+
+// Tables read at wave-uniform addresses, in the constant address space: scalar loads, which do not queue behind the
+// projection values in flight.
+typedef const __attribute__((address_space(4))) float *UniformF;
+typedef const __attribute__((address_space(4))) int *UniformI;
 
 // Value of the lane 8 further in its row of 16 lanes.
 __device__ __forceinline__ float dpp_ror8(float v) {
@@ -265,21 +272,33 @@ __device__ __forceinline__ float dpp_ror8(float v) {
 // of positive shifts of the lattice. Each lane loads its row's projection values (lane l: orientation l % 16, x pairs
 // 2 (l / 16) of every 8) and forms A in registers, so that the operands of the x contraction
 // (v_mfma_f32_16x16x4_f32: lane l supplies row or column l % 16 at k = l / 16 and receives rows 4 (l / 16) .. + 3 of
-// column l % 16) need neither LDS nor barriers; the column operand is the same for every row, particle and
-// orientation. The results leave through LDS so that whole rows are stored.
+// column l % 16) go from memory to the matrix units through registers alone; the column operand is the same for every
+// row, particle and orientation. The particle's rows, shared by the block, are staged in LDS: read from memory by every
+// wave they took more of the vector memory path than the projections (busy 81% of the time). The steps alternate
+// between two register sets, the next step's loads in flight. The results leave through LDS so that whole rows are
+// stored. Bound by the FP32 matrix rate and the vector instructions that form A, about evenly.
 // The lattice form needs 4 (2 M) + 4 (2 M + 1)^2 / s flops per pixel and orientation where the direct cross term needs
 // 4 NT (113 translations, coarse size 54: 57 against 452), which is why FP32 matrix products here are faster than BF16
-// hi+lo products of the direct form, and 6 to 11 times faster than direct squared differences on the vector units.
-// Measured (box 128, 36,864 orientations x 113 translations): 101 particles 81 -> 7.3 ms against direct FP32 squared
-// differences; 151 particles and 4 classes 63.6 -> 44 ms against BF16 hi+lo.
+// hi+lo products of the direct form, and much faster than direct squared differences on the vector units.
+// Measured (box 128, coarse size 54, 36,864 orientations x 113 translations): 101 particles 5.4 ms (81 ms with direct
+// FP32 squared differences, 7.3 ms without the staged rows), 151 particles and 4 classes 31.9 ms (63.6 ms with BF16
+// hi+lo products of the direct cross term): 79 G poses/s. Reading all LDS operands of a step at once and running the
+// missing row -y on zeros instead of a branch costs 16 registers, one wave per SIMD and 4 to 10% of the time.
 // grid (tiles, column tiles), dynamic LDS: xtab of the column tile.
 template <int M>
 __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
     constexpr bool kZero = M == kColShift;  // the tx = 0 column has no lane: summed beside the others
     constexpr int kY = 2 * M + 1;
-    __shared__ float s_out[kBlock / 64][4][256];
+    __shared__ union {
+        struct {
+            float4 w[8 * kStepChunk];
+            float2 c[8 * kStepChunk];
+        } in;
+        float out[kBlock / 64][4][256];
+    } lds;
     extern __shared__ float2 s_x[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform, and so is what follows from it
     const int n = lane & 15, g = lane >> 4;
     const CoarseTile tile = a.tiles[blockIdx.x];
     const int b = tile.b;
@@ -288,10 +307,9 @@ __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
     const int n_rows = max(0, min(16, n_o - o0));
     const int og = n < n_rows ? a.or_proj[a.or_off[b] + o0 + n] : -1;
     for (int i = tid; i < a.n_xsteps * 64; i += kBlock) s_x[i] = a.xtab[(size_t)blockIdx.y * a.n_xsteps * 64 + i];
-    __syncthreads();
     const float4 *pr = reinterpret_cast<const float4 *>(og >= 0 ? a.pf + (size_t)og * a.Kc : a.zero_row) + g;
-    const float4 *wr = reinterpret_cast<const float4 *>(a.w + (size_t)b * a.Kc) + g;
-    const float2 *cr = reinterpret_cast<const float2 *>(a.ctf2 + (size_t)b * a.Kc) + g;
+    const float4 *wr = reinterpret_cast<const float4 *>(a.w + (size_t)b * a.Kc);
+    const float2 *cr = reinterpret_cast<const float2 *>(a.ctf2 + (size_t)b * a.Kc);
     const float sgn = n < 8 ? 1.f : -1.f;
     float cc[M + 1][4], cs[M + 1][4];  // cos and sin parts per |ty| of this lane's 4 rows (cs[0] unused)
     float zc[M + 1], zs[M + 1];        // the tx = 0 column, this lane's share of row n
@@ -302,84 +320,93 @@ __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
         zc[k] = zs[k] = 0.f;
     }
     float an = 0.f;  // this lane's share of sum_p c_p^2 |P_o(p)|^2 of row n
-    float4 pp, pm, wp, wm;
-    float2 cp, cm;
-    auto load = [&](int st) {  // step st of the layout: 8 float4 of complex pairs, 4 of row y and 4 of row -y
-        pp = pr[8 * st];
-        pm = pr[8 * st + 4];
-        wp = wr[8 * st];
-        wm = wr[8 * st + 4];
-        cp = cr[8 * st];
-        cm = cr[8 * st + 4];
-    };
+    floatx4_t da = {0.f, 0.f, 0.f, 0.f}, db = da, ea = da, eb = da;
+    float zpa = 0.f, zpb = 0.f, zma = 0.f, zmb = 0.f;
+    UniformF yt = (UniformF)a.ytab;
+    UniformI steps = (UniformI)a.steps;
     auto norm = [&](const float4 &p, const float2 &c2) {
         an = fmaf(p.x * p.x + p.y * p.y, c2.x, an);
         an = fmaf(p.z * p.z + p.w * p.w, c2.y, an);
     };
-    const int n_steps = a.Kc / 16;
-    if (n_rows > 0 && n_steps > 0) {
-        int st = 0;
-        load(0);
-        for (int k = 0; k < a.n_pairs; ++k) {
-            const int2 pd = a.pairs[k];
-            floatx4_t da = {0.f, 0.f, 0.f, 0.f}, db = da, ea = da, eb = da;
-            float zpa = 0.f, zpb = 0.f, zma = 0.f, zmb = 0.f;
-            for (int j = 0; j < pd.x; ++j) {
-                const float4 p = pp, w = wp, pn = pm, wn = wm;
-                const float2 c = cp, cn = cm;
-                st += 1;
-                if (st < n_steps) load(st);
-                const float2 x = s_x[64 * j + lane];
-                // A = P conj(w)
-                const float a0 = p.x * w.x + p.y * w.y, b0 = p.y * w.x - p.x * w.y;
-                const float a1 = p.z * w.z + p.w * w.w, b1 = p.w * w.z - p.z * w.w;
-                da = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, x.x, da, 0, 0, 0);
-                db = __builtin_amdgcn_mfma_f32_16x16x4f32(b0, x.x, db, 0, 0, 0);
-                da = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, x.y, da, 0, 0, 0);
-                db = __builtin_amdgcn_mfma_f32_16x16x4f32(b1, x.y, db, 0, 0, 0);
-                norm(p, c);
-                if (kZero) {
-                    zpa += a0 + a1;
-                    zpb += b0 + b1;
-                }
-                if (pd.y) {
-                    const float a2 = pn.x * wn.x + pn.y * wn.y, b2 = pn.y * wn.x - pn.x * wn.y;
-                    const float a3 = pn.z * wn.z + pn.w * wn.w, b3 = pn.w * wn.z - pn.z * wn.w;
-                    ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a2, x.x, ea, 0, 0, 0);
-                    eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b2, x.x, eb, 0, 0, 0);
-                    ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a3, x.y, ea, 0, 0, 0);
-                    eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b3, x.y, eb, 0, 0, 0);
-                    norm(pn, cn);
-                    if (kZero) {
-                        zma += a2 + a3;
-                        zmb += b2 + b3;
-                    }
-                }
-            }
-            const float *yt = a.ytab + (size_t)k * kY;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                // cos lanes (+tx): U = Sa + Sb', V = Tb - Ta'; sin lanes (-tx): U = Sa' - Sb, V = Tb' + Ta, primes
-                // from the partner lane, S and T the sum and difference of rows y and -y
-                const float su = n < 8 ? da[r] + ea[r] : db[r] + eb[r];
-                const float sv = n < 8 ? db[r] - eb[r] : da[r] - ea[r];
-                const float U = fmaf(sgn, su, dpp_ror8(su)), V = fmaf(-sgn, dpp_ror8(sv), sv);
-                cc[0][r] += yt[0] * U;
-#pragma unroll
-                for (int m = 1; m <= M; ++m) {
-                    cc[m][r] = fmaf(yt[m], U, cc[m][r]);
-                    cs[m][r] = fmaf(yt[M + m], V, cs[m][r]);
-                }
-            }
+    // one step: 4 float4 of complex pairs of row y (pp) and of row -y (pm); st within the staged chunk
+    auto step = [&](const float4 &pp, const float4 &pm, int st, int xoff, int flags) {
+        const float2 x = s_x[xoff + lane];
+        {
+            const float4 w = lds.in.w[8 * st + g];
+            // A = P conj(w)
+            const float a0 = pp.x * w.x + pp.y * w.y, b0 = pp.y * w.x - pp.x * w.y;
+            const float a1 = pp.z * w.z + pp.w * w.w, b1 = pp.w * w.z - pp.z * w.w;
+            da = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, x.x, da, 0, 0, 0);
+            db = __builtin_amdgcn_mfma_f32_16x16x4f32(b0, x.x, db, 0, 0, 0);
+            da = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, x.y, da, 0, 0, 0);
+            db = __builtin_amdgcn_mfma_f32_16x16x4f32(b1, x.y, db, 0, 0, 0);
+            norm(pp, lds.in.c[8 * st + g]);
             if (kZero) {
-                const float U = zpa + zma, V = zpb - zmb;
-                zc[0] += yt[0] * U;
-#pragma unroll
-                for (int m = 1; m <= M; ++m) {
-                    zc[m] = fmaf(yt[m], U, zc[m]);
-                    zs[m] = fmaf(yt[M + m], V, zs[m]);
-                }
+                zpa += a0 + a1;
+                zpb += b0 + b1;
             }
+        }
+        if (flags & kStepMinus) {
+            const float4 w = lds.in.w[8 * st + 4 + g];
+            const float a0 = pm.x * w.x + pm.y * w.y, b0 = pm.y * w.x - pm.x * w.y;
+            const float a1 = pm.z * w.z + pm.w * w.w, b1 = pm.w * w.z - pm.z * w.w;
+            ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, x.x, ea, 0, 0, 0);
+            eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b0, x.x, eb, 0, 0, 0);
+            ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, x.y, ea, 0, 0, 0);
+            eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b1, x.y, eb, 0, 0, 0);
+            norm(pm, lds.in.c[8 * st + 4 + g]);
+            if (kZero) {
+                zma += a0 + a1;
+                zmb += b0 + b1;
+            }
+        }
+        if (!(flags & kStepEnd)) return;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            // cos lanes (+tx): U = Sa + Sb', V = Tb - Ta'; sin lanes (-tx): U = Sa' - Sb, V = Tb' + Ta, primes from
+            // the partner lane, S and T the sum and difference of rows y and -y
+            const float su = n < 8 ? da[r] + ea[r] : db[r] + eb[r];
+            const float sv = n < 8 ? db[r] - eb[r] : da[r] - ea[r];
+            const float U = fmaf(sgn, su, dpp_ror8(su)), V = fmaf(-sgn, dpp_ror8(sv), sv);
+            cc[0][r] = fmaf(yt[0], U, cc[0][r]);
+#pragma unroll
+            for (int m = 1; m <= M; ++m) {
+                cc[m][r] = fmaf(yt[m], U, cc[m][r]);
+                cs[m][r] = fmaf(yt[M + m], V, cs[m][r]);
+            }
+        }
+        if (kZero) {
+            const float U = zpa + zma, V = zpb - zmb;
+            zc[0] = fmaf(yt[0], U, zc[0]);
+#pragma unroll
+            for (int m = 1; m <= M; ++m) {
+                zc[m] = fmaf(yt[m], U, zc[m]);
+                zs[m] = fmaf(yt[M + m], V, zs[m]);
+            }
+            zpa = zpb = zma = zmb = 0.f;
+        }
+        da = db = ea = eb = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        yt += kY;
+    };
+    for (int s0 = 0; s0 < a.n_steps; s0 += kStepChunk) {
+        const int ns = min(kStepChunk, a.n_steps - s0);
+        __syncthreads();  // the previous chunk's rows were read (and s_x is written, first time)
+        for (int i = tid; i < 8 * ns; i += kBlock) {
+            lds.in.w[i] = wr[8 * s0 + i];
+            lds.in.c[i] = cr[8 * s0 + i];
+        }
+        __syncthreads();
+        if (n_rows == 0) continue;  // uniform over the wave
+        const float4 *p = pr + 8 * s0;
+        float4 p0 = p[0], m0 = p[4], p1, m1;
+        for (int st = 0; st < ns; st += 2) {
+            p1 = p[8 * st + 8];
+            m1 = p[8 * st + 12];
+            step(p0, m0, st, steps[2 * (s0 + st)], steps[2 * (s0 + st) + 1]);
+            const int nx = min(st + 2, ns - 1);  // the last load is repeated, not used
+            p0 = p[8 * nx];
+            m0 = p[8 * nx + 4];
+            step(p1, m1, st + 1, steps[2 * (s0 + st) + 2], steps[2 * (s0 + st) + 3]);
         }
     }
     an += __shfl_xor(an, 16);  // the four lanes of row n
@@ -403,7 +430,8 @@ __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
         const float v = (float)(base + (double)(norm2 - 2.f * cross));
         return v < 0.f ? 0.f : v;  // rounding of a match without noise; NaN stays
     };
-    float (*so)[256] = s_out[wave];
+    float (*so)[256] = lds.out[wave];
+    __syncthreads();  // the staged rows were read
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         // rows 4 g + r of the four lane groups; row n of the zero column's lanes is one of them when n % 4 == r
