@@ -223,7 +223,7 @@ struct Engine {
     long long need_pairs = 0;
     int need_jobs = 0, need_small = 0, need_wide = 0;
     DevBuf d_plan, d_cp, d_items_s, d_items_w;
-    DevBuf d_wsegs, d_seg_first, d_wpart, d_hcnt, d_hsum, d_wcand, d_segbest, d_ocnt;  // segmented coarse weights
+    DevBuf d_wsegs, d_seg_first, d_wpart, d_hcnt, d_hsum, d_wcand, d_wcand_i, d_segbest, d_ocnt;  // coarse weights
     PinnedBuf h_stage[2];  // a chunk's lists packed for upload, alternating between consecutive chunks
     std::unique_ptr<ChunkHost> chunk_host[2];  // host lists of consecutive chunks, kept to reuse their memory
     rlnk::ChunkPtrs cp_host{};
@@ -672,7 +672,7 @@ struct ChunkHost {
     std::vector<float> xi2half, scale, scale_w;
     std::vector<double> old_off, prior_off;
     HostList<rlnk::CoarseTile> tiles;
-    HostList<rlnk::WSeg> segs;  // coarse-weight segments (kSegEntries entries each)
+    HostList<rlnk::WSeg> segs;  // coarse-weight segments
     std::vector<int> seg_first;    // [B+1] first segment of each particle
     long long total_entries = 0;
     // per-particle scalars as uploaded, with the chunk capacity cap_B as stride so that their device addresses do
@@ -745,7 +745,9 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
         h.np[b] = np;
         h.or_cnt[b] = K * nd * np;
     }
-    long long tot_or = any_full ? n_grid : 0, d2 = 0, tot_oc = 0;
+    long long tot_or = any_full ? n_grid : 0, d2 = 0, tot_oc = 0, total = 0;
+    for (int b = 0; b < B; ++b) total += (long long)h.or_cnt[b] * NT;
+    const long long seg = rlnk::choose_segment(total);
     std::vector<int> tile_off(B + 1, 0), seg_off(B + 1, 0);
     for (int b = 0; b < B; ++b) {
         h.oc_off[b] = (int)tot_oc;
@@ -760,7 +762,7 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
         h.d2_off[b] = d2;
         d2 += h.n_entries[b];
         tile_off[b + 1] = tile_off[b] + (h.or_cnt[b] + rlnk::kCoTO - 1) / rlnk::kCoTO;
-        const long long ns = std::max(1LL, (h.n_entries[b] + rlnk::kSegEntries - 1) / rlnk::kSegEntries);
+        const long long ns = std::max(1LL, (h.n_entries[b] + seg - 1) / seg);
         seg_off[b + 1] = seg_off[b] + (int)ns;
     }
     h.total_entries = d2;
@@ -904,7 +906,7 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
         const long long n = h.n_entries[b];
         for (int sI = seg_off[b]; sI < seg_off[b + 1]; ++sI) {
             const long long qs = sI - seg_off[b];
-            h.segs[sI] = rlnk::WSeg{b, 0, qs * rlnk::kSegEntries, std::min(n, (qs + 1) * rlnk::kSegEntries)};
+            h.segs[sI] = rlnk::WSeg{b, 0, qs * seg, std::min(n, (qs + 1) * seg)};
         }
         h.xi2half[b] = (float)(m.highres_Xi2 / 2.);
         const double sc = cfg.do_scale_correction ? m.scale : 1.;
@@ -1036,6 +1038,8 @@ struct FineLaunch {
     long long *pair_off, *fine_n, *foff;
     int *job_off, *pairs;
     rlnk::FinePlan *plan;
+    const rlnk::WPart *wpart;
+    const int *sig;
     const unsigned char *mask;
     const long long *d2off;
     const int *or_cnt, *oc_off, *ocnt;
@@ -1061,8 +1065,8 @@ static void launch_plan(Engine &e, const FineLaunch &L) {
     hipStream_t st = e.stream;
     hipLaunchKernelGGL(rlnk::k_fine_plan, dim3(1), dim3(rlnk::kWBlock), 0, st, L.np, L.nj, L.cp, L.cap_pairs,
                        L.cap_jobs, L.pair_off, L.job_off, L.fine_n, L.foff, L.plan);
-    hipLaunchKernelGGL(rlnk::k_write_jobs, dim3(L.grid_B), dim3(rlnk::kWBlock), 0, st, L.mask, L.d2off, L.or_cnt,
-                       L.oc_off, L.ocnt, L.NT,
+    hipLaunchKernelGGL(rlnk::k_write_jobs, dim3(L.grid_B), dim3(rlnk::kWBlock), 0, st, L.wpart, L.sig, L.mask, L.d2off,
+                       L.or_cnt, L.oc_off, L.ocnt, L.NT,
                        (const long long *)L.pair_off, (const int *)L.job_off, L.pairs, L.jobs,
                        (const rlnk::FinePlan *)L.plan);
     const rlnk::FineShape sh = rlnk::kFineShapes[L.shape];
@@ -1415,7 +1419,7 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     RLN_TRY(launch_check("k_prep_coarse"));
     HIP_TRY(hipEventRecord(e.ev[kStCoarse], st));
     RLN_TRY(e.d_diff2.ensure(sizeof(float) * std::max<long long>(1, h.total_entries)));
-    RLN_TRY(e.d_weight.ensure(sizeof(double) * std::max<long long>(1, h.total_entries)));
+    if (e.keep) RLN_TRY(e.d_weight.ensure(sizeof(double) * std::max<long long>(1, h.total_entries)));
     RLN_TRY(e.d_mask.ensure(std::max<long long>(1, h.total_entries)));
     // per-particle selection state; the coarse kernel folds the minimum diff2 into it as it writes
     const unsigned gB = (unsigned)((B + rlnk::kBlock - 1) / rlnk::kBlock);
@@ -1424,66 +1428,65 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     if (!h.tiles.empty()) RLN_TRY(launch_coarse(e, (unsigned)h.tiles.size(), d_xi2, d_d2off.as<const long long>()));
     HIP_TRY(hipEventRecord(e.ev[kStCoarseW], st));
     RLN_TRY(e.d_stats_c.ensure(sizeof(rlnk::PassStats) * B));
-    rlnk::WeightArgs wa{};
-    wa.diff2 = e.d_diff2.as<const float>();
-    wa.d2_off = d_d2off.as<const long long>();
-    wa.n_entries = d_nent_tmp.as<const long long>();
-    wa.or_prior = e.d_or_prior.as<const double>();
-    wa.or_off = e.d_or_off.as<const int>();
-    wa.oc_off = e.d_oc_off.as<const int>();
-    wa.tr_prior = e.d_tr_prior.as<const double>();
-    wa.NT = NT;
-    wa.fine = 0;
-    wa.adaptive_fraction = cfg.adaptive_fraction;
-    wa.maxsig = cfg.maximum_significants;
-    wa.weight = e.d_weight.as<double>();
-    wa.mask = e.d_mask.as<unsigned char>();
-    wa.stats = e.d_stats_c.as<rlnk::PassStats>();
-    // coarse weights over segments of kSegEntries poses (multi-block per particle)
+    // coarse weights over segments of the poses (multi-block per particle)
     {
         const unsigned nseg = (unsigned)h.segs.size();
         RLN_TRY(upload_packed(e.d_wsegs, h, kPkSegs, st));
         RLN_TRY(upload_packed(e.d_seg_first, h, kPkSegFirst, st));
-        RLN_TRY(e.d_hcnt.ensure(sizeof(unsigned int) * 256 * B));
-        RLN_TRY(e.d_hsum.ensure(sizeof(double) * 256 * B));
+        RLN_TRY(e.d_hcnt.ensure(sizeof(unsigned int) * rlnk::kExpBins * B));
+        RLN_TRY(e.d_hsum.ensure(sizeof(double) * rlnk::kExpBins * B));
         RLN_TRY(e.d_wcand.ensure(sizeof(double) * rlnk::kGather * B));
+        RLN_TRY(e.d_wcand_i.ensure(sizeof(int) * rlnk::kGather * B));
         RLN_TRY(e.d_segbest.ensure(sizeof(rlnk::WSegBest) * nseg));
-        HIP_TRY(hipMemsetAsync(e.d_hcnt.ptr, 0, sizeof(unsigned int) * 256 * B, st));
-        // per-orientation significant counts and per-particle job counts of the fine pass
-        RLN_TRY(ensure_fine_capacity(e));
         RLN_TRY(e.d_ocnt.ensure(sizeof(int) * std::max<long long>(1, h.total_oc)));
-        HIP_TRY(hipMemsetAsync(e.d_ocnt.ptr, 0, sizeof(int) * std::max<long long>(1, h.total_oc), st));
-        HIP_TRY(hipMemsetAsync(e.d_npairs.as<int>() + cB, 0, sizeof(int) * B, st));
-        HIP_TRY(hipMemsetAsync(e.d_hsum.ptr, 0, sizeof(double) * 256 * B, st));
-        const rlnk::WSeg *sg = e.d_wsegs.as<const rlnk::WSeg>();
-        rlnk::WPart *wp = e.d_wpart.as<rlnk::WPart>();
-        unsigned int *hc = e.d_hcnt.as<unsigned int>();
-        double *hs = e.d_hsum.as<double>();
-        hipLaunchKernelGGL(rlnk::k_wseg_exp, dim3(nseg), dim3(rlnk::kBlock), 0, st, wa, sg, wp, hc, hs);
-        hipLaunchKernelGGL(rlnk::k_wsel_start, dim3(gB), dim3(rlnk::kBlock), 0, st, wa, wp, B);
-        for (int shift = 56; shift >= 0; shift -= 8) {
-            if (shift < 56)  // the top byte's histogram came with the weights
-                hipLaunchKernelGGL(rlnk::k_wseg_hist, dim3(nseg), dim3(rlnk::kBlock), 0, st, wa, sg,
-                                   (const rlnk::WPart *)wp, shift, hc, hs);
-            hipLaunchKernelGGL(rlnk::k_wsel_pick, dim3(gB), dim3(rlnk::kBlock), 0, st, wp, B, shift, hc, hs);
-        }
-        hipLaunchKernelGGL(rlnk::k_wseg_gather, dim3(nseg), dim3(rlnk::kBlock), 0, st, wa, sg, wp,
-                           e.d_wcand.as<double>());
-        hipLaunchKernelGGL(rlnk::k_wsel_final, dim3(B), dim3(rlnk::kWBlock), 0, st, wa, wp,
-                           e.d_wcand.as<const double>());
-        if (wa.maxsig > 0) hipLaunchKernelGGL(rlnk::k_wsel_maxsig, dim3(B), dim3(rlnk::kWBlock), 0, st, wa, wp);
-        hipLaunchKernelGGL(rlnk::k_wseg_mask, dim3(nseg), dim3(rlnk::kBlock), 0, st, wa, sg, wp,
-                           e.d_segbest.as<rlnk::WSegBest>(), e.d_ocnt.as<int>(), e.d_npairs.as<int>() + cB);
-        hipLaunchKernelGGL(rlnk::k_wsel_stats, dim3(gB), dim3(rlnk::kBlock), 0, st, (const rlnk::WPart *)wp,
-                           e.d_seg_first.as<const int>(), e.d_segbest.as<const rlnk::WSegBest>(), B, 0,
-                           e.d_stats_c.as<rlnk::PassStats>(), e.d_npairs.as<int>());
+        RLN_TRY(ensure_fine_capacity(e));
+        HIP_TRY(hipMemsetAsync(e.d_hcnt.ptr, 0, sizeof(unsigned int) * rlnk::kExpBins * B, st));
+        HIP_TRY(hipMemsetAsync(e.d_hsum.ptr, 0, sizeof(double) * rlnk::kExpBins * B, st));
+        rlnk::CoarseWeightArgs wa{};
+        wa.segs = e.d_wsegs.as<const rlnk::WSeg>();
+        wa.seg_first = e.d_seg_first.as<const int>();
+        wa.diff2 = e.d_diff2.as<const float>();
+        wa.d2_off = d_d2off.as<const long long>();
+        wa.n_entries = d_nent_tmp.as<const long long>();
+        wa.or_prior = e.d_or_prior.as<const double>();
+        wa.or_off = e.d_or_off.as<const int>();
+        wa.or_cnt = e.d_or_cnt.as<const int>();
+        wa.oc_off = e.d_oc_off.as<const int>();
+        wa.tr_prior = e.d_tr_prior.as<const double>();
+        wa.NT = NT;
+        // priors are normalised by their means over at most all orientations and over the translations
+        wa.prior_max = 1.001 * K * (double)e.n_or * NT;
+        wa.adaptive_fraction = cfg.adaptive_fraction;
+        wa.maxsig = cfg.maximum_significants;
+        wa.part = e.d_wpart.as<rlnk::WPart>();
+        wa.hcnt = e.d_hcnt.as<unsigned int>();
+        wa.hsum = e.d_hsum.as<double>();
+        wa.cand_w = e.d_wcand.as<double>();
+        wa.cand_i = e.d_wcand_i.as<int>();
+        wa.weight = e.keep ? e.d_weight.as<double>() : nullptr;
+        wa.mask = e.d_mask.as<unsigned char>();
+        wa.want_mask = e.keep ? 1 : 0;
+        wa.best = e.d_segbest.as<rlnk::WSegBest>();
+        wa.ocnt = e.d_ocnt.as<int>();
+        wa.npairs = e.d_npairs.as<int>();
+        wa.njobs = e.d_npairs.as<int>() + e.cap_B;
+        wa.stats = e.d_stats_c.as<rlnk::PassStats>();
+        wa.B = B;
+        const dim3 blk(rlnk::kBlock);
+        hipLaunchKernelGGL(rlnk::k_wseg_exp, dim3(nseg), blk, 0, st, wa);
+        hipLaunchKernelGGL(rlnk::k_wsel_pick, dim3(B), dim3(rlnk::kWBlock), 0, st, wa);
+        hipLaunchKernelGGL(rlnk::k_wseg_gather, dim3(nseg), blk, 0, st, wa);
+        hipLaunchKernelGGL(rlnk::k_wsel_final, dim3(B), blk, 0, st, wa);
+        if (wa.maxsig > 0) hipLaunchKernelGGL(rlnk::k_wsel_maxsig, dim3(B), blk, 0, st, wa);
+        hipLaunchKernelGGL(rlnk::k_wseg_mask, dim3(nseg), blk, 0, st, wa);
+        hipLaunchKernelGGL(rlnk::k_wsel_stats, dim3((B + rlnk::kBlock / 64 - 1) / (rlnk::kBlock / 64)), blk, 0, st, wa);
         RLN_TRY(launch_check("coarse weights"));
     }
     HIP_TRY(hipEventRecord(e.ev[kStJobs], st));
     // ---------------------------------------------------------------- fine pass, planned on the device
     // per-particle counts; everything after runs from device-side counts (FinePlan) without host round trips,
     // as persistent kernels, captured once into a graph and replayed for every chunk
-    // (per-particle pair and job counts were counted by k_wseg_mask / k_wsel_stats)
+    // (per-particle pair and job counts were counted by k_wsel_final / k_wseg_mask / k_wsel_stats)
     e.cp_host.fimg = dX;
     e.cp_host.fimg_nomask = dXn;
     e.cp_host.fctf = dC;
@@ -1512,6 +1515,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         L.job_off = e.d_job_off.as<int>();
         L.pairs = e.d_pairs.as<int>();
         L.plan = e.d_plan.as<rlnk::FinePlan>();
+        L.wpart = e.d_wpart.as<const rlnk::WPart>();
+        L.sig = e.d_wcand_i.as<const int>();
         L.mask = e.d_mask.as<const unsigned char>();
         L.d2off = d_d2off.as<const long long>();
         L.or_cnt = e.d_or_cnt.as<const int>();
@@ -1565,17 +1570,17 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         fa.do_ctf = cfg.do_ctf_correction;
         fa.diff2 = e.d_fdiff2.as<double>();
         rlnk::WeightArgs &wf = L.wf;
-        wf = wa;
-        wf.diff2 = nullptr;
+        wf.or_prior = e.d_or_prior.as<const double>();
+        wf.or_off = e.d_or_off.as<const int>();
+        wf.tr_prior = e.d_tr_prior.as<const double>();
+        wf.NT = NT;
+        wf.adaptive_fraction = cfg.adaptive_fraction;
         wf.diff2d = e.d_fdiff2.as<const double>();
         wf.d2_off = e.d_foff.as<const long long>();
         wf.n_entries = e.d_fine_n.as<const long long>();
         wf.pairs = e.d_pairs.as<const int>();
         wf.pair_off = e.d_pair_off.as<const long long>();
-        wf.fine = 1;
-        wf.maxsig = 0;
         wf.weight = e.d_fweight.as<double>();
-        wf.mask = nullptr;
         wf.stats = e.d_stats_f.as<rlnk::PassStats>();
         wf.plan = e.d_plan.as<const rlnk::FinePlan>();
         L.shell = e.d_shell_acc.as<double>();
@@ -2026,7 +2031,8 @@ extern "C" int rln_estep_destroy(rln_estep *e) {
                            &e->d_jobs, &e->d_job_order, &e->d_chunk_job, &e->d_chunk_first, &e->d_fdiff2, &e->d_fbase, &e->d_fweight,
                            &e->d_fine_n, &e->d_nent, &e->d_foff, &e->d_shell_acc, &e->d_part_acc, &e->d_pdfc_acc, &e->d_pdfd_acc,
                            &e->d_shell_tot, &e->d_plan, &e->d_cp, &e->d_items_s, &e->d_items_w, &e->d_wsegs, &e->d_seg_first,
-                           &e->d_wpart, &e->d_hcnt, &e->d_hsum, &e->d_wcand, &e->d_segbest, &e->d_ocnt};
+                           &e->d_wpart, &e->d_hcnt, &e->d_hsum, &e->d_wcand, &e->d_wcand_i, &e->d_segbest,
+                           &e->d_ocnt};
     rln::drop_fine_graphs(*e);
     for (rln::DevBuf *b : bufs) b->release();
     for (int i = 0; i <= rln::kStCount; ++i)
@@ -2209,11 +2215,11 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
     const bool have_sets = !set_off.empty();
     if (have_sets && (int)set_off.size() != n + 1)
         RLN_FAIL(RLN_ERR_ARG, "orientation lists were set for %d particles, run has %d", (int)set_off.size() - 1, n);
-    // chunk boundaries from a device-memory budget for the coarse intermediates (13 bytes per coarse pose:
-    // diff2, FP64 weight, mask), with per-particle pose counts: the explicit list, the whole grid, or a fraction
+    // chunk boundaries from a device-memory budget for the coarse intermediates (5 bytes per coarse pose: diff2 and
+    // mask; the weights are stored only with the intermediates kept, in one chunk), with per-particle pose counts: the explicit list, the whole grid, or a fraction
     // of it for local searches
     const size_t Pf = e->igf.P;
-    const double fixed = 12.0 * e->Kc + 20.0 * Pf + 64.0 * 1024;
+    const double fixed = 12.0 * e->Kc + 20.0 * Pf + 128.0 * 1024;
     const double budget = 24.0e9;
     std::vector<int> starts;
     {
@@ -2225,7 +2231,7 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
         for (int i = 0; i < n; ++i) {
             long long orients = e->cfg.local_search ? std::max(1, e->n_or / 8) : e->n_or;
             if (have_sets && set_off[i + 1] > set_off[i]) orients = set_off[i + 1] - set_off[i];
-            const double need = 13.0 * (double)e->K * (double)orients * e->NT + fixed;
+            const double need = 5.0 * (double)e->K * (double)orients * e->NT + fixed;
             const int pool = starts.size() == 1 ? first_pool : e->max_pool;
             if (cnt == 0 || (!e->keep && (used + need > budget || cnt >= pool))) {
                 starts.push_back(i);

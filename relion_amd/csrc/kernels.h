@@ -216,15 +216,20 @@ struct WPart {
     int status;
     double sum;             // sum of weights
     double target;          // adaptive_fraction * sum
-    unsigned long long prefix, mask;  // radix selection state
-    double above_sum;       // weights in digit bins above the crossing bin
+    unsigned long long prefix, mask;  // radix selection state: the crossing bin's leading bits
+    double above_sum;       // weights in bins above the crossing bin
     long long above_cnt;
-    int gather;             // 1: crossing bin small enough, elements gathered
+    double dcut;            // entries with diff2 - min above it weigh less than every element of the crossing bin
+    unsigned long long seen; // bits of the largest weight some finished segment has seen (a lower bound on the sum)
+    int state;              // kSel*
     int ncand;
     double thr;             // significance threshold
     long long nr_sign;
     long long n_above;      // entries >= thr
 };
+// Selection state of a particle: crossing bin not fine enough yet; every entry from the crossing bin up fits the
+// candidate list; only the crossing bin does; no weights (zero or NaN sum).
+constexpr int kSelRefine = 0, kSelAll = 1, kSelBin = 2, kSelNone = 3;
 
 // Columns of the x contraction: 16 lanes hold one signed x shift each, tx = +(n + 1) on lane n < 8 (matrix column
 // cos) and -(n - 7) on lane n >= 8 (column sin), counted from kColShift * tile; where a tile
@@ -504,23 +509,6 @@ __device__ __forceinline__ double block_sum_d(double v, double *red) {
     return r;
 }
 
-__device__ __forceinline__ float block_min_f(float v, float *red) {
-    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[w] = v;
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        float t = (threadIdx.x < (blockDim.x >> 6)) ? red[threadIdx.x] : 3.0e38f;
-        for (int o = 32; o > 0; o >>= 1) t = fminf(t, __shfl_xor(t, o));
-        if (threadIdx.x == 0) red[0] = t;
-    }
-    __syncthreads();
-    const float r = red[0];
-    __syncthreads();
-    return r;
-}
-
 __device__ __forceinline__ double block_min_d(double v, double *red) {
     for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -534,6 +522,33 @@ __device__ __forceinline__ double block_min_d(double v, double *red) {
     }
     __syncthreads();
     const double r = red[0];
+    __syncthreads();
+    return r;
+}
+
+__device__ __forceinline__ int block_exclusive_scan_i(int v, int *tmp, int &total) {
+    // wave-level inclusive scan
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    __syncthreads();
+    if (lane == 63) tmp[w] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int acc = 0;
+        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) {
+            const int t = tmp[i];
+            tmp[i] = acc;
+            acc += t;
+        }
+        tmp[blockDim.x >> 6] = acc;
+    }
+    __syncthreads();
+    const int r = x - v + tmp[w];
+    total = tmp[blockDim.x >> 6];
     __syncthreads();
     return r;
 }
@@ -582,44 +597,33 @@ struct ChunkPtrs {
     int pad_;
 };
 
-// Mode of k_weights: coarse entries are e = o*NT + t; fine entries are e = s*32 + r*4 + u where pair s
-// holds the coarse index (o*NT + t) in pairs[].
+// Arguments of k_weights: entries of the fine pass are e = s*32 + r*4 + u where pair s holds the coarse index
+// (o*NT + t) in pairs[].
 struct WeightArgs {
-    const float *diff2;          // coarse mode: per particle at d2_off[b]; entries < 0 were not evaluated
-    const double *diff2d;        // fine mode: per particle at d2_off[b], every entry evaluated
+    const double *diff2d;        // per particle at d2_off[b], every entry evaluated
     const long long *d2_off;
     const long long *n_entries;  // per particle
     const double *or_prior;      // normalised pdf_orientation per orientation entry (or_off based)
     const int *or_off;
-    const int *oc_off;          // per-particle offsets of per-orientation state (ocnt)
     const double *tr_prior;      // normalised pdf_offset [b][NT]
-    const int *pairs;            // fine mode: coarse index per pair, at pair_off[b]
+    const int *pairs;            // coarse index per pair, at pair_off[b]
     const long long *pair_off;
     int NT;
-    int fine;                    // 0 coarse, 1 fine
     double adaptive_fraction;
-    long long maxsig;            // <= 0: none (coarse pass only)
-    double *weight;              // out, same indexing as diff2
-    unsigned char *mask;         // out (coarse mode), weight >= threshold
+    double *weight;              // out, same indexing as diff2d
     PassStats *stats;            // out [b]
-    const FinePlan *plan;        // fine mode: chunk header (overflow: skip; blocks >= plan->B: idle); else null
+    const FinePlan *plan;        // chunk header (overflow: skip; blocks >= plan->B: idle)
 };
 
 __device__ __forceinline__ double entry_prior(const WeightArgs &a, int b, long long e) {
-    long long c;
-    if (a.fine) {
-        c = a.pairs[a.pair_off[b] + (e >> 5)];
-    } else {
-        c = e;
-    }
-    const long long o = c / a.NT, t = c - o * a.NT;
+    const int c = a.pairs[a.pair_off[b] + (e >> 5)];
+    const int o = c / a.NT, t = c - o * a.NT;
     return a.or_prior[a.or_off[b] + o] * a.tr_prior[(size_t)b * a.NT + t];
 }
 
 // Key that orders entries like storeWeightedSums visits them (class, direction, psi, iover_rot, itrans,
 // iover_trans; src/ml_optimiser.cpp:8329-8470), used to break ties of the max weight as the reference does.
 __device__ __forceinline__ long long wsum_order_key(const WeightArgs &a, int b, long long e) {
-    if (!a.fine) return e;
     const long long s = e >> 5;
     const int r = (int)((e >> 2) & 7), u = (int)(e & 3);
     const long long c = a.pairs[a.pair_off[b] + s];
@@ -628,13 +632,11 @@ __device__ __forceinline__ long long wsum_order_key(const WeightArgs &a, int b, 
 }
 
 // One 1024-thread block per particle: min diff2, weights in FP64, their sum, the significance threshold by
-// radix selection over the weights' bit patterns (positive doubles order like their uint64 patterns), the
-// coarse significance mask and the max weight. The threshold is the weight at which the descending
-// cumulative sum first exceeds adaptive_fraction * sum (src/ml_optimiser.cpp:8145-8168); maxsig caps the
-// count as in :8147-8157.
+// radix selection over the weights' bit patterns (positive doubles order like their uint64 patterns) and the max
+// weight. The threshold is the weight at which the descending
+// cumulative sum first exceeds adaptive_fraction * sum (src/ml_optimiser.cpp:8145-8168).
 __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
     __shared__ double red_d[16];
-    __shared__ float red_f[16];
     __shared__ long long red_l[16];
     __shared__ unsigned int hcnt[256];
     __shared__ double hsum[256];
@@ -647,36 +649,19 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
     __shared__ long long s_above_cnt;
     __shared__ int s_done;
     const int b = blockIdx.x;
-    if (a.plan && (a.plan->overflow || b >= a.plan->B)) return;
+    if (a.plan->overflow || b >= a.plan->B) return;
     const long long n = a.n_entries[b];
     double *w = a.weight + a.d2_off[b];
     const int tid = threadIdx.x;
 
-    // fine entries are FP64 and all evaluated; coarse entries FP32, < 0 where not evaluated
-    const float *d2 = a.fine ? nullptr : a.diff2 + a.d2_off[b];
-    const double *d2d = a.fine ? a.diff2d + a.d2_off[b] : nullptr;
-    double mind;
-    if (a.fine) {
-        double mnd = 1.0e300;
-        for (long long e = tid; e < n; e += kWBlock) mnd = fmin(mnd, d2d[e]);
-        mind = block_min_d(mnd, red_d);
-    } else {
-        float mn = 3.0e38f;
-        for (long long e = tid; e < n; e += kWBlock) {
-            const float v = d2[e];
-            if (v >= 0.f) mn = fminf(mn, v);
-        }
-        mind = (double)block_min_f(mn, red_f);
-    }
+    const double *d2d = a.diff2d + a.d2_off[b];
+    double mind = 1.0e300;
+    for (long long e = tid; e < n; e += kWBlock) mind = fmin(mind, d2d[e]);
+    mind = block_min_d(mind, red_d);
     double sum = 0.;
     for (long long e = tid; e < n; e += kWBlock) {
-        const double v = a.fine ? d2d[e] : (double)d2[e];
-        double wt = 0.;
-        if (a.fine || v >= 0.) {
-            const double diff = v - mind;
-            wt = entry_prior(a, b, e);
-            wt = (diff > 700.) ? 0. : wt * exp(-diff);
-        }
+        const double diff = d2d[e] - mind;
+        const double wt = (diff > 700.) ? 0. : entry_prior(a, b, e) * exp(-diff);
         w[e] = wt;
         sum += wt;
     }
@@ -766,7 +751,6 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
                 }
                 if (tid == 0) {
                     long long nsig = rank + 1;
-                    if (crossed && a.maxsig > 0 && !a.fine && nsig > a.maxsig) nsig = a.maxsig;
                     s_cand_ok = crossed;
                     s_cand_nsig = nsig;
                     s_cand_thr = crossed ? s_cand[n2 - nsig] : 0.;
@@ -845,54 +829,14 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
         if (m < 1) m = 1;
         nr_sign = s_above_cnt + m;
     }
-    if (a.maxsig > 0 && !a.fine && nr_sign > a.maxsig) {
-        // rank selection of the maxsig-th largest weight
-        if (tid == 0) {
-            s_prefix = 0ULL;
-            s_mask = 0ULL;
-            s_above_cnt = 0;
-        }
-        __syncthreads();
-        for (int shift = 56; shift >= 0; shift -= 8) {
-            for (int i = tid; i < 256; i += kWBlock) hcnt[i] = 0;
-            __syncthreads();
-            const unsigned long long pre = s_prefix, msk = s_mask;
-            for (long long e = tid; e < n; e += kWBlock) {
-                const double v = w[e];
-                if (!(v > 0.)) continue;
-                const unsigned long long key = (unsigned long long)__double_as_longlong(v);
-                if ((key & msk) != pre) continue;
-                atomicAdd(&hcnt[(int)((key >> shift) & 255ULL)], 1u);
-            }
-            __syncthreads();
-            if (tid == 0) {
-                long long cnt = s_above_cnt;
-                int bin = 0;
-                for (int k = 255; k >= 0; --k) {
-                    if (cnt + (long long)hcnt[k] >= a.maxsig) {
-                        bin = k;
-                        break;
-                    }
-                    cnt += hcnt[k];
-                }
-                s_above_cnt = cnt;
-                s_prefix |= ((unsigned long long)bin << shift);
-                s_mask |= (255ULL << shift);
-            }
-            __syncthreads();
-        }
-        thr = __longlong_as_double((long long)s_prefix);
-        nr_sign = a.maxsig;
-    }
     }  // radix selection
-    // mask, count above threshold, max weight with the reference's loop-order tie break
+    // count above threshold, max weight with the reference's loop-order tie break
     long long above = 0;
     double bw = -1.;
     long long bkey = 0x7fffffffffffffffLL, bidx = -1;
     for (long long e = tid; e < n; e += kWBlock) {
         const double v = w[e];
         const bool sig = v >= thr && v > 0.;
-        if (!a.fine) a.mask[a.d2_off[b] + e] = sig ? 1 : 0;
         above += sig ? 1 : 0;
         if (v > 0.) {
             const long long key = wsum_order_key(a, b, e);
@@ -935,21 +879,41 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
         st.max_weight = bw;
         st.best_key = bkey;
         st.best_index = bidx;
-        if (!a.fine && nr_sign == 0) st.status = -5;
         a.stats[b] = st;
     }
 }
 
 // --------------------------------------------------------------------------------------------------
-// Coarse weights over segments: the same results as k_weights (min, FP64 weights, sum, significance
-// threshold, mask, max weight), with every pass over the entries split into blocks of kSegEntries, so that a
-// particle with millions of coarse poses (an exhaustive search) is spread over the whole GPU. The threshold is
-// found by a multi-block radix selection over the weights' bit patterns (8-bit digits from the top; positive
-// doubles order like their uint64 patterns) until the crossing digit bin holds at most kGather elements, which
-// are then sorted in LDS and scanned exactly.
+// Coarse weights over segments: min, FP64 weights, their sum, the significance threshold and the significant poses,
+// with every pass over the entries split into blocks of a segment, so that a particle with millions of coarse poses
+// (an exhaustive search) is spread over the whole GPU. The weights are not stored (unless they are asked for): every
+// pass forms those it needs from the FP32 diff2, 4 bytes a pose, the same FP64 expression each time.
+//   k_wseg_exp     weights' sum and a histogram of their binary exponents
+//   k_wsel_pick    the bin where the descending cumulative sum crosses the target, and its further mantissa digits while
+//                  it holds more than the candidate list (one block per particle: the poses of such a flat posterior
+//                  cost far more in the fine pass)
+//   k_wseg_gather  candidates: every entry from the crossing bin up when they fit the list (kSelAll), else the bin's
+//                  (kSelBin)
+//   k_wsel_final   exact threshold from the sorted candidates; for kSelAll also the significant poses in order, which
+//                  are then all the fine pass needs
+//   k_wseg_mask, k_wsel_stats  the mask, per-orientation counts and maximum over all entries of kSelBin particles
+// Bound by the two reads of diff2 (4 bytes a pose each) and, where many poses are close, by the exponentials. Measured:
+// 2.5e9 poses 20.0 -> 5.5 ms (20 GB: 3.7 TB/s), 4.2e8 poses 3.6 -> 1.1 ms, 2,048 particles of 35,000 poses 2.2 -> 0.66
+// ms, against stored FP64 weights with 8-bit digits in a launch each. Several diff2 values a thread in flight: 1 8.8 ms,
+// 4 5.5, 8 6.5. Finding the bin in the last block of a particle instead of a launch of its own needs device-wide fences,
+// which made the first pass wait on the caches for 16 ms.
 // --------------------------------------------------------------------------------------------------
-constexpr long long kSegEntries = 32768;  // entries per segment block
-constexpr int kGather = 4096;             // crossing-bin elements sorted exactly
+constexpr int kExpBins = 1088;    // binary exponents of the weights (a weight is below 2^64: the prior's mean is 1)
+constexpr int kGather = 4096;     // candidates sorted exactly
+constexpr int kSegBatch = 4;      // diff2 values a thread has in flight
+constexpr int kSegMin = 4096, kSegMax = 32768;  // entries per segment (choose_segment)
+
+// Entries per segment of a chunk of `total` entries: long enough that a block's histogram (cleared and written once a
+// segment) is a small part of its work, short enough that small chunks still fill the GPU.
+inline long long choose_segment(long long total) {
+    const long long want = total / 4096 / kBlock * kBlock;
+    return want < kSegMin ? kSegMin : want > kSegMax ? kSegMax : want;
+}
 
 struct WSeg {
     int b;             // particle
@@ -958,11 +922,73 @@ struct WSeg {
     long long end;
 };
 
-
 struct WSegBest {
     double w;
     long long key, idx;
 };
+
+struct CoarseWeightArgs {
+    const WSeg *segs;
+    const int *seg_first;        // [B + 1] first segment of each particle
+    const float *diff2;          // per particle at d2_off[b]; entries < 0 were not evaluated
+    const long long *d2_off;
+    const long long *n_entries;  // per particle
+    const double *or_prior;      // normalised pdf_orientation per orientation entry (or_off based)
+    const int *or_off;
+    const int *or_cnt;
+    const int *oc_off;           // per-particle offsets of per-orientation state (ocnt)
+    const double *tr_prior;      // normalised pdf_offset [b][NT]
+    int NT;
+    double prior_max;            // no entry's prior exceeds it
+    double adaptive_fraction;
+    long long maxsig;            // <= 0: none
+    WPart *part;
+    unsigned int *hcnt;          // [b][kExpBins], zero before k_wseg_exp
+    double *hsum;
+    double *cand_w;              // [b][kGather] candidate weights
+    int *cand_i;                 // [b][kGather] their entries; then the significant entries of kSelAll in order
+    double *weight;              // out, same indexing as diff2, or null
+    unsigned char *mask;         // out, weight >= threshold (kSelBin, or every particle with want_mask)
+    int want_mask;
+    WSegBest *best;              // per segment (kSelBin)
+    int *ocnt;                   // significant translations per orientation entry (kSelBin)
+    int *npairs, *njobs;         // out [b] significant poses, orientations with any
+    PassStats *stats;            // out [b]
+    int B;
+};
+
+// Entries of one segment as a block of S threads visits them: e, and its orientation and translation without a
+// division per entry.
+template <int S>
+struct SegCursor {
+    long long e;
+    int o, t, step_o, step_t, NT;
+    __device__ __forceinline__ SegCursor(long long begin, int nt) {
+        NT = nt;
+        step_o = S / nt;
+        step_t = S % nt;
+        e = begin + threadIdx.x;
+        o = (int)((unsigned)e / (unsigned)nt);
+        t = (int)e - o * nt;
+    }
+    __device__ __forceinline__ void next() {
+        e += S;
+        o += step_o;
+        t += step_t;
+        if (t >= NT) {
+            t -= NT;
+            ++o;
+        }
+    }
+};
+
+// Weight of a coarse pose: 0 where it was not evaluated or lies more than 700 above the minimum.
+__device__ __forceinline__ double coarse_weight(float v, double mind, const double *orp, const double *trp, int o,
+                                                int t) {
+    if (!(v >= 0.f)) return 0.;
+    const double diff = (double)v - mind;
+    return (diff > 700.) ? 0. : orp[o] * trp[t] * exp(-diff);
+}
 
 __global__ void __launch_bounds__(kBlock) k_wpart_init(WPart *__restrict__ part, int B) {
     const int b = blockIdx.x * kBlock + threadIdx.x;
@@ -972,37 +998,52 @@ __global__ void __launch_bounds__(kBlock) k_wpart_init(WPart *__restrict__ part,
     part[b] = p;
 }
 
-// Weights of one segment, their sum, and the first radix pass of the selection (the top byte of every positive
-// weight: the pass before any prefix is fixed), accumulated here instead of in a separate read of the weights.
-__global__ void __launch_bounds__(kBlock) k_wseg_exp(WeightArgs a, const WSeg *__restrict__ segs,
-                                                     WPart *__restrict__ part, unsigned int *__restrict__ hcnt,
-                                                     double *__restrict__ hsum) {
+// Weights of one segment, their sum, and the histogram of their exponents. Two bounds from the largest weight seen so
+// far, s (at most the sum), spare most entries the LDS atomics and the exponential:
+//   - the weights below x = (1 - f) sum / n together hold less than the (1 - f) tail, so the threshold is at least x and
+//     its bin's lower edge at least x / 2: weights below (1 - f) s / (4 n) are left out of the histogram;
+//   - weights below 2^-64 s / n, all together, do not change the FP64 sum: they are not formed.
+__global__ void __launch_bounds__(kBlock) k_wseg_exp(CoarseWeightArgs a) {
     __shared__ double red[kBlock / 64];
-    __shared__ unsigned int c[256];
-    __shared__ double sm[256];
-    c[threadIdx.x] = 0;
-    sm[threadIdx.x] = 0.;
-    const WSeg sg = segs[blockIdx.x];
+    __shared__ unsigned int c[kExpBins];
+    __shared__ double sm[kExpBins];
+    __shared__ unsigned long long s_seen;
+    for (int k = threadIdx.x; k < kExpBins; k += kBlock) {
+        c[k] = 0;
+        sm[k] = 0.;
+    }
+    const WSeg sg = a.segs[blockIdx.x];
     const int b = sg.b;
     const float *d2 = a.diff2 + a.d2_off[b];
-    double *w = a.weight + a.d2_off[b];
-    const double mind = (double)__uint_as_float(part[b].mn_bits);
+    const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
+    const double mind = (double)__uint_as_float(a.part[b].mn_bits);
+    if (threadIdx.x == 0) s_seen = atomicAdd(&a.part[b].seen, 0ULL);
     __syncthreads();
-    double sum = 0.;
-    for (long long e = sg.begin + threadIdx.x; e < sg.end; e += kBlock) {
-        const float v = d2[e];
-        double wt = 0.;
-        if (v >= 0.f) {
-            const double diff = (double)v - mind;
-            wt = entry_prior(a, b, e);
-            wt = (diff > 700.) ? 0. : wt * exp(-diff);
+    const double n = (double)a.n_entries[b], tail = (1. - a.adaptive_fraction) / (4. * n);
+    double sum = 0., seen = 0., hist_min = 0., cut = 1e300;
+    for (SegCursor<kBlock> k(sg.begin, a.NT); k.e < sg.end;) {
+        float v[kSegBatch];
+#pragma unroll
+        for (int u = 0; u < kSegBatch; ++u) v[u] = k.e + u * kBlock < sg.end ? d2[k.e + u * kBlock] : -1.f;
+        const double s = __longlong_as_double(
+            (long long)__hip_atomic_load(&s_seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        if (s > seen) {  // rare: the bounds follow the largest weight
+            seen = s;
+            hist_min = tail * s;
+            if (!a.weight) cut = log(a.prior_max / s * n) + 44.4;  // 2^-64 = exp(-44.36)
         }
-        w[e] = wt;
-        sum += wt;
-        if (wt > 0.) {
-            const int bin = (int)((unsigned long long)__double_as_longlong(wt) >> 56);
+#pragma unroll
+        for (int u = 0; u < kSegBatch; ++u, k.next()) {
+            if (k.e >= sg.end || (double)v[u] - mind > cut) continue;
+            const double wt = coarse_weight(v[u], mind, orp, trp, k.o, k.t);
+            if (a.weight) a.weight[a.d2_off[b] + k.e] = wt;
+            sum += wt;
+            if (!(wt > 0.) || wt < hist_min) continue;
+            const unsigned long long bits = (unsigned long long)__double_as_longlong(wt);
+            const int bin = min((int)(bits >> 52), kExpBins - 1);
             atomicAdd(&c[bin], 1u);
             atomicAdd(&sm[bin], wt);
+            if (wt > seen) atomicMax(&s_seen, bits);
         }
     }
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
@@ -1010,153 +1051,219 @@ __global__ void __launch_bounds__(kBlock) k_wseg_exp(WeightArgs a, const WSeg *_
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int i = 1; i < kBlock / 64; ++i) sum += red[i];
-        atomicAdd(&part[b].sum, sum);
+        atomicAdd(&a.part[b].sum, sum);
+        if (s_seen) atomicMax(&a.part[b].seen, s_seen);
     }
-    if (c[threadIdx.x]) {
-        atomicAdd(&hcnt[(size_t)b * 256 + threadIdx.x], c[threadIdx.x]);
-        atomicAdd(&hsum[(size_t)b * 256 + threadIdx.x], sm[threadIdx.x]);
+    for (int k = threadIdx.x; k < kExpBins; k += kBlock)
+        if (c[k]) {
+            atomicAdd(&a.hcnt[(size_t)b * kExpBins + k], c[k]);
+            atomicAdd(&a.hsum[(size_t)b * kExpBins + k], sm[k]);
+        }
+}
+
+// The crossing bin of one particle among nb histogram bins (digit at `shift`) by wave 0: the bin where the descending
+// cumulative sum from above_sum exceeds the target, or (rounding: the total may not exceed it) the smallest bin present.
+__device__ __forceinline__ void pick_bin(const CoarseWeightArgs &a, WPart &p, const unsigned int *c, const double *sm,
+                                         int nb, int shift, unsigned long long digit_mask) {
+    const int lane = threadIdx.x;
+    double acc = p.above_sum, low_sum = 0.;
+    long long cnt = p.above_cnt, low_cnt = 0;
+    int low = 0;
+    unsigned int in_low = 0;
+    for (int k0 = nb - 1; k0 >= 0; k0 -= 64) {
+        const int k = k0 - lane;
+        const unsigned int ck = k >= 0 ? c[k] : 0u;
+        const unsigned long long present = __ballot(ck > 0);
+        if (!present) continue;
+        const double s = ck > 0 ? sm[k] : 0.;
+        double xs = s;  // inclusive sums from the top
+        long long xc = ck;
+        for (int o = 1; o < 64; o <<= 1) {
+            const double ys = __shfl_up(xs, o);
+            const long long yc = __shfl_up(xc, o);
+            if (lane >= o) {
+                xs += ys;
+                xc += yc;
+            }
+        }
+        const unsigned long long hit = __ballot(ck > 0 && acc + xs > p.target);
+        const int q = hit ? __ffsll((long long)hit) - 1 : 63 - __clzll((long long)present);
+        low = k0 - q;
+        low_sum = acc + __shfl(xs - s, q);
+        low_cnt = cnt + __shfl(xc - (long long)ck, q);
+        in_low = __shfl(ck, q);
+        if (hit) break;
+        acc += __shfl(xs, 63);
+        cnt += __shfl(xc, 63);
+    }
+    p.above_sum = low_sum;
+    p.above_cnt = low_cnt;
+    p.prefix |= (unsigned long long)low << shift;
+    p.mask |= digit_mask;
+    // the smallest weight with this prefix; below it no entry is a candidate
+    const double lo = __longlong_as_double((long long)p.prefix);
+    p.dcut = lo > 0. ? log(a.prior_max / lo) + 1e-6 : 1e300;
+    p.state = low_cnt + in_low <= kGather ? kSelAll : (in_low <= kGather || shift == 0) ? kSelBin : kSelRefine;
+}
+
+// One block per particle: the crossing exponent bin, then the crossing bins of further digits of its mantissa while the
+// bin holds more than kGather entries.
+__global__ void __launch_bounds__(kWBlock) k_wsel_pick(CoarseWeightArgs a) {
+    __shared__ unsigned int c[kExpBins];
+    __shared__ double sm[kExpBins];
+    __shared__ WPart s_p;
+    const int b = blockIdx.x, tid = threadIdx.x;
+    const unsigned int *hc = a.hcnt + (size_t)b * kExpBins;
+    const double *hs = a.hsum + (size_t)b * kExpBins;
+    for (int k = tid; k < kExpBins; k += kWBlock) {
+        c[k] = hc[k];
+        sm[k] = hs[k];
+    }
+    if (tid == 0) {
+        s_p = a.part[b];
+        s_p.target = a.adaptive_fraction * s_p.sum;
+        s_p.state = kSelRefine;
+        if (!(s_p.sum > 0.)) {
+            s_p.status = -6;  // zero or NaN sum (src/ml_optimiser.cpp:8054-8104)
+            s_p.state = kSelNone;
+        }
+    }
+    __syncthreads();
+    if (s_p.state != kSelNone) {
+        if (tid < 64) {
+            WPart p = s_p;
+            pick_bin(a, p, c, sm, kExpBins, 52, 0xfffULL << 52);
+            if (tid == 0) s_p = p;
+        }
+        const float *d2 = a.diff2 + a.d2_off[b];
+        const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
+        const double mind = (double)__uint_as_float(a.part[b].mn_bits);
+        const long long n = a.n_entries[b];
+        int shift = 52;
+        for (int digit = 0; digit < 6; ++digit) {  // 9, 9, 9, 9, 8, 8 bits of the mantissa
+            __syncthreads();
+            if (s_p.state != kSelRefine) break;
+            const int bits = digit < 4 ? 9 : 8, nb = 1 << bits;
+            shift -= bits;
+            for (int k = tid; k < nb; k += kWBlock) {
+                c[k] = 0;
+                sm[k] = 0.;
+            }
+            const unsigned long long prefix = s_p.prefix, mask = s_p.mask;
+            const double dcut = s_p.dcut;
+            __syncthreads();
+            for (SegCursor<kWBlock> k(0, a.NT); k.e < n; k.next()) {
+                const float v = d2[k.e];
+                if (!((double)v - mind <= dcut)) continue;
+                const double wt = coarse_weight(v, mind, orp, trp, k.o, k.t);
+                const unsigned long long key = (unsigned long long)__double_as_longlong(wt);
+                if (!(wt > 0.) || (key & mask) != prefix) continue;
+                const int bin = (int)((key >> shift) & (unsigned long long)(nb - 1));
+                atomicAdd(&c[bin], 1u);
+                atomicAdd(&sm[bin], wt);
+            }
+            __syncthreads();
+            if (tid < 64) {
+                WPart p = s_p;
+                pick_bin(a, p, c, sm, nb, shift, (unsigned long long)(nb - 1) << shift);
+                if (tid == 0) s_p = p;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) a.part[b] = s_p;
+}
+
+// Candidates into the particle's list: all entries from the crossing bin up, or the crossing bin's weights.
+__global__ void __launch_bounds__(kBlock) k_wseg_gather(CoarseWeightArgs a) {
+    const WSeg sg = a.segs[blockIdx.x];
+    const int b = sg.b;
+    const WPart p = a.part[b];
+    if (p.state == kSelNone) return;
+    const float *d2 = a.diff2 + a.d2_off[b];
+    const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
+    const double mind = (double)__uint_as_float(p.mn_bits);
+    for (SegCursor<kBlock> k(sg.begin, a.NT); k.e < sg.end;) {
+        float v[kSegBatch];
+#pragma unroll
+        for (int u = 0; u < kSegBatch; ++u) v[u] = k.e + u * kBlock < sg.end ? d2[k.e + u * kBlock] : -1.f;
+#pragma unroll
+        for (int u = 0; u < kSegBatch; ++u, k.next()) {
+            if (!(v[u] >= 0.f) || !((double)v[u] - mind <= p.dcut)) continue;
+            const double wt = coarse_weight(v[u], mind, orp, trp, k.o, k.t);
+            if (!(wt > 0.)) continue;
+            const unsigned long long key = (unsigned long long)__double_as_longlong(wt);
+            if (p.state == kSelAll ? key < p.prefix : (key & p.mask) != p.prefix) continue;
+            const int slot = atomicAdd(&a.part[b].ncand, 1);
+            if (slot < kGather) {
+                a.cand_w[(size_t)b * kGather + slot] = wt;
+                a.cand_i[(size_t)b * kGather + slot] = (int)k.e;
+            }
+        }
     }
 }
 
-// per particle: status and selection start
-__global__ void __launch_bounds__(kBlock) k_wsel_start(WeightArgs a, WPart *__restrict__ part, int B) {
-    const int b = blockIdx.x * kBlock + threadIdx.x;
-    if (b >= B) return;
-    WPart &p = part[b];
-    if (!(p.sum > 0.)) {
-        p.status = -6;  // zero or NaN sum (src/ml_optimiser.cpp:8054-8104)
-        p.gather = 2;   // no selection
+// per particle (one block): exact threshold from the sorted candidates, maxsig cap by rank
+// (src/ml_optimiser.cpp:8145-8168). kSelAll: also the significant entries in ascending order, their counts and the
+// particle's statistics; kSelBin: its per-orientation counts cleared for k_wseg_mask.
+__global__ void __launch_bounds__(kBlock) k_wsel_final(CoarseWeightArgs a) {
+    __shared__ double s_w[kGather];
+    __shared__ int s_i[kGather];
+    __shared__ int s_rank, s_crossed, s_above;
+    __shared__ int tmp[8];
+    const int b = blockIdx.x, tid = threadIdx.x;
+    WPart &p = a.part[b];
+    PassStats st{};
+    st.min_diff2 = (double)__uint_as_float(p.mn_bits);
+    st.sum_weight = p.sum;
+    st.best_key = st.best_index = -1;
+    const int state = p.state;
+    if (state == kSelNone) {
+        if (tid == 0) {
+            st.status = p.status;
+            a.stats[b] = st;
+            a.npairs[b] = a.njobs[b] = 0;
+        }
         return;
     }
-    p.target = a.adaptive_fraction * p.sum;
-}
-
-// one radix pass: per-particle digit histograms (count, sum) of the weights that match the prefix
-__global__ void __launch_bounds__(kBlock) k_wseg_hist(WeightArgs a, const WSeg *__restrict__ segs,
-                                                      const WPart *__restrict__ part, int shift,
-                                                      unsigned int *__restrict__ hcnt, double *__restrict__ hsum) {
-    __shared__ unsigned int c[256];
-    __shared__ double sm[256];
-    const WSeg sg = segs[blockIdx.x];
-    const WPart p = part[sg.b];
-    if (p.gather) return;
-    c[threadIdx.x] = 0;
-    sm[threadIdx.x] = 0.;
-    __syncthreads();
-    const double *w = a.weight + a.d2_off[sg.b];
-    for (long long e = sg.begin + threadIdx.x; e < sg.end; e += kBlock) {
-        const double v = w[e];
-        if (!(v > 0.)) continue;
-        const unsigned long long key = (unsigned long long)__double_as_longlong(v);
-        if ((key & p.mask) != p.prefix) continue;
-        const int bin = (int)((key >> shift) & 255ULL);
-        atomicAdd(&c[bin], 1u);
-        atomicAdd(&sm[bin], v);
-    }
-    __syncthreads();
-    if (c[threadIdx.x]) {
-        atomicAdd(&hcnt[(size_t)sg.b * 256 + threadIdx.x], c[threadIdx.x]);
-        atomicAdd(&hsum[(size_t)sg.b * 256 + threadIdx.x], sm[threadIdx.x]);
-    }
-}
-
-// per particle: the digit bin where the descending cumulative sum crosses the target; histograms cleared
-__global__ void __launch_bounds__(kBlock) k_wsel_pick(WPart *__restrict__ part, int B, int shift,
-                                                      unsigned int *__restrict__ hcnt, double *__restrict__ hsum) {
-    const int b = blockIdx.x * kBlock + threadIdx.x;
-    if (b >= B) return;
-    WPart &p = part[b];
-    unsigned int *hc = hcnt + (size_t)b * 256;
-    double *hs = hsum + (size_t)b * 256;
-    if (!p.gather) {
-        double acc = p.above_sum;
-        long long cnt = p.above_cnt;
-        int bin = -1;
-        for (int k = 255; k >= 0; --k) {
-            if (hc[k] == 0) continue;
-            if (acc + hs[k] > p.target) {
-                bin = k;
-                break;
-            }
-            acc += hs[k];
-            cnt += hc[k];
-        }
-        if (bin < 0) {  // rounding: the total never exceeds the target; take the smallest present bin
-            for (int k = 0; k < 256; ++k)
-                if (hc[k]) {
-                    bin = k;
-                    break;
-                }
-            acc -= hs[bin];
-            cnt -= hc[bin];
-        }
-        p.above_sum = acc;
-        p.above_cnt = cnt;
-        p.prefix |= ((unsigned long long)bin << shift);
-        p.mask |= (255ULL << shift);
-        if (hc[bin] <= (unsigned)kGather || shift == 0) p.gather = 1;
-    }
-    for (int k = 0; k < 256; ++k) {
-        hc[k] = 0;
-        hs[k] = 0.;
-    }
-}
-
-// elements of the crossing bin (weights matching the prefix) into the per-particle candidate buffer
-__global__ void __launch_bounds__(kBlock) k_wseg_gather(WeightArgs a, const WSeg *__restrict__ segs,
-                                                        WPart *__restrict__ part, double *__restrict__ cand) {
-    const WSeg sg = segs[blockIdx.x];
-    const WPart p = part[sg.b];
-    if (p.gather != 1) return;
-    const double *w = a.weight + a.d2_off[sg.b];
-    for (long long e = sg.begin + threadIdx.x; e < sg.end; e += kBlock) {
-        const double v = w[e];
-        if (!(v > 0.)) continue;
-        const unsigned long long key = (unsigned long long)__double_as_longlong(v);
-        if ((key & p.mask) != p.prefix) continue;
-        const int slot = atomicAdd(&part[sg.b].ncand, 1);
-        if (slot < kGather) cand[(size_t)sg.b * kGather + slot] = v;
-    }
-}
-
-// per particle (one block): exact threshold from the sorted crossing-bin elements, maxsig cap by rank
-__global__ void __launch_bounds__(kWBlock) k_wsel_final(WeightArgs a, WPart *__restrict__ part,
-                                                        const double *__restrict__ cand) {
-    __shared__ double s_c[kGather];
-    __shared__ long long s_rank;
-    __shared__ int s_ok;
-    const int b = blockIdx.x, tid = threadIdx.x;
-    WPart &p = part[b];
-    if (p.gather == 2) return;
-    const int nc = min(p.ncand, kGather);
-    // sort size: the next power of two holding the candidates (uniform over the block), padded with -1 below
-    // every weight
+    const bool all = state == kSelAll;
+    const int ncand = p.ncand, nc = min(ncand, kGather);
+    const double above_sum = all ? 0. : p.above_sum;
+    if (tid == 0) s_above = 0;
+    // sort size: the next power of two holding the candidates (uniform over the block), padded with -1 below every
+    // weight; descending weight, ascending entry among equal weights
     int n2 = 2;
     while (n2 < nc) n2 <<= 1;
-    for (int i = tid; i < n2; i += kWBlock) s_c[i] = (i < nc) ? cand[(size_t)b * kGather + i] : -1.;
+    for (int i = tid; i < n2; i += kBlock) {
+        s_w[i] = (i < nc) ? a.cand_w[(size_t)b * kGather + i] : -1.;
+        s_i[i] = (i < nc) ? a.cand_i[(size_t)b * kGather + i] : 0x7fffffff;
+    }
     __syncthreads();
-    for (int ks = 2; ks <= n2; ks <<= 1)  // bitonic sort, ascending
+    for (int ks = 2; ks <= n2; ks <<= 1)
         for (int j = ks >> 1; j > 0; j >>= 1) {
-            for (int i = tid; i < n2; i += kWBlock) {
+            for (int i = tid; i < n2; i += kBlock) {
                 const int l = i ^ j;
                 if (l > i) {
-                    const double x = s_c[i], y = s_c[l];
-                    if (((i & ks) == 0) ? (x > y) : (x < y)) {
-                        s_c[i] = y;
-                        s_c[l] = x;
+                    const double x = s_w[i], y = s_w[l];
+                    const int xi = s_i[i], yi = s_i[l];
+                    const bool after = x < y || (x == y && xi > yi);  // x belongs after y
+                    if (((i & ks) == 0) == after) {
+                        s_w[i] = y;
+                        s_w[l] = x;
+                        s_i[i] = yi;
+                        s_i[l] = xi;
                     }
                 }
             }
             __syncthreads();
         }
-    // descending cumulative sum from above_sum, 64 elements per step (wave 0)
+    // descending cumulative sum, 64 elements per step (wave 0)
     if (tid < 64) {
-        double base = p.above_sum;
-        int crossed = 0;
-        long long rank = nc - 1;
+        double base = above_sum;
+        int crossed = 0, rank = nc - 1;
         for (int r0 = 0; r0 < nc; r0 += 64) {
             const int r = r0 + tid;
-            double x = (r < nc) ? s_c[n2 - 1 - r] : 0.;
+            double x = (r < nc) ? s_w[r] : 0.;
             for (int o = 1; o < 64; o <<= 1) {
                 const double y = __shfl_up(x, o);
                 if (tid >= o) x += y;
@@ -1172,18 +1279,18 @@ __global__ void __launch_bounds__(kWBlock) k_wsel_final(WeightArgs a, WPart *__r
         }
         if (tid == 0) {
             s_rank = rank;
-            s_ok = crossed;
+            s_crossed = crossed;
         }
     }
     __syncthreads();
-    if (tid != 0) return;
     double thr;
     long long nr_sign;
-    if (p.ncand <= kGather && nc > 0) {
-        // rank within the bin; without a crossing (rounding) the smallest element, as the reference's loop ends
-        const long long rank = s_ok ? s_rank : (long long)nc - 1;
-        thr = s_c[n2 - 1 - rank];
-        nr_sign = p.above_cnt + rank + 1;
+    if (ncand <= kGather && nc > 0) {
+        // without a crossing (rounding) the smallest element, as the reference's loop ends
+        long long rank = s_rank;
+        if (all && a.maxsig > 0 && rank + 1 > a.maxsig) rank = a.maxsig - 1;
+        thr = s_w[rank];
+        nr_sign = (all ? 0 : p.above_cnt) + rank + 1;
     } else {
         // all 64 bits fixed and more than kGather equal elements: the bin is one value
         thr = __longlong_as_double((long long)p.prefix);
@@ -1191,21 +1298,79 @@ __global__ void __launch_bounds__(kWBlock) k_wsel_final(WeightArgs a, WPart *__r
         if (m < 1) m = 1;
         nr_sign = p.above_cnt + m;
     }
-    p.thr = thr;
-    p.nr_sign = nr_sign;
+    if (!all) {
+        if (tid == 0) {
+            p.thr = thr;
+            p.nr_sign = nr_sign;
+            a.njobs[b] = 0;
+        }
+        for (int o = tid; o < a.or_cnt[b]; o += kBlock) a.ocnt[a.oc_off[b] + o] = 0;
+        return;
+    }
+    int mine = 0;
+    for (int i = tid; i < nc; i += kBlock) mine += s_w[i] >= thr ? 1 : 0;
+    if (mine) atomicAdd(&s_above, mine);
+    const double best_w = s_w[0];
+    const int best_i = s_i[0];
+    __syncthreads();
+    const int na = s_above;
+    int m2 = 2;
+    while (m2 < na) m2 <<= 1;
+    for (int i = tid; i < m2; i += kBlock)
+        if (i >= na) s_i[i] = 0x7fffffff;
+    __syncthreads();
+    for (int ks = 2; ks <= m2; ks <<= 1)  // ascending entries
+        for (int j = ks >> 1; j > 0; j >>= 1) {
+            for (int i = tid; i < m2; i += kBlock) {
+                const int l = i ^ j;
+                if (l > i) {
+                    const int x = s_i[i], y = s_i[l];
+                    if (((i & ks) == 0) ? (x > y) : (x < y)) {
+                        s_i[i] = y;
+                        s_i[l] = x;
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    int jobs = 0;
+    for (int i = tid; i < na; i += kBlock) {
+        const int e = s_i[i];
+        a.cand_i[(size_t)b * kGather + i] = e;
+        jobs += (i == 0 || e / a.NT != s_i[i - 1] / a.NT) ? 1 : 0;
+    }
+    int n_jobs;
+    block_exclusive_scan_i(jobs, tmp, n_jobs);
+    if (tid == 0) {
+        p.thr = thr;
+        p.nr_sign = nr_sign;
+        p.n_above = na;
+        st.threshold = thr;
+        st.nr_sign = nr_sign;
+        st.n_above = na;
+        st.max_weight = best_w;
+        st.best_key = st.best_index = best_i;
+        if (nr_sign == 0) st.status = -5;
+        a.stats[b] = st;
+        a.npairs[b] = na;
+        a.njobs[b] = n_jobs;
+    }
 }
 
-// maxsig cap (src/ml_optimiser.cpp:8147-8157): the maxsig-th largest weight becomes the threshold. One block
-// per capped particle, radix selection by counts over the particle's entries.
-__global__ void __launch_bounds__(kWBlock) k_wsel_maxsig(WeightArgs a, WPart *__restrict__ part) {
+// maxsig cap (src/ml_optimiser.cpp:8147-8157) of the particles whose candidates are only the crossing bin: the
+// maxsig-th largest weight becomes the threshold. One block per capped particle, radix selection by counts over the
+// particle's entries.
+__global__ void __launch_bounds__(kBlock) k_wsel_maxsig(CoarseWeightArgs a) {
     __shared__ unsigned int hc[256];
     __shared__ unsigned long long s_prefix, s_mask;
     __shared__ long long s_cnt;
     const int b = blockIdx.x, tid = threadIdx.x;
-    WPart &p = part[b];
-    if (p.gather == 2 || a.maxsig <= 0 || p.nr_sign <= a.maxsig) return;
+    WPart &p = a.part[b];
+    if (p.state != kSelBin || a.maxsig <= 0 || p.nr_sign <= a.maxsig) return;
     const long long n = a.n_entries[b];
-    const double *w = a.weight + a.d2_off[b];
+    const float *d2 = a.diff2 + a.d2_off[b];
+    const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
+    const double mind = (double)__uint_as_float(p.mn_bits);
     if (tid == 0) {
         s_prefix = 0ULL;
         s_mask = 0ULL;
@@ -1213,11 +1378,11 @@ __global__ void __launch_bounds__(kWBlock) k_wsel_maxsig(WeightArgs a, WPart *__
     }
     __syncthreads();
     for (int shift = 56; shift >= 0; shift -= 8) {
-        for (int i = tid; i < 256; i += kWBlock) hc[i] = 0;
+        hc[tid] = 0;
         __syncthreads();
         const unsigned long long pre = s_prefix, msk = s_mask;
-        for (long long e = tid; e < n; e += kWBlock) {
-            const double v = w[e];
+        for (SegCursor<kBlock> k(0, a.NT); k.e < n; k.next()) {
+            const double v = coarse_weight(d2[k.e], mind, orp, trp, k.o, k.t);
             if (!(v > 0.)) continue;
             const unsigned long long key = (unsigned long long)__double_as_longlong(v);
             if ((key & msk) != pre) continue;
@@ -1246,55 +1411,49 @@ __global__ void __launch_bounds__(kWBlock) k_wsel_maxsig(WeightArgs a, WPart *__
     }
 }
 
-// mask, count above threshold, and each segment's max weight with the wsum-order tie break
-// Also counts the significant translations of every orientation entry (ocnt) and, per particle, the orientations
-// with at least one (njobs): the inputs of the fine-pass job lists.
-__global__ void __launch_bounds__(kBlock) k_wseg_mask(WeightArgs a, const WSeg *__restrict__ segs,
-                                                      WPart *__restrict__ part, WSegBest *__restrict__ best,
-                                                      int *__restrict__ ocnt, int *__restrict__ njobs) {
+// Particles with more significant poses than the candidate list holds: mask, count above threshold, significant
+// translations of every orientation entry (ocnt), orientations with at least one, and each segment's max weight, the
+// first entry among equal ones. With want_mask the mask of every particle.
+__global__ void __launch_bounds__(kBlock) k_wseg_mask(CoarseWeightArgs a) {
     __shared__ double s_bw[kBlock / 64];
-    __shared__ long long s_bk[kBlock / 64], s_bi[kBlock / 64], s_ab[kBlock / 64];
-    const WSeg sg = segs[blockIdx.x];
+    __shared__ long long s_bi[kBlock / 64], s_ab[kBlock / 64];
+    const WSeg sg = a.segs[blockIdx.x];
     const int b = sg.b;
-    const WPart p = part[b];
+    const WPart p = a.part[b];
+    const bool bin = p.state == kSelBin;
+    if (!bin && !a.want_mask) return;
     const double thr = p.thr;
-    const bool ok = p.gather != 2;
-    const double *w = a.weight + a.d2_off[b];
+    const float *d2 = a.diff2 + a.d2_off[b];
+    const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
+    const double mind = (double)__uint_as_float(p.mn_bits);
     long long above = 0;
     double bw = -1.;
-    long long bkey = 0x7fffffffffffffffLL, bidx = -1;
-    for (long long e = sg.begin + threadIdx.x; e < sg.end; e += kBlock) {
-        const double v = w[e];
-        const bool sig = ok && v >= thr && v > 0.;
-        a.mask[a.d2_off[b] + e] = sig ? 1 : 0;
+    long long bidx = 0x7fffffffffffffffLL;
+    for (SegCursor<kBlock> k(sg.begin, a.NT); k.e < sg.end; k.next()) {
+        const double v = coarse_weight(d2[k.e], mind, orp, trp, k.o, k.t);
+        const bool sig = p.state != kSelNone && v >= thr && v > 0.;
+        a.mask[a.d2_off[b] + k.e] = sig ? 1 : 0;
+        if (!bin) continue;
         above += sig ? 1 : 0;
-        if (sig) {
-            const int o = (int)(e / a.NT);
-            if (atomicAdd(&ocnt[a.oc_off[b] + o], 1) == 0) atomicAdd(&njobs[b], 1);
-        }
-        if (v > 0.) {
-            const long long key = wsum_order_key(a, b, e);
-            if (v > bw || (v == bw && key < bkey)) {
-                bw = v;
-                bkey = key;
-                bidx = e;
-            }
+        if (sig && atomicAdd(&a.ocnt[a.oc_off[b] + k.o], 1) == 0) atomicAdd(&a.njobs[b], 1);
+        if (v > 0. && v > bw) {  // ascending entries: the first of equal weights stays
+            bw = v;
+            bidx = k.e;
         }
     }
+    if (!bin) return;
     for (int o = 32; o > 0; o >>= 1) {
         above += __shfl_xor(above, o);
         const double ow = __shfl_xor(bw, o);
-        const long long ok2 = __shfl_xor(bkey, o), oi = __shfl_xor(bidx, o);
-        if (ow > bw || (ow == bw && ok2 < bkey)) {
+        const long long oi = __shfl_xor(bidx, o);
+        if (ow > bw || (ow == bw && oi < bidx)) {
             bw = ow;
-            bkey = ok2;
             bidx = oi;
         }
     }
     const int wv = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
         s_bw[wv] = bw;
-        s_bk[wv] = bkey;
         s_bi[wv] = bidx;
         s_ab[wv] = above;
     }
@@ -1302,54 +1461,51 @@ __global__ void __launch_bounds__(kBlock) k_wseg_mask(WeightArgs a, const WSeg *
     if (threadIdx.x == 0) {
         for (int i = 1; i < kBlock / 64; ++i) {
             above += s_ab[i];
-            if (s_bw[i] > bw || (s_bw[i] == bw && s_bk[i] < bkey)) {
+            if (s_bw[i] > bw || (s_bw[i] == bw && s_bi[i] < bidx)) {
                 bw = s_bw[i];
-                bkey = s_bk[i];
                 bidx = s_bi[i];
             }
         }
-        if (above) atomicAdd((unsigned long long *)&part[b].n_above, (unsigned long long)above);
-        best[blockIdx.x] = WSegBest{bw, bkey, bidx};
+        if (above) atomicAdd((unsigned long long *)&a.part[b].n_above, (unsigned long long)above);
+        a.best[blockIdx.x] = WSegBest{bw, bidx, bidx};
     }
 }
 
-// per particle: PassStats from the particle state and its segments' maxima
-__global__ void __launch_bounds__(kBlock) k_wsel_stats(const WPart *__restrict__ part, const int *__restrict__ seg_first,
-                                                       const WSegBest *__restrict__ best, int B, int fine,
-                                                       PassStats *__restrict__ stats, int *__restrict__ npairs) {
-    const int b = blockIdx.x * kBlock + threadIdx.x;
-    if (b >= B) return;
-    const WPart p = part[b];
-    npairs[b] = (int)p.n_above;
-    PassStats st;
+// per particle of k_wseg_mask: PassStats from the particle state and its segments' maxima. One wave per particle.
+__global__ void __launch_bounds__(kBlock) k_wsel_stats(CoarseWeightArgs a) {
+    const int b = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (b >= a.B) return;
+    const WPart p = a.part[b];
+    if (p.state != kSelBin) return;
+    double bw = -1.;
+    long long bidx = 0x7fffffffffffffffLL;
+    for (int s = a.seg_first[b] + lane; s < a.seg_first[b + 1]; s += 64) {
+        const WSegBest q = a.best[s];
+        if (q.w > bw || (q.w == bw && q.idx < bidx)) {
+            bw = q.w;
+            bidx = q.idx;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const double ow = __shfl_xor(bw, o);
+        const long long oi = __shfl_xor(bidx, o);
+        if (ow > bw || (ow == bw && oi < bidx)) {
+            bw = ow;
+            bidx = oi;
+        }
+    }
+    if (lane != 0) return;
+    PassStats st{};
     st.min_diff2 = (double)__uint_as_float(p.mn_bits);
     st.sum_weight = p.sum;
     st.threshold = p.thr;
     st.nr_sign = p.nr_sign;
     st.n_above = p.n_above;
-    st.status = p.status;
-    st.pad_ = 0;
-    double bw = -1.;
-    long long bkey = 0x7fffffffffffffffLL, bidx = -1;
-    for (int s = seg_first[b]; s < seg_first[b + 1]; ++s) {
-        const WSegBest q = best[s];
-        if (q.w > bw || (q.w == bw && q.key < bkey)) {
-            bw = q.w;
-            bkey = q.key;
-            bidx = q.idx;
-        }
-    }
-    st.max_weight = p.status ? 0. : bw;
-    st.best_key = p.status ? -1 : bkey;
-    st.best_index = p.status ? -1 : bidx;
-    if (!p.status) {
-        if (!fine && p.nr_sign == 0) st.status = -5;
-    } else {
-        st.threshold = 0.;
-        st.nr_sign = 0;
-        st.n_above = 0;
-    }
-    stats[b] = st;
+    st.max_weight = bw;
+    st.best_key = st.best_index = bidx;
+    if (p.nr_sign == 0) st.status = -5;
+    a.npairs[b] = (int)p.n_above;
+    a.stats[b] = st;
 }
 
 // --------------------------------------------------------------------------------------------------
@@ -1365,34 +1521,6 @@ struct FineJob {
     int s_begin;    // first pair (particle-local)
     int s_count;    // number of significant translations
 };
-
-
-__device__ __forceinline__ int block_exclusive_scan_i(int v, int *tmp, int &total) {
-    // wave-level inclusive scan
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o);
-        if (lane >= o) x += y;
-    }
-    __syncthreads();
-    if (lane == 63) tmp[w] = x;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) {
-            const int t = tmp[i];
-            tmp[i] = acc;
-            acc += t;
-        }
-        tmp[blockDim.x >> 6] = acc;
-    }
-    __syncthreads();
-    const int r = x - v + tmp[w];
-    total = tmp[blockDim.x >> 6];
-    __syncthreads();
-    return r;
-}
 
 
 // Offsets of the chunk's fine pass from the per-particle counts: exclusive scans over particles of pairs and
@@ -1432,9 +1560,10 @@ __global__ void __launch_bounds__(kWBlock) k_fine_plan(const int *__restrict__ n
     }
 }
 
-// Writes pairs and jobs at the offsets computed by k_fine_plan from the per-orientation significant counts
-// (ocnt, counted by k_wseg_mask). grid (B), block 1024.
-__global__ void __launch_bounds__(kWBlock) k_write_jobs(const unsigned char *__restrict__ mask,
+// Writes pairs and jobs at the offsets computed by k_fine_plan: from the particle's ordered list of significant
+// entries (kSelAll), or from the mask and the per-orientation significant counts (k_wseg_mask). grid (B), block 1024.
+__global__ void __launch_bounds__(kWBlock) k_write_jobs(const WPart *__restrict__ part, const int *__restrict__ sig,
+                                                        const unsigned char *__restrict__ mask,
                                                         const long long *__restrict__ d2_off,
                                                         const int *__restrict__ or_cnt, const int *__restrict__ oc_off,
                                                         const int *__restrict__ ocnt, int NT,
@@ -1443,9 +1572,33 @@ __global__ void __launch_bounds__(kWBlock) k_write_jobs(const unsigned char *__r
                                                         FineJob *__restrict__ jobs, const FinePlan *__restrict__ plan) {
     __shared__ int tmp[24];
     const int b = blockIdx.x;
-    if (plan && (plan->overflow || b >= plan->B)) return;
-    const unsigned char *m = mask + d2_off[b];
+    if (plan->overflow || b >= plan->B) return;
+    const int state = part[b].state;
+    if (state == kSelNone) return;
     int pair_base = 0, job_base = 0;
+    if (state == kSelAll) {
+        const int *e = sig + (size_t)b * kGather;
+        const int na = (int)part[b].n_above;
+        for (int i0 = 0; i0 < na; i0 += kWBlock) {
+            const int i = i0 + threadIdx.x;
+            int o = 0, first = 0;
+            if (i < na) {
+                o = e[i] / NT;
+                first = (i == 0 || e[i - 1] / NT != o) ? 1 : 0;
+                pairs[pair_off[b] + i] = e[i];
+            }
+            int tot_j;
+            const int js = block_exclusive_scan_i(first, tmp, tot_j);
+            if (first) {
+                int c = 1;  // its entries follow
+                while (i + c < na && e[i + c] / NT == o) ++c;
+                jobs[job_off[b] + job_base + js] = FineJob{b, o, i, c};
+            }
+            job_base += tot_j;
+        }
+        return;
+    }
+    const unsigned char *m = mask + d2_off[b];
     const int n_o = or_cnt[b];
     for (int o0 = 0; o0 < n_o; o0 += kWBlock) {
         const int o = o0 + threadIdx.x;
