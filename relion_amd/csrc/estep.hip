@@ -54,8 +54,8 @@ int pack_device_into_projector(rln_projector *p, const float2 *dev_plain, hipStr
 // Sums the backprojector's corner slots into plain [z][y][x] data (re, im) and weight volumes on the device.
 int fold_backprojector_device(rln_backprojector *b, float *re, float *im, float *w, hipStream_t st) {
     const rlnk::VolGeom g{b->dims.xdim, b->dims.ydim, b->dims.zdim, b->dims.inity, b->dims.initz};
-    hipLaunchKernelGGL(rlnk::k_fold_slots, dim3(rlnk::fold_blocks(g)), dim3(rlnk::kBlock), 0, st,
-                       b->slots.as<const float>(), g, 0, re, im, w);
+    hipLaunchKernelGGL(rlnk::k_fold_slots, rlnk::fold_grid(g, g.zdim), dim3(rlnk::kBlock), 0, st,
+                       b->slots.as<const float4>(), g, 0, g.zdim, re, im, w);
     HIP_TRY(hipGetLastError());
     return RLN_OK;
 }
@@ -1898,6 +1898,8 @@ extern "C" int rln_backprojector_set_mdl_dim(rln_backprojector *b, int xdim, int
         b->slots.release();
         b->dims = d;
         RLN_TRY(b->slots.ensure(sizeof(float) * rlnk::kSlot * b->bases()));
+        // the slots out of reach are never written again (k_zero_slots)
+        HIP_TRY(hipMemset(b->slots.ptr, 0, sizeof(float) * rlnk::kSlot * b->bases()));
     }
     if (bytes) *bytes = sizeof(float) * rlnk::kSlot * b->bases();
     return RLN_OK;
@@ -1906,7 +1908,12 @@ extern "C" int rln_backprojector_set_mdl_dim(rln_backprojector *b, int xdim, int
 extern "C" int rln_backprojector_init_mdl(rln_backprojector *b) {
     if (!b || !b->slots.ptr) RLN_FAIL(RLN_ERR_STATE, "backprojector not dimensioned");
     HIP_TRY(hipSetDevice(b->device));
-    HIP_TRY(hipMemset(b->slots.ptr, 0, sizeof(float) * rlnk::kSlot * b->bases()));
+    const rlnk::VolGeom g{b->dims.xdim, b->dims.ydim, b->dims.zdim, b->dims.inity, b->dims.initz};
+    const size_t bricks = b->bases() >> (3 * rlnk::kBrickLog);
+    hipLaunchKernelGGL(rlnk::k_zero_slots, dim3((unsigned)std::min<size_t>(bricks, 4096)), dim3(rlnk::kBlock), 0, 0,
+                       b->slots.as<float4>(), g);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(0));  // the engines' streams do not wait for the null stream
     return RLN_OK;
 }
 
@@ -1918,10 +1925,7 @@ extern "C" int rln_backprojector_get_mdl_data(rln_backprojector *b, float *real,
     rln::DevBuf plain;
     RLN_TRY(plain.ensure(3 * sizeof(float) * nv));
     float *d_re = plain.as<float>(), *d_im = d_re + nv, *d_w = d_im + nv;
-    const rlnk::VolGeom g{b->dims.xdim, b->dims.ydim, b->dims.zdim, b->dims.inity, b->dims.initz};
-    hipLaunchKernelGGL(rlnk::k_fold_slots, dim3(rlnk::fold_blocks(g)), dim3(rlnk::kBlock), 0, 0,
-                       b->slots.as<const float>(), g, 0, d_re, d_im, d_w);
-    HIP_TRY(hipGetLastError());
+    RLN_TRY(rln::fold_backprojector_device(b, d_re, d_im, d_w, 0));
     HIP_TRY(hipDeviceSynchronize());
     if (real) HIP_TRY(hipMemcpy(real, d_re, sizeof(float) * nv, hipMemcpyDeviceToHost));
     if (imag) HIP_TRY(hipMemcpy(imag, d_im, sizeof(float) * nv, hipMemcpyDeviceToHost));
@@ -1976,8 +1980,8 @@ extern "C" int rln_backprojector_get_mdl_data_noalloc(rln_backprojector *b, floa
         const int z0 = 4 * l0, nz = std::min(4 * nl, d.zdim - z0);
         const size_t stride = 4 * (size_t)nl * plane;  // floats per component in the staging array
         float *d_re = sp, *d_im = sp + stride, *d_w = sp + 2 * stride;
-        hipLaunchKernelGGL(rlnk::k_fold_slots, dim3(rlnk::fold_blocks(g, nl)), dim3(rlnk::kBlock), 0, 0,
-                           b->slots.as<const float>(), g, l0, d_re, d_im, d_w);
+        hipLaunchKernelGGL(rlnk::k_fold_slots, rlnk::fold_grid(g, nz), dim3(rlnk::kBlock), 0, 0,
+                           b->slots.as<const float4>(), g, z0, nz, d_re, d_im, d_w);
         HIP_TRY(hipGetLastError());
         // synchronous copies on the null stream: the next pass overwrites the staging only after they complete
         const size_t off = (size_t)z0 * plane, bytes = sizeof(float) * (size_t)nz * plane;

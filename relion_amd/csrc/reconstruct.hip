@@ -3,11 +3,12 @@
 // backprojector's accumulated data and weight never leave the device:
 //   k_rc_init        decenter data and weight into the half-complex layout of the pad_size^3 box, MAP
 //                    regularisation of the weight per shell, division by normalise, Fnewweight = 1 in the sphere
-//   without gridding iterations (skip_gridding, relion_refine's default): k_rc_radavg (shell sums of the weight),
-//                    k_rc_skip (data / max(weight, shell average / 1000))
+//   without gridding iterations (skip_gridding, relion_refine's default): k_rc_radavg (shell sums of the regularised
+//                    weight), k_rc_skip_window (data / max(weight, shell average / 1000) straight into the padded box)
 //   gridding iterations (max_iter_preweight): k_rc_product (Fconv = Fnewweight * Fweight), Z2D, k_rc_blob (times the
 //                    tabulated blob transform in real space), D2Z, k_rc_update (Fnewweight /= max(1e-6, |Fconv|))
-//   k_rc_window      Fconv = data * Fnewweight, window to the padded box, CenterFFTbySign; Z2D
+//   k_rc_window      Fconv = data * Fnewweight, window to the padded box, CenterFFTbySign
+//   Z2D of the padded box
 //   k_rc_bg, k_rc_out  real-space window to the original box, 1 / (pad^3 ori), soft mask with the average background,
 //                    griddingCorrect
 // Everything in FP64 (hipFFT D2Z / Z2D), as the reference's default CPU build (DoublePrec_CPU, CMakeLists.txt:135)
@@ -40,6 +41,23 @@ struct Geo {
 
 __device__ __forceinline__ int fftw_k(int k, int n, int ncols) { return k < ncols ? k : k - n; }
 
+// Weight of the element at squared radius r2 <= max_r2 with its MAP term (src/backprojector.cpp:1440-1473).
+__device__ __forceinline__ double map_weight(double fw, long long r2, const Geo &g, int do_map,
+                                             const double *__restrict__ tau2, int ntau2, double inv_ovs_fudge,
+                                             int minres_map) {
+    if (do_map && r2 < g.max_r2) {
+        const int ires = (int)floor(sqrt((double)r2) / g.pad + 0.5);
+        const double t = tau2[min(ires, ntau2 - 1)];
+        double inv = 0.;
+        if (t > 0.)
+            inv = inv_ovs_fudge / t;
+        else if (fw > 1e-20)
+            inv = 1. / (0.001 * fw);
+        if (ires >= minres_map) fw += inv;
+    }
+    return fw;
+}
+
 // Decenter (src/projector.h:249-259), MAP regularisation (src/backprojector.cpp:1440-1473), normalise, initial
 // Fnewweight. One thread per element of the half-complex S^3 layout [S][S][h+1].
 __global__ void __launch_bounds__(kThreads) k_rc_init(const float *__restrict__ re, const float *__restrict__ im,
@@ -63,16 +81,7 @@ __global__ void __launch_bounds__(kThreads) k_rc_init(const float *__restrict__ 
         fw = (double)w[src];
         fd = make_double2((double)re[src], (double)im[src]);
     }
-    if (do_map && r2 < g.max_r2) {
-        const int ires = (int)floor(sqrt((double)r2) / g.pad + 0.5);
-        const double t = tau2[min(ires, ntau2 - 1)];
-        double inv = 0.;
-        if (t > 0.)
-            inv = inv_ovs_fudge / t;
-        else if (fw > 1e-20)
-            inv = 1. / (0.001 * fw);
-        if (ires >= minres_map) fw += inv;
-    }
+    fw = map_weight(fw, r2, g, do_map, tau2, ntau2, inv_ovs_fudge, minres_map);
     fweight[e] = fw / normalise;
     fnew[e] = r2 < g.max_r2 ? 1. : 0.;
     fdata[e] = make_double2(fd.x / normalise, fd.y / normalise);
@@ -80,57 +89,77 @@ __global__ void __launch_bounds__(kThreads) k_rc_init(const float *__restrict__ 
 
 // Radial sums of the regularised weight for the path without gridding iterations (src/backprojector.cpp:1513-1532):
 // shells FLOOR(r / pad) over r^2 < ROUND((r_max pad)^2), FP64 shared-memory bins; grid-stride over a bounded
-// grid so that each global bin takes few atomics.
-__global__ void __launch_bounds__(kThreads) k_rc_radavg(const double *__restrict__ fweight, Geo g, long long round_max_r2,
+// grid so that each global bin takes few atomics. w: the folded weight, centred [S][S][h+1].
+__global__ void __launch_bounds__(kThreads) k_rc_radavg(const float *__restrict__ w, Geo g, int do_map,
+                                                        const double *__restrict__ tau2, int ntau2,
+                                                        double inv_ovs_fudge, int minres_map, long long round_max_r2,
                                                         int r_max, double *__restrict__ acc) {
-    __shared__ double s_sum[kMaxShells], s_cnt[kMaxShells];
-    for (int t = threadIdx.x; t < r_max; t += kThreads) s_sum[t] = s_cnt[t] = 0.;
+    __shared__ double s_sum[kMaxShells];
+    __shared__ unsigned int s_cnt[kMaxShells];
+    for (int t = threadIdx.x; t < r_max; t += kThreads) {
+        s_sum[t] = 0.;
+        s_cnt[t] = 0;
+    }
     __syncthreads();
     const int S = g.S, xs = g.h + 1;
-    const size_t n = (size_t)S * S * xs;
-    for (size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x; e < n; e += (size_t)gridDim.x * kThreads) {
-        const int j = (int)(e % xs);
-        const size_t zy = e / xs;
-        const int i = (int)(zy % S), k = (int)(zy / S);
-        const int kp = fftw_k(k, S, xs), ip = fftw_k(i, S, xs);
-        const long long r2 = (long long)kp * kp + (long long)ip * ip + (long long)j * j;
-        if (r2 < round_max_r2) {
+    // whole rows (z, y), so that the index arithmetic is a division per row
+    for (int zy = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); zy < S * S; zy += gridDim.x * (kThreads / 64)) {
+        const int kp = zy / S - g.h, ip = zy - (zy / S) * S - g.h;
+        const long long r2zy = (long long)kp * kp + (long long)ip * ip;
+        if (r2zy >= round_max_r2) continue;
+        for (int j = threadIdx.x & 63; j < xs; j += 64) {
+            const long long r2 = r2zy + (long long)j * j;
+            if (r2 >= round_max_r2) break;
+            const double fw = r2 <= g.max_r2 ? (double)w[(size_t)zy * xs + j] : 0.;
             const int ires = min((int)floor(sqrt((double)r2) / g.pad), r_max - 1);
-            atomicAdd(&s_sum[ires], fweight[e]);
-            atomicAdd(&s_cnt[ires], 1.);
+            atomicAdd(&s_sum[ires], map_weight(fw, r2, g, do_map, tau2, ntau2, inv_ovs_fudge, minres_map));
+            atomicAdd(&s_cnt[ires], 1u);
         }
     }
     __syncthreads();
     for (int t = threadIdx.x; t < r_max; t += kThreads)
-        if (s_cnt[t] != 0.) {
+        if (s_cnt[t]) {
             atomicAdd(&acc[t], s_sum[t]);
-            atomicAdd(&acc[r_max + t], s_cnt[t]);
+            atomicAdd(&acc[r_max + t], (double)s_cnt[t]);
         }
 }
 
-// data / max(weight, radial average / 1000), no division where that is 0 (src/backprojector.cpp:1535-1571); the
-// gridding weight becomes 1 everywhere so that the window keeps every decentred element.
-__global__ void __launch_bounds__(kThreads) k_rc_skip(const double *__restrict__ fweight, Geo g, int r_max,
-                                                      const double *__restrict__ acc, double2 *__restrict__ fdata,
-                                                      double *__restrict__ fnew) {
-    const int S = g.S, xs = g.h + 1;
-    const size_t n = (size_t)S * S * xs;
+// The path without gridding iterations from the folded sums (centred [S][S][h+1] FP32) to the padded transform: data /
+// max(weight, radial average / 1000), no division where that is 0 (src/backprojector.cpp:1535-1571), windowed as by
+// k_rc_window with a gridding weight of 1, CenterFFTbySign. One pass over the folded sums: through FP64 arrays of the
+// S box (weight, data and gridding weight written, read back, written and read again) it took 1.75 ms at box 256. One
+// thread per P element.
+__global__ void __launch_bounds__(kThreads) k_rc_skip_window(const float *__restrict__ re, const float *__restrict__ im,
+                                                             const float *__restrict__ w, Geo g, int do_map,
+                                                             const double *__restrict__ tau2, int ntau2,
+                                                             double inv_ovs_fudge, int minres_map, int r_max,
+                                                             const double *__restrict__ acc, int P,
+                                                             double2 *__restrict__ out) {
+    const int xp = P / 2 + 1, S = g.S, xs = g.h + 1;
+    const size_t n = (size_t)P * P * xp;
     const size_t e = (size_t)blockIdx.x * kThreads + threadIdx.x;
     if (e >= n) return;
-    const int j = (int)(e % xs);
-    const size_t zy = e / xs;
-    const int i = (int)(zy % S), k = (int)(zy / S);
-    const int kp = fftw_k(k, S, xs), ip = fftw_k(i, S, xs);
-    const long long r2 = (long long)kp * kp + (long long)ip * ip + (long long)j * j;
-    const int ires = min((int)floor(sqrt((double)r2) / g.pad), r_max - 1);
-    const double c = acc[r_max + ires];
-    const double avg = c > 0. ? acc[ires] / (1000. * c) : 0.;
-    const double w = fmax(fweight[e], avg);
-    if (w != 0.) {
-        const double2 d = fdata[e];
-        fdata[e] = make_double2(d.x / w, d.y / w);
+    const int jp = (int)(e % xp);
+    const int zy = (int)(e / xp);
+    const int i = zy % P, k = zy / P;
+    const int kp = fftw_k(k, P, xp), ip = fftw_k(i, P, xp);
+    const long long r2 = (long long)kp * kp + (long long)ip * ip + (long long)jp * jp;
+    // shrinking: every element of the smaller transform; growing: those of the smaller one within (S/2)^2; the data
+    // end at max_r2 either way
+    const bool take = r2 <= g.max_r2 && (xp <= xs || r2 <= (long long)g.h * g.h);
+    double2 v = make_double2(0., 0.);
+    if (take) {
+        const size_t src = ((size_t)(kp + g.h) * S + (ip + g.h)) * xs + jp;
+        const double fw = map_weight((double)w[src], r2, g, do_map, tau2, ntau2, inv_ovs_fudge, minres_map);
+        const int ires = min((int)floor(sqrt((double)r2) / g.pad), r_max - 1);
+        const double c = acc[r_max + ires];
+        const double avg = c > 0. ? acc[ires] / (1000. * c) : 0.;
+        const double d = fmax(fw, avg);
+        v = make_double2((double)re[src], (double)im[src]);
+        if (d != 0.) v = make_double2(v.x / d, v.y / d);
+        if ((k + i + jp) & 1) v = make_double2(-v.x, -v.y);
     }
-    fnew[e] = 1.;
+    out[e] = v;
 }
 
 __global__ void __launch_bounds__(kThreads) k_rc_product(const double *__restrict__ fnew, const double *__restrict__ fweight,
@@ -350,41 +379,53 @@ extern "C" int rln_backprojector_reconstruct(rln_backprojector *b, int ori_size,
     DevBuf &d_plain = ws.buf[0], &d_fw = ws.buf[1], &d_fn = ws.buf[2], &d_fd = ws.buf[3], &d_fc = ws.buf[4],
            &d_m = ws.buf[5], &d_table = ws.buf[6], &d_tau = ws.buf[7], &d_acc = ws.buf[8], &d_out = ws.buf[9];
     RLN_TRY(d_plain.ensure(3 * sizeof(float) * nv));
-    RLN_TRY(d_fw.ensure(sizeof(double) * nS));
-    RLN_TRY(d_fn.ensure(sizeof(double) * nS));
-    RLN_TRY(d_fd.ensure(sizeof(double2) * nS));
-    RLN_TRY(d_fc.ensure(sizeof(double2) * std::max(nS, nP)));
-    RLN_TRY(d_m.ensure(sizeof(double) * std::max(nR, nPr)));
-    RLN_TRY(d_table.ensure(sizeof(double) * rlnc::kBlobTable));
+    if (gridding) {
+        RLN_TRY(d_fw.ensure(sizeof(double) * nS));
+        RLN_TRY(d_fn.ensure(sizeof(double) * nS));
+        RLN_TRY(d_fd.ensure(sizeof(double2) * nS));
+        RLN_TRY(d_table.ensure(sizeof(double) * rlnc::kBlobTable));
+    }
+    RLN_TRY(d_fc.ensure(sizeof(double2) * std::max(gridding ? nS : 0, nP)));
+    RLN_TRY(d_m.ensure(sizeof(double) * std::max(gridding ? nR : 0, nPr)));
     RLN_TRY(d_tau.ensure(sizeof(double) * std::max(1, n_tau2)));
     RLN_TRY(d_acc.ensure(sizeof(double) * 2 * r_max));
     float *re = d_plain.as<float>(), *im = re + nv, *wt = im + nv;
     RLN_TRY(rln::fold_backprojector_device(b, re, im, wt, st));
-    // blob transform table (radius 2 * 1.9, alpha 15, order 0: src/backprojector.h:80, 113-115)
-    std::vector<double> table(rlnc::kBlobTable);
-    for (int i = 0; i < rlnc::kBlobTable; ++i) table[i] = rlnc::kaiser_ft(i * (0.5 / rlnc::kBlobTable), 2. * 1.9, 15.);
-    HIP_TRY(hipMemcpyAsync(d_table.ptr, table.data(), sizeof(double) * table.size(), hipMemcpyHostToDevice, st));
+    // blob transform table (radius 2 * 1.9, alpha 15, order 0: src/backprojector.h:80, 113-115), the same for every map
+    if (gridding) {
+        static const std::vector<double> table = [] {
+            std::vector<double> t(rlnc::kBlobTable);
+            for (int i = 0; i < rlnc::kBlobTable; ++i) t[i] = rlnc::kaiser_ft(i * (0.5 / rlnc::kBlobTable), 2. * 1.9, 15.);
+            return t;
+        }();
+        HIP_TRY(hipMemcpyAsync(d_table.ptr, table.data(), sizeof(double) * table.size(), hipMemcpyHostToDevice, st));
+    }
     if (do_map) HIP_TRY(hipMemcpyAsync(d_tau.ptr, tau2, sizeof(double) * n_tau2, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemsetAsync(d_acc.ptr, 0, sizeof(double) * 2 * r_max, st));
     auto grid = [](size_t n) { return dim3((unsigned)((n + rlnc::kThreads - 1) / rlnc::kThreads)); };
-    // reductions: at most 2048 blocks (8 per CU), each looping over its share
+    // reductions: at most 2048 blocks (8 per CU), each looping over its share of at least 16 elements a thread, so that
+    // small boxes do not spend their time on the blocks' atomics
     auto reduce_grid = [](size_t n) {
-        return dim3((unsigned)std::min<size_t>(2048, (n + rlnc::kThreads - 1) / rlnc::kThreads));
+        const size_t per = 16 * rlnc::kThreads;
+        return dim3((unsigned)std::min<size_t>(2048, (n + per - 1) / per));
     };
     const double ovs = pad * pad * pad;
-    hipLaunchKernelGGL(rlnc::k_rc_init, grid(nS), dim3(rlnc::kThreads), 0, st, re, im, wt, g, do_map ? 1 : 0,
-                       d_tau.as<const double>(), std::max(1, n_tau2), 1. / (ovs * tau2_fudge), minres_map,
-                       gridding ? normalise : 1., d_fw.as<double>(), d_fn.as<double>(), d_fd.as<double2>());
-    HIP_TRY(hipGetLastError());
-    if (!gridding) {
+    const double *tau = d_tau.as<const double>();
+    const double inv_ovs_fudge = 1. / (ovs * tau2_fudge);
+    const int nt = std::max(1, n_tau2);
+    if (gridding) {
+        hipLaunchKernelGGL(rlnc::k_rc_init, grid(nS), dim3(rlnc::kThreads), 0, st, re, im, wt, g, do_map ? 1 : 0, tau, nt,
+                           inv_ovs_fudge, minres_map, normalise, d_fw.as<double>(), d_fn.as<double>(),
+                           d_fd.as<double2>());
+    } else {
         const double rm = (double)r_max * pad;
-        hipLaunchKernelGGL(rlnc::k_rc_radavg, reduce_grid(nS), dim3(rlnc::kThreads), 0, st, d_fw.as<const double>(), g,
-                           (long long)ROUND(rm * rm), r_max, d_acc.as<double>());
-        hipLaunchKernelGGL(rlnc::k_rc_skip, grid(nS), dim3(rlnc::kThreads), 0, st, d_fw.as<const double>(), g, r_max,
-                           d_acc.as<const double>(), d_fd.as<double2>(), d_fn.as<double>());
-        HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(rlnc::k_rc_radavg, reduce_grid(nS), dim3(rlnc::kThreads), 0, st, wt, g, do_map ? 1 : 0, tau, nt,
+                           inv_ovs_fudge, minres_map, (long long)ROUND(rm * rm), r_max, d_acc.as<double>());
+        hipLaunchKernelGGL(rlnc::k_rc_skip_window, grid(nP), dim3(rlnc::kThreads), 0, st, re, im, wt, g, do_map ? 1 : 0,
+                           tau, nt, inv_ovs_fudge, minres_map, r_max, d_acc.as<const double>(), P, d_fc.as<double2>());
         HIP_TRY(hipMemsetAsync(d_acc.ptr, 0, sizeof(double) * 2, st));  // reused by the soft mask's background sums
     }
+    HIP_TRY(hipGetLastError());
     hipfftHandle c2r_s = 0, r2c_s = 0, c2r_p = 0;
     if (gridding) {
         RLN_TRY(ws.plan3d(S, HIPFFT_Z2D, st, &c2r_s));
@@ -403,9 +444,11 @@ extern "C" int rln_backprojector_reconstruct(rln_backprojector *b, int ori_size,
                            1. / (double)nR, d_fn.as<double>());
         HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(rlnc::k_rc_window, grid(nP), dim3(rlnc::kThreads), 0, st, d_fd.as<const double2>(),
-                       d_fn.as<const double>(), g, P, d_fc.as<double2>());
-    HIP_TRY(hipGetLastError());
+    if (gridding) {
+        hipLaunchKernelGGL(rlnc::k_rc_window, grid(nP), dim3(rlnc::kThreads), 0, st, d_fd.as<const double2>(),
+                           d_fn.as<const double>(), g, P, d_fc.as<double2>());
+        HIP_TRY(hipGetLastError());
+    }
     RLN_TRY(ws.plan3d(P, HIPFFT_Z2D, st, &c2r_p));
     if (hipfftExecZ2D(c2r_p, d_fc.as<hipfftDoubleComplex>(), d_m.as<hipfftDoubleReal>()) != HIPFFT_SUCCESS)
         RLN_FAIL(RLN_ERR_HIP, "Z2D of the padded box failed");
