@@ -216,7 +216,8 @@ struct Engine {
     DevBuf d_fdiff2, d_fweight, d_fine_n, d_nent, d_foff;
     DevBuf d_fbase;  // pose-independent part of each particle's fine diff2 (FP64)
     DevBuf d_shell_acc, d_part_acc, d_pdfc_acc, d_pdfd_acc;
-    DevBuf d_shell_tot;  // [nshell] the chunk's sigma2_noise sums over its particles
+    DevBuf d_res;        // the chunk's results (k_pack_results), copied to h_res
+    PinnedBuf h_res;
     // fine pass planned on the device: capacities (elements) the buffers were sized for, the chunk capacity B,
     // the plan header, per-chunk image pointers, work items, the tuned persistent grids and the captured graph
     int cap_B = 0;
@@ -228,6 +229,7 @@ struct Engine {
     std::unique_ptr<ChunkHost> chunk_host[2];  // host lists of consecutive chunks, kept to reuse their memory
     rlnk::ChunkPtrs cp_host{};
     bool tuned = false;
+    int last_items = 0;                      // fine work items of the last chunk
     int grid_fine = 1024, grid_wsum = 2048;  // persistent grids (fine: tuned; weighted sums: resident blocks)
     int band_choice = 0;                     // index into kBandChoices of the fine pass's band count (tuned)
     int fine_shape = 0;                      // index into rlnk::kFineShapes of the work-item shape (tuned)
@@ -1011,7 +1013,6 @@ static int ensure_fine_capacity(Engine &e) {
     RLN_TRY(e.d_foff.ensure(sizeof(long long) * cB));
     RLN_TRY(e.d_stats_f.ensure(sizeof(rlnk::PassStats) * cB));
     RLN_TRY(e.d_shell_acc.ensure(sizeof(double) * e.nshell * cB));
-    RLN_TRY(e.d_shell_tot.ensure(sizeof(double) * e.nshell));
     RLN_TRY(e.d_part_acc.ensure(sizeof(double) * 8 * cB));
     RLN_TRY(e.d_pdfc_acc.ensure(sizeof(double) * e.K * cB));
     RLN_TRY(e.d_plan.ensure(sizeof(rlnk::FinePlan)));
@@ -1057,6 +1058,7 @@ struct FineLaunch {
     double *shell, *part, *pdfc;
     long long n_shell, n_part, n_pdfc;
     int grid_fine, grid_wsum;
+    int n_particles;  // of the chunk; cleared in the graph's key
 };
 
 // part 0: plan, job lists and work items; part 1: fine diff2; part 2: fine weights; part 3: weighted sums and
@@ -1072,7 +1074,7 @@ static void launch_plan(Engine &e, const FineLaunch &L) {
     const rlnk::FineShape sh = rlnk::kFineShapes[L.shape];
     hipLaunchKernelGGL(rlnk::k_fine_items, dim3(1), dim3(rlnk::kWBlock), 0, st, (const rlnk::FineJob *)L.jobs,
                        L.or_off, L.or_frame, L.or_class, L.n_or_grid, L.key_shift, L.sorted, sh.tc, 4 * sh.cw,
-                       L.cap_small, L.cap_wide, L.job_order, L.items_s, L.items_w, L.plan);
+                       L.cap_small, L.cap_wide, L.fa.n_pix, L.ws.n_wpix, L.job_order, L.items_s, L.items_w, L.plan);
 }
 
 static int launch_fine(Engine &e, const FineLaunch &L, int part) {
@@ -1111,6 +1113,7 @@ static int launch_fine(Engine &e, const FineLaunch &L, int part) {
 // A candidate replaces the best one found so far only when it is at least 1% faster, so that candidates within the
 // timing noise of each other do not alternate between engines.
 constexpr float kTuneMargin = 0.99f;
+constexpr int kTuneItems = 512;  // work items of a chunk worth tuning on
 
 static int tune_fine(Engine &e, FineLaunch L) {
     hipStream_t st = e.stream;
@@ -1135,7 +1138,7 @@ static int tune_fine(Engine &e, FineLaunch L) {
         rlnk::FinePlan plan{};
         HIP_TRY(hipMemcpyAsync(&plan, L.plan, sizeof(plan), hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
-        ok = !plan.overflow && plan.n_small + plan.n_wide >= 512;
+        ok = !plan.overflow && plan.n_small + plan.n_wide >= kTuneItems;
         return RLN_OK;
     };
     auto time_one = [&](int sh, int oi, int ci, int gi, float &ms) -> int {
@@ -1241,6 +1244,14 @@ static int tune_fine(Engine &e, FineLaunch L) {
     return RLN_OK;
 }
 
+// Band count of the weighted sums: fixed or tuned, else the plan's choice (0).
+static void set_wsum_bands(const Engine &e, rlnk::WsumArgs &ws) {
+    const bool fixed = e.tuned || e.wsum_bands > 0;
+    const int c = fixed ? wsum_band_choice(e) : 0;
+    ws.wpix = e.d_wsum_pix.as<const int2>() + (size_t)c * e.n_wsum_pix;
+    ws.n_bands = fixed ? kBandChoices[c] : 0;
+}
+
 static void drop_fine_graphs(Engine &e) {
     for (int q = 0; q < kFineGraphs; ++q) {
         if (e.fine_exec[q]) (void)hipGraphExecDestroy(e.fine_exec[q]);
@@ -1252,19 +1263,22 @@ static void drop_fine_graphs(Engine &e) {
 
 static int run_fine_stage(Engine &e, const FineLaunch &L0) {
     FineLaunch L = L0;
-    if (!e.tuned) {
-        RLN_TRY(tune_fine(e, L));
+    // tuned on the first chunk that is known to hold enough work items: one per particle at least, or as many as the
+    // chunk before (asking the device first would cost every small run a plan and a synchronisation)
+    const bool tune = !e.tuned && (L.n_particles >= kTuneItems || e.last_items >= kTuneItems);
+    if (tune) RLN_TRY(tune_fine(e, L));
+    if (tune && e.tuned) {
         L.grid_fine = e.grid_fine;
         L.shape = e.fine_shape;
         L.sorted = kFineOrders[e.fine_order].sorted;
         L.fa.item_major = kFineOrders[e.fine_order].item_major;
         L.fa.xcd_queues = kFineOrders[e.fine_order].xcd_queues;
         L.fa.n_bands = kBandChoices[e.band_choice];
-        L.ws.n_bands = kBandChoices[wsum_band_choice(e)];
-        L.ws.wpix = e.d_wsum_pix.as<const int2>() + (size_t)wsum_band_choice(e) * e.n_wsum_pix;
+        set_wsum_bands(e, L.ws);
         L.fa.pix = e.d_band_pix.as<const int2>() + (size_t)e.band_choice * e.pf_sampled;
     }
     if (!e.graph_off) {
+        L.n_particles = 0;
         const unsigned char *kb = reinterpret_cast<const unsigned char *>(&L);
         std::vector<unsigned char> key(kb, kb + sizeof(L));
         if (!e.fine_exec[0] || key != e.fine_key) {
@@ -1496,7 +1510,35 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     hipLaunchKernelGGL(rlnk::k_fine_base, dim3(B), dim3(rlnk::kBlock), 0, st, e.d_cp.as<const rlnk::ChunkPtrs>(),
                        e.d_q_f.as<const float>(), (int)Pf, d_xi2d, e.d_fbase.as<double>());
     RLN_TRY(launch_check("k_fine_base"));
+    // the chunk's results in one device block and one copy into page-locked memory
     rlnk::FinePlan plan{};
+    const rlnk::ChunkResult *res = nullptr;
+    const double *pdfc = nullptr, *shells = nullptr;
+    const size_t off_pdfc = sizeof(rlnk::ChunkResult) * B, off_shell = off_pdfc + sizeof(double) * K * B,
+                 off_plan = off_shell + sizeof(double) * e.nshell, res_bytes = off_plan + sizeof(rlnk::FinePlan);
+    auto fetch_results = [&]() -> int {
+        RLN_TRY(e.d_res.ensure(res_bytes));
+        RLN_TRY(e.h_res.ensure(res_bytes));
+        char *d = e.d_res.as<char>();
+        hipLaunchKernelGGL(rlnk::k_shell_total, dim3(e.nshell), dim3(rlnk::kBlock), 0, st,
+                           e.d_shell_acc.as<const double>(), B, e.nshell, reinterpret_cast<double *>(d + off_shell));
+        hipLaunchKernelGGL(rlnk::k_pack_results, dim3(gB), dim3(rlnk::kBlock), 0, st, e.d_plan.as<const rlnk::FinePlan>(),
+                           B, K, e.d_stats_c.as<const rlnk::PassStats>(), e.d_stats_f.as<const rlnk::PassStats>(),
+                           e.d_part_acc.as<const double>(), e.d_npairs.as<const int>(), e.d_pairs.as<const int>(),
+                           e.d_pair_off.as<const long long>(), e.d_pdfc_acc.as<const double>(),
+                           reinterpret_cast<rlnk::ChunkResult *>(d), reinterpret_cast<double *>(d + off_pdfc),
+                           reinterpret_cast<rlnk::FinePlan *>(d + off_plan));
+        RLN_TRY(launch_check("chunk results"));
+        HIP_TRY(hipEventRecord(e.ev[kStCount], st));
+        HIP_TRY(hipMemcpyAsync(e.h_res.ptr, d, res_bytes, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        const char *h0 = static_cast<const char *>(e.h_res.ptr);
+        res = reinterpret_cast<const rlnk::ChunkResult *>(h0);
+        pdfc = reinterpret_cast<const double *>(h0 + off_pdfc);
+        shells = reinterpret_cast<const double *>(h0 + off_shell);
+        std::memcpy(&plan, h0 + off_plan, sizeof(plan));
+        return RLN_OK;
+    };
     for (int attempt = 0;; ++attempt) {
         RLN_TRY(ensure_fine_capacity(e));
         FineLaunch L;
@@ -1559,9 +1601,10 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         fa.ey = e.d_ey_f.as<const float2>();
         fa.tr_ix = e.d_tr_ix.as<const int>();
         fa.tr_iy = e.d_tr_iy.as<const int>();
-        fa.pix = e.d_band_pix.as<const int2>() + (size_t)e.band_choice * e.pf_sampled;
+        // untuned: the plan picks the band count from the chunk's items
+        fa.pix = e.d_band_pix.as<const int2>() + (e.tuned ? (size_t)e.band_choice * e.pf_sampled : 0);
         fa.n_pix = (int)e.pf_sampled;
-        fa.n_bands = kBandChoices[e.band_choice];
+        fa.n_bands = e.tuned ? kBandChoices[e.band_choice] : 0;
         fa.item_major = kFineOrders[e.fine_order].item_major;
         fa.xcd_queues = kFineOrders[e.fine_order].xcd_queues;
         L.fbase = e.d_fbase.as<const double>();
@@ -1606,9 +1649,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         ws.scale_w = d_scale_w;
         ws.minv_w = e.d_minv_w.as<const float>();
         ws.mresol = e.d_mresol.as<const int>();
-        ws.wpix = e.d_wsum_pix.as<const int2>() + (size_t)wsum_band_choice(e) * e.n_wsum_pix;
         ws.n_wpix = e.n_wsum_pix;
-        ws.n_bands = kBandChoices[wsum_band_choice(e)];
+        set_wsum_bands(e, ws);
         ws.unit_order = e.wsum_order;
         ws.job_order = e.d_job_order.as<const int>();
         ws.xa_shell = (cfg.do_scale_correction && e.d_xa_shell.ptr) ? e.d_xa_shell.as<const unsigned char>() : nullptr;
@@ -1636,9 +1678,9 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         ws.K = K;
         L.grid_fine = e.grid_fine;
         L.grid_wsum = e.grid_wsum;
+        L.n_particles = B;
         RLN_TRY(run_fine_stage(e, L));
-        HIP_TRY(hipMemcpyAsync(&plan, e.d_plan.ptr, sizeof(plan), hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+        RLN_TRY(fetch_results());
         if (!plan.overflow) break;
         if (attempt >= 2) RLN_FAIL(RLN_ERR_MEMORY, "fine pass capacity not reached after %d attempts", attempt + 1);
         // grow to what the plan asked for, with headroom, and run the pass again
@@ -1650,36 +1692,17 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     }
     const long long n_pairs = plan.n_pairs;
     const int n_jobs = plan.n_jobs;
-    std::vector<int> counts(B);
-    std::vector<long long> pair_off(B), foff(B);
-    std::vector<rlnk::PassStats> stc(B);
-    HIP_TRY(hipMemcpyAsync(counts.data(), e.d_npairs.ptr, sizeof(int) * B, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(pair_off.data(), e.d_pair_off.ptr, sizeof(long long) * B, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(stc.data(), e.d_stats_c.ptr, sizeof(rlnk::PassStats) * B, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    for (int b = 0; b < B; ++b) foff[b] = 32LL * pair_off[b];
+    e.last_items = plan.n_small + plan.n_wide;
     for (int b = 0; b < B; ++b)
-        if (stc[b].status != 0) {
-            int code = stc[b].status;
+        if (res[b].c.status != 0) {
+            int code = res[b].c.status;
             RLN_FAIL(code, "coarse pass of particle %d: %s", b,
                      code == RLN_ERR_SUM_WEIGHT_ZERO ? "zero or NaN sum of weights" : "no significant samples");
         }
-    HIP_TRY(hipEventRecord(e.ev[kStCount], st));
-    // results
-    std::vector<rlnk::PassStats> stf(B);
-    std::vector<double> shells(e.nshell), pacc(8 * (size_t)B), pdfc((size_t)K * B);
-    hipLaunchKernelGGL(rlnk::k_shell_total, dim3(e.nshell), dim3(rlnk::kBlock), 0, st, e.d_shell_acc.as<const double>(),
-                       B, e.nshell, e.d_shell_tot.as<double>());
-    RLN_TRY(launch_check("shell sums"));
-    HIP_TRY(hipMemcpyAsync(stf.data(), e.d_stats_f.ptr, sizeof(rlnk::PassStats) * B, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(shells.data(), e.d_shell_tot.ptr, sizeof(double) * shells.size(), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(pacc.data(), e.d_part_acc.ptr, sizeof(double) * pacc.size(), hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(pdfc.data(), e.d_pdfc_acc.ptr, sizeof(double) * pdfc.size(), hipMemcpyDeviceToHost, st));
-    // best fine pose per particle: the pair's coarse index and the job's orientation entry
-    std::vector<int> all_pairs(std::max<long long>(1, n_pairs));
-    if (n_pairs)
-        HIP_TRY(hipMemcpyAsync(all_pairs.data(), e.d_pairs.ptr, sizeof(int) * n_pairs, hipMemcpyDeviceToHost, st));
     if (e.keep) {
+        std::vector<long long> pair_off(B);
+        HIP_TRY(hipMemcpyAsync(pair_off.data(), e.d_pair_off.ptr, sizeof(long long) * B, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipStreamSynchronize(st));
         e.kept.assign(B, Engine::Kept());
         for (int b = 0; b < B; ++b) {
             Engine::Kept &kp = e.kept[b];
@@ -1695,24 +1718,24 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
                                    sizeof(double) * kp.n_coarse, hipMemcpyDeviceToHost, st));
             HIP_TRY(hipMemcpyAsync(kp.cmask.data(), e.d_mask.as<unsigned char>() + h.d2_off[b], kp.n_coarse,
                                    hipMemcpyDeviceToHost, st));
-            const long long nf = 32LL * counts[b];
-            std::vector<int> pr(counts[b]);
+            const int n_pairs_b = res[b].n_pairs;
+            const long long nf = 32LL * n_pairs_b;
+            std::vector<int> pr(n_pairs_b);
             kp.fdiff2.resize(nf);
             kp.fweight.resize(nf);
             kp.f_index.resize(nf);
-            if (counts[b]) {
-                HIP_TRY(hipMemcpyAsync(pr.data(), e.d_pairs.as<int>() + pair_off[b], sizeof(int) * counts[b],
+            if (n_pairs_b) {
+                HIP_TRY(hipMemcpyAsync(pr.data(), e.d_pairs.as<int>() + pair_off[b], sizeof(int) * n_pairs_b,
                                        hipMemcpyDeviceToHost, st));
-                HIP_TRY(hipMemcpyAsync(kp.fdiff2.data(), e.d_fdiff2.as<double>() + foff[b], sizeof(double) * nf,
+                HIP_TRY(hipMemcpyAsync(kp.fdiff2.data(), e.d_fdiff2.as<double>() + 32 * pair_off[b], sizeof(double) * nf,
                                        hipMemcpyDeviceToHost, st));
-                HIP_TRY(hipMemcpyAsync(kp.fweight.data(), e.d_fweight.as<double>() + foff[b], sizeof(double) * nf,
+                HIP_TRY(hipMemcpyAsync(kp.fweight.data(), e.d_fweight.as<double>() + 32 * pair_off[b], sizeof(double) * nf,
                                        hipMemcpyDeviceToHost, st));
             }
             HIP_TRY(hipStreamSynchronize(st));
             for (long long f = 0; f < nf; ++f) kp.f_index[f] = (long long)pr[f >> 5] * 32 + (f & 31);
         }
     }
-    HIP_TRY(hipStreamSynchronize(st));
     const clk::time_point t_epi = clk::now();
     for (int i = 0; i < kStCount; ++i) {
         float ms = 0.f;
@@ -1727,8 +1750,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     e.counters[4] = (long long)Pf;
     e.counters[5] += (long long)plan.n_small + plan.n_wide;
     for (int b = 0; b < B; ++b) {
-        e.counters[6] += (long long)pacc[8 * b + 5];
-        e.counters[7] += (long long)pacc[8 * b + 6];
+        e.counters[6] += (long long)res[b].part[5];
+        e.counters[7] += (long long)res[b].part[6];
     }
     e.counters[9] += (long long)h.tiles.size();
     e.counters[10] += n_jobs;
@@ -1736,34 +1759,34 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     e.counters[14] = e.grid_fine;
     e.counters[15] = e.grid_wsum;
     e.counters[16] = e.pf_sampled;
-    e.counters[17] = kBandChoices[e.band_choice];
+    e.counters[17] = e.tuned ? kBandChoices[e.band_choice] : 1 << plan.fine_choice;
     e.counters[18] = rlnk::kFineShapes[e.fine_shape].tc;
     e.counters[19] = rlnk::kFineShapes[e.fine_shape].cw;
     e.counters[20] = e.fine_order;
     e.counters[21] = e.wsum_order;
-    e.counters[22] = kBandChoices[wsum_band_choice(e)];
+    e.counters[22] = e.tuned || e.wsum_bands > 0 ? kBandChoices[wsum_band_choice(e)] : 1 << plan.wsum_choice;
     for (int b = 0; b < B; ++b) {
-        if (stf[b].status != 0) RLN_FAIL(stf[b].status, "fine pass of particle %d: zero or NaN sum of weights", b);
-        if (stf[b].best_index < 0) RLN_FAIL(RLN_ERR_FILTERED_ZERO, "no positive fine weight for particle %d", b);
+        if (res[b].f.status != 0) RLN_FAIL(res[b].f.status, "fine pass of particle %d: zero or NaN sum of weights", b);
+        if (res[b].f.best_index < 0) RLN_FAIL(RLN_ERR_FILTERED_ZERO, "no positive fine weight for particle %d", b);
     }
     // per-particle results (the best pose decoded to angles and offsets) on several host threads; the sums over
     // particles below in particle order
     auto decode = [&](int b0, int b1) {
         for (int b = b0; b < b1; ++b) {
-            const rlnk::PassStats &sf = stf[b];
+            const rlnk::PassStats &sc = res[b].c, &sf = res[b].f;
             rln_particle_result &r = results[b];
             std::memset(&r, 0, sizeof(r));
-            r.coarse_min_diff2 = stc[b].min_diff2;
-            r.coarse_sum_weight = stc[b].sum_weight;
-            r.coarse_significant_weight = stc[b].threshold;
-            r.nr_significant = (double)stc[b].nr_sign;
+            r.coarse_min_diff2 = sc.min_diff2;
+            r.coarse_sum_weight = sc.sum_weight;
+            r.coarse_significant_weight = sc.threshold;
+            r.nr_significant = (double)sc.nr_sign;
             r.min_diff2 = sf.min_diff2;
             r.sum_weight = sf.sum_weight;
             r.significant_weight = sf.threshold;
-            r.nr_fine_evaluated = 32 * counts[b];
+            r.nr_fine_evaluated = 32 * res[b].n_pairs;
             r.pmax = sf.max_weight / sf.sum_weight;
             // decode the best pose
-            const int c = all_pairs[pair_off[b] + (sf.best_index >> 5)];
+            const int c = res[b].best_pair;
             const int o = c / NT, t = c % NT;
             const int rr = (int)((sf.best_index >> 2) & 7), u = (int)(sf.best_index & 3);
             const int og = h.or_frame[h.or_off[b] + o] / 8, k = h.or_class[h.or_off[b] + o];
@@ -1772,8 +1795,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
             r.yoff = meta[b].old_offset_y + e.over_y[t * 4 + u];
             r.iclass = k + 1;
             r.best_ihidden_over = ((long long)o * NT + t) * 32 + rr * 4 + u;
-            r.wsum_norm_correction = pacc[8 * b + 2];
-            double xa = pacc[8 * b + 3], aa = pacc[8 * b + 4];
+            r.wsum_norm_correction = res[b].part[2];
+            double xa = res[b].part[3], aa = res[b].part[4];
             if (cfg.do_scale_correction) {
                 xa /= meta[b].scale;
                 aa /= meta[b].scale * meta[b].scale;
@@ -1799,8 +1822,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         if (wsum) {
             if (wsum->pdf_class)
                 for (int kk = 0; kk < K; ++kk) wsum->pdf_class[kk] += pdfc[(size_t)b * K + kk];
-            wsum->sumw_group += pacc[8 * b + 0];
-            wsum->sigma2_offset += pacc[8 * b + 1];
+            wsum->sumw_group += res[b].part[0];
+            wsum->sigma2_offset += res[b].part[1];
             wsum->signal_product += xa;
             wsum->reference_power += aa;
             wsum->LL += r.dLL;
@@ -2034,7 +2057,7 @@ extern "C" int rln_estep_destroy(rln_estep *e) {
                            &e->d_njobs, &e->d_nchunks, &e->d_pair_off, &e->d_job_off, &e->d_chunk_off, &e->d_pairs,
                            &e->d_jobs, &e->d_job_order, &e->d_chunk_job, &e->d_chunk_first, &e->d_fdiff2, &e->d_fbase, &e->d_fweight,
                            &e->d_fine_n, &e->d_nent, &e->d_foff, &e->d_shell_acc, &e->d_part_acc, &e->d_pdfc_acc, &e->d_pdfd_acc,
-                           &e->d_shell_tot, &e->d_plan, &e->d_cp, &e->d_items_s, &e->d_items_w, &e->d_wsegs, &e->d_seg_first,
+                           &e->d_res, &e->d_plan, &e->d_cp, &e->d_items_s, &e->d_items_w, &e->d_wsegs, &e->d_seg_first,
                            &e->d_wpart, &e->d_hcnt, &e->d_hsum, &e->d_wcand, &e->d_wcand_i, &e->d_segbest,
                            &e->d_ocnt};
     rln::drop_fine_graphs(*e);

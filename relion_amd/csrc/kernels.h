@@ -647,8 +647,21 @@ struct FinePlan {
     int next_wsum;       // next work item of k_wsum_bp
     int next_fine_x[8];  // next work unit of each XCD's share (k_fine_diff2 with per-XCD queues)
     int next_wsum_x[8];  // the same for k_wsum_bp
+    int fine_choice;     // log2 of the band count that fills the GPU with the chunk's items (k_fine_items)
+    int wsum_choice;     // the same for the jobs of k_wsum_bp
     int pad_;
 };
+
+// log2 of the number of radial bands (1 .. 32) that cuts n items of n_pix pixels into at least 4 units per CU, as long
+// as a band keeps kMinBandPix pixels (two of a block's four waves). For engines whose band count is not tuned or fixed:
+// a few items on one band each leave most of the GPU idle. 11 items of 1,604 pixels: fine pass stage 165 us on 1 band, 54
+// on 8; weighted sums 208 and 62 us; 108 items of 6,426 pixels: 650 and 190 us, 420 and 150 us.
+constexpr int kMinBandPix = 128, kFillUnits = 1024;
+__device__ __forceinline__ int fill_choice(int n, int n_pix) {
+    int c = 0;
+    while (c < 5 && ((long long)n << c) < kFillUnits && (n_pix >> (c + 1)) >= kMinBandPix) ++c;
+    return c;
+}
 
 // Per-chunk input images (device pointers), read by the fine-pass kernels through one indirection so that a
 // captured graph of the pass serves every chunk.
@@ -1704,7 +1717,7 @@ constexpr int kJobKeys = 4096;
 __global__ void __launch_bounds__(kWBlock) k_fine_items(const FineJob *__restrict__ jobs, const int *__restrict__ or_off,
                                                         const int *__restrict__ or_frame, const int *__restrict__ or_class,
                                                         int n_or_grid, int key_shift, int sorted, int small_max,
-                                                        int wide_tc, int cap_small, int cap_wide,
+                                                        int wide_tc, int cap_small, int cap_wide, int n_pix, int n_wpix,
                                                         int *__restrict__ job_order, int2 *__restrict__ small_items,
                                                         int2 *__restrict__ wide_items, FinePlan *__restrict__ plan) {
     __shared__ int tmp[24];
@@ -1766,6 +1779,8 @@ __global__ void __launch_bounds__(kWBlock) k_fine_items(const FineJob *__restric
     if (threadIdx.x == 0) {
         plan->n_small = sbase;
         plan->n_wide = wbase;
+        plan->fine_choice = fill_choice(sbase + wbase, n_pix);
+        plan->wsum_choice = fill_choice(n_jobs, n_wpix);
         if (sbase > cap_small || wbase > cap_wide) plan->overflow = 1;
     }
 }
@@ -1794,7 +1809,8 @@ struct FineArgs {
     const int2 *pix;               // sampled pixels (Minvsigma2 > 0, inside the projection radius) as (p, x | row
                                    // << 16), in n_bands bands of equal count by radius, pixel order within a band
     int n_pix;
-    int n_bands;                   // band b: pix[b n_pix / n_bands .. (b + 1) n_pix / n_bands)
+    int n_bands;                   // band b: pix[b n_pix / n_bands .. (b + 1) n_pix / n_bands); 0: the plan's choice, pix
+                                   // the lists of all choices one after the other
     int item_major;                // unit order: 0 band-major (all items of band 0, then band 1, ...), 1 item-major
     int xcd_queues;                // 1: each XCD takes its own eighth of the items (band-major), then helps the others
     int NT;
@@ -2104,6 +2120,11 @@ __global__ void __launch_bounds__(kBlock, 3) k_fine_diff2(FineArgs a) {
     } lds;
     __shared__ int s_item;
     if (a.plan->overflow) return;
+    if (a.n_bands == 0) {
+        const int c = a.plan->fine_choice;
+        a.n_bands = 1 << c;
+        a.pix += (size_t)c * a.n_pix;
+    }
     const int n_wide = a.plan->n_wide;
     const int n_items = n_wide + a.plan->n_small;
     const int n_units = n_items * a.n_bands;
@@ -2187,7 +2208,6 @@ __global__ void k_reset_items(FinePlan *plan) {
     }
 }
 
-// Zero fill used inside captured graphs instead of memset nodes.
 // Sum over the B particles of each shell's weighted sigma2_noise contribution: block s sums column s of the
 // [B][nshell] per-particle accumulators in a fixed order (strided partial sums, then a tree). grid (nshell).
 __global__ void __launch_bounds__(kBlock) k_shell_total(const double *__restrict__ acc, int B, int nshell,
@@ -2205,6 +2225,38 @@ __global__ void __launch_bounds__(kBlock) k_shell_total(const double *__restrict
     if (tid == 0) out[s] = red[0];
 }
 
+// What the host needs of a particle at the end of a chunk.
+struct ChunkResult {
+    PassStats c, f;    // coarse and fine pass
+    double part[8];    // WsumArgs::part_acc
+    int n_pairs;       // significant coarse poses
+    int best_pair;     // coarse index of the pair that holds the best fine pose
+};
+
+// The chunk's results in one block of memory, so that they reach the host in one copy: [B] ChunkResult, then [B][K]
+// pdf_class sums, then the plan's header. (Ten separate copies of a chunk of 8 particles took 0.33 of 1.15 ms.)
+__global__ void __launch_bounds__(kBlock) k_pack_results(const FinePlan *__restrict__ plan, int B, int K,
+                                                         const PassStats *__restrict__ sc,
+                                                         const PassStats *__restrict__ sf,
+                                                         const double *__restrict__ part, const int *__restrict__ npairs,
+                                                         const int *__restrict__ pairs,
+                                                         const long long *__restrict__ pair_off,
+                                                         const double *__restrict__ pdfc, ChunkResult *__restrict__ out,
+                                                         double *__restrict__ out_pdfc, FinePlan *__restrict__ out_plan) {
+    const int b = blockIdx.x * kBlock + threadIdx.x;
+    if (b == 0) *out_plan = *plan;
+    if (b >= B || plan->overflow) return;
+    ChunkResult r;
+    r.c = sc[b];
+    r.f = sf[b];
+    for (int i = 0; i < 8; ++i) r.part[i] = part[8 * (size_t)b + i];
+    r.n_pairs = npairs[b];
+    r.best_pair = r.f.best_index >= 0 ? pairs[pair_off[b] + (r.f.best_index >> 5)] : 0;
+    out[b] = r;
+    for (int k = 0; k < K; ++k) out_pdfc[(size_t)b * K + k] = pdfc[(size_t)b * K + k];
+}
+
+// Zero fill used inside captured graphs instead of memset nodes.
 __global__ void __launch_bounds__(kBlock) k_zero_d(double *__restrict__ p, long long n) {
     for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long long)gridDim.x * kBlock) p[i] = 0.;
 }
@@ -2236,7 +2288,7 @@ struct WsumArgs {
     const int2 *wpix;               // the pixels that contribute (a shell >= 0 or backprojected) as (p, x | row << 16),
                                     // n_bands bands of equal count by radius, pixel order within a band
     int n_wpix;
-    int n_bands;
+    int n_bands;                    // 0: the plan's choice, wpix the lists of all choices one after the other
     int unit_order;                 // 0 band-major, 1 item-major (the bands of a job in a row), 2 band-major in per-XCD
                                     // queues
     const unsigned char *xa_shell;  // [K][nshell] data_vs_prior > 3 (scale correction) or null
@@ -2276,6 +2328,11 @@ __global__ void __launch_bounds__(kBlock, 5) k_wsum_bp(WsumArgs a) {
     __shared__ float sx_w[kBlock][8];
     __shared__ int s_item;
     if (a.plan->overflow) return;
+    if (a.n_bands == 0) {
+        const int c = a.plan->wsum_choice;
+        a.n_bands = 1 << c;
+        a.wpix += (size_t)c * a.n_wpix;
+    }
     const int n_items = a.plan->n_jobs;
     const int n_units = n_items * a.n_bands;
     const int tid = threadIdx.x;
