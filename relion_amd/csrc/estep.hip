@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -39,14 +40,19 @@ const char *last_error() { return g_last_error.c_str(); }
 #include "host_common.h"
 
 namespace rln {
-// Packs a plain [z][y][x] float2 volume already on the device into the projector's corner layout.
-int pack_device_into_projector(rln_projector *p, const float2 *dev_plain, hipStream_t st) {
+// Packs a plain [z][y][x] float2 volume already on the device into the projector's corner layout. windowed: the volume
+// is zero beyond ROUND(pad maxr), so only base voxels within one corner of that radius are packed, and the bricks beyond
+// are cleared once for as long as only windowed volumes follow.
+int pack_device_into_projector(rln_projector *p, const float2 *dev_plain, bool windowed, hipStream_t st) {
     const rln::MdlDims &d = p->dims;
     const rlnk::VolGeom g{d.xdim, d.ydim, d.zdim, d.inity, d.initz};
-    const size_t n = p->bases();
-    hipLaunchKernelGGL(rlnk::k_pack_volume, dim3((unsigned)((n + rlnk::kBlock - 1) / rlnk::kBlock)),
-                       dim3(rlnk::kBlock), 0, st, dev_plain, g, p->data.as<float4>());
+    const size_t bricks = p->bases() >> (3 * rlnk::kBrickLog);
+    const long long reach = ROUND(d.pad * d.maxr) + 2;
+    hipLaunchKernelGGL(rlnk::k_pack_volume, dim3((unsigned)((bricks + rlnk::kPackBricks - 1) / rlnk::kPackBricks)),
+                       dim3(rlnk::kBlock), 0, st, dev_plain, g, windowed ? reach * reach : LLONG_MAX,
+                       p->far_zero ? 0 : 1, p->data.as<float4>());
     HIP_TRY(hipGetLastError());
+    p->far_zero = windowed;
     p->version++;
     return RLN_OK;
 }
@@ -66,11 +72,7 @@ static int pack_into_projector(rln_projector *p, const float2 *host_plain) {
     DevBuf plain;
     RLN_TRY(plain.ensure(sizeof(float2) * d.voxels()));
     HIP_TRY(hipMemcpy(plain.ptr, host_plain, sizeof(float2) * d.voxels(), hipMemcpyHostToDevice));
-    const rlnk::VolGeom g{d.xdim, d.ydim, d.zdim, d.inity, d.initz};
-    const size_t n = p->bases();
-    hipLaunchKernelGGL(rlnk::k_pack_volume, dim3((unsigned)((n + rlnk::kBlock - 1) / rlnk::kBlock)),
-                       dim3(rlnk::kBlock), 0, 0, plain.as<const float2>(), g, p->data.as<float4>());
-    HIP_TRY(hipGetLastError());
+    RLN_TRY(pack_device_into_projector(p, plain.as<const float2>(), false, 0));
     HIP_TRY(hipDeviceSynchronize());
     return RLN_OK;
 }
@@ -1866,6 +1868,7 @@ extern "C" int rln_projector_set_mdl_dim(rln_projector *p, int xdim, int ydim, i
     p->data.release();
     p->dims = d;
     RLN_TRY(p->data.ensure(4 * sizeof(float4) * p->bases()));
+    p->far_zero = false;
     p->version++;
     return RLN_OK;
 }

@@ -109,6 +109,7 @@ struct rln_projector {
     int device = 0;
     rln::MdlDims dims;
     rln::DevBuf data;  // corner-packed volume: 4 float4 per trilinear base voxel, in bricks
+    bool far_zero = false;  // the bricks beyond ROUND(pad maxr) + 2 hold zeros
     unsigned long long version = 0;
     size_t bases() const { return rlnk::packed_bases(dims.xdim, dims.ydim, dims.zdim); }
 };
@@ -122,7 +123,7 @@ struct rln_backprojector {
 
 namespace rln {
 // Packs a plain [z][y][x] float2 volume on the device (dims of p) into p's corner layout, on stream st.
-int pack_device_into_projector(rln_projector *p, const float2 *dev_plain, hipStream_t st);
+int pack_device_into_projector(rln_projector *p, const float2 *dev_plain, bool windowed, hipStream_t st);
 // Sums b's corner slots into plain [z][y][x] data (re, im) and weight volumes (dims of b) on the device, on stream st.
 int fold_backprojector_device(rln_backprojector *b, float *re, float *im, float *w, hipStream_t st);
 }  // namespace rln

@@ -12,26 +12,49 @@
 
 namespace rlnk {
 
-// Builds the corner-packed volume from the plain [z][y][x] float2 volume. One thread per base voxel.
-__global__ void __launch_bounds__(kBlock) k_pack_volume(const float2 *__restrict__ plain, VolGeom g,
-                                                        float4 *__restrict__ packed) {
-    const size_t n = (size_t)(g.xdim - 1) * (g.ydim - 1) * (g.zdim - 1);
-    const size_t idx = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (idx >= n) return;
-    const int bx = g.xdim - 1, by = g.ydim - 1;
-    const int x0 = (int)(idx % bx);
-    const size_t zy = idx / bx;
-    const int y0 = (int)(zy % by), z0 = (int)(zy / by);
-    const size_t row = (size_t)g.xdim, slab = row * (size_t)g.ydim;
-    const float2 *b = plain + (size_t)z0 * slab + (size_t)y0 * row + x0;
-    const float2 d000 = b[0], d001 = b[1], d010 = b[row], d011 = b[row + 1];
-    const float2 d100 = b[slab], d101 = b[slab + 1], d110 = b[slab + row], d111 = b[slab + row + 1];
-    float4 *o = packed + 4 * packed_index(g, x0, y0, z0);
-    o[0] = make_float4(d000.x, d000.y, d001.x, d001.y);
-    o[1] = make_float4(d010.x, d010.y, d011.x, d011.y);
-    o[2] = make_float4(d100.x, d100.y, d101.x, d101.y);
-    o[3] = make_float4(d110.x, d110.y, d111.x, d111.y);
+// Whether any base voxel of brick br lies within squared distance reach2 of the origin.
+__device__ __forceinline__ bool brick_in_reach(const VolGeom &g, int bx, int by, int bz, long long reach2) {
+    constexpr int e = (1 << kBrickLog) - 1;
+    const long long x = bx << kBrickLog;
+    const int y0 = (by << kBrickLog) + g.starty, z0 = (bz << kBrickLog) + g.startz;
+    const long long y = y0 > 0 ? y0 : y0 + e < 0 ? y0 + e : 0, z = z0 > 0 ? z0 : z0 + e < 0 ? z0 + e : 0;
+    return x * x + y * y + z * z <= reach2;
 }
+
+// Builds the corner-packed volume from the plain [z][y][x] float2 volume: four lanes per base voxel, one 16-byte quarter
+// (an x pair of corners) each, so that the stores of a wave are 1 KB of consecutive memory; kPackBricks bricks of 64
+// base voxels per block, their loads in flight together. Bricks beyond squared radius reach2, where the plain volume
+// is zero, are not read: they are cleared if clear_far, else they hold zeros already.
+// Bound by the write of the packed volume: 2.3 GB of it in reach at box 256, 0.83 ms (a thread per base voxel, whose
+// 64-byte stores lie 64 bytes apart, and every brick written: 1.85 ms).
+constexpr int kPackBricks = 4;
+__global__ void __launch_bounds__(kBlock) k_pack_volume(const float2 *__restrict__ plain, VolGeom g, long long reach2,
+                                                        int clear_far, float4 *__restrict__ packed) {
+    const int nx = brick_count(g.xdim), ny = brick_count(g.ydim), nz = brick_count(g.zdim);
+    const int base = threadIdx.x >> 2, q = threadIdx.x & 3;
+    const size_t row = (size_t)g.xdim, slab = row * (size_t)g.ydim;
+    float2 lo[kPackBricks], hi[kPackBricks];
+    bool on[kPackBricks];
+#pragma unroll
+    for (int u = 0; u < kPackBricks; ++u) {
+        const int br = blockIdx.x * kPackBricks + u;
+        const int bx = br % nx, by = (br / nx) % ny, bz = br / (nx * ny);
+        const int x0 = 4 * bx + (base & 3), y0 = 4 * by + ((base >> 2) & 3), z0 = 4 * bz + (base >> 4);
+        lo[u] = hi[u] = make_float2(0.f, 0.f);
+        const bool far = !brick_in_reach(g, bx, by, bz, reach2);
+        on[u] = bz < nz && x0 < g.xdim - 1 && y0 < g.ydim - 1 && z0 < g.zdim - 1 && (!far || clear_far);
+        if (far || !on[u]) continue;
+        const float2 *p = plain + (size_t)(z0 + (q >> 1)) * slab + (size_t)(y0 + (q & 1)) * row + x0;
+        lo[u] = p[0];
+        hi[u] = p[1];
+    }
+#pragma unroll
+    for (int u = 0; u < kPackBricks; ++u)
+        if (on[u])
+            packed[((size_t)blockIdx.x * kPackBricks + u) * kBlock + threadIdx.x] =
+                make_float4(lo[u].x, lo[u].y, hi[u].x, hi[u].y);
+}
+static_assert(kBrickLog == 2 && kBlock == 256, "k_pack_volume: 64 base voxels of 4 lanes per block");
 
 // Backprojection accumulators in corner slots: per base voxel 32 floats = one 128-byte line,
 // [re c0..c7 | im c0..c7 | weight c0..c7 | unused], corner c = 4*dz + 2*dy + dx. All 24 atomics of one
@@ -51,14 +74,9 @@ __global__ void __launch_bounds__(kBlock) k_zero_slots(float4 *__restrict__ slot
     const int nx = brick_count(g.xdim), ny = brick_count(g.ydim), nz = brick_count(g.zdim);
     const int n = nx * ny * nz;
     const long long reach = slot_reach2(g);
-    constexpr int e = (1 << kBrickLog) - 1;
     for (int br = blockIdx.x; br < n; br += gridDim.x) {
         const int bx = br % nx, by = (br / nx) % ny, bz = br / (nx * ny);
-        // the brick's base voxel nearest to the origin
-        const long long x = bx << kBrickLog;
-        const int y0 = (by << kBrickLog) + g.starty, z0 = (bz << kBrickLog) + g.startz;
-        const long long y = y0 > 0 ? y0 : y0 + e < 0 ? y0 + e : 0, z = z0 > 0 ? z0 : z0 + e < 0 ? z0 + e : 0;
-        if (x * x + y * y + z * z > reach) continue;
+        if (!brick_in_reach(g, bx, by, bz, reach)) continue;
         float4 *p = slots + (size_t)br * (kSlot / 4 << 3 * kBrickLog);
         for (int i = threadIdx.x; i < kSlot / 4 << 3 * kBrickLog; i += kBlock) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }

@@ -5,7 +5,7 @@
 //   hipFFT R2C        3-D forward transform of the padded map
 //   k_fourier_window  1/padoridim^3 and pad^3 * ori scaling, CenterFFTbySign, the r <= ROUND(pad r_max) window into
 //                     the projector's plain array, per-shell power (FP64 shared-memory bins), low-resolution cut
-//   k_pack_volume     the plain array into the bricked corner layout of the projector
+//   k_pack_volume     the plain array into the bricked corner layout of the projector, the bricks within the window
 // All three kernels stream through their volumes once (HBM-bound); the FFT is the library's.
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
@@ -156,7 +156,7 @@ extern "C" int rln_projector_compute_fourier_map(rln_projector *p, const float *
                        normfft / (double)npad, pad, nshell, d_data.as<float2>(), d_pow.as<double>(),
                        d_pow.as<double>() + nshell);
     HIP_TRY(hipGetLastError());
-    RLN_TRY(rln::pack_device_into_projector(p, d_data.as<const float2>(), st));
+    RLN_TRY(rln::pack_device_into_projector(p, d_data.as<const float2>(), true, st));
     std::vector<double> pw(2 * (size_t)nshell);
     HIP_TRY(hipMemcpyAsync(pw.data(), d_pow.ptr, sizeof(double) * 2 * nshell, hipMemcpyDeviceToHost, st));
     std::vector<float2> hd;
