@@ -243,7 +243,8 @@ int rln_estep_use_graphs(rln_estep *e, int enable);
 /* Work-unit shape of the fine diff2 kernel. The kernel splits every work item's sampled pixels into n_bands radial
  * shells of equal pixel count and runs all items' band 0, then band 1, ..., so that the gathers in flight touch one
  * shell of the reference at a time. By default (n_bands = 0) the engine times the band counts 1, 2, 4, 8, 16, 32
- * and the persistent grid sizes on its first chunk with enough work and keeps the fastest; n_bands in that set fixes
+ * and the persistent grid sizes on its first chunk with enough work (512 work items) and keeps the fastest; before
+ * that the device chooses the count for each chunk, enough bands to fill the GPU; n_bands in that set fixes
  * the band count (grid: the resident-block count) and turns the tuning off. Results do not depend on it, up to the
  * order of the FP64 sums of the bands. No counterpart in the reference, whose launch geometry is fixed
  * (src/acc/cuda/cuda_settings.h:86-141). RLN_ERR_ARG for other values. */
@@ -260,8 +261,9 @@ int rln_estep_set_fine_bands(rln_estep *e, int n_bands);
  * RLN_ERR_ARG for other values. */
 int rln_estep_set_fine_order(rln_estep *e, int order, int wsum_order);
 /* Radial pixel bands per work unit of the weighted sums and backprojection (1, 2, 4, 8, 16, 32), or 0 (the default)
- * for the fine pass's tuned count. The weighted sums accumulate into the backprojectors, so they are not timed by the
- * tuning. Results do not depend on it, up to the order of FP32 atomic sums. RLN_ERR_ARG for other values. */
+ * for the fine pass's tuned count, or, before any tuning, the device's choice for the chunk. The weighted sums
+ * accumulate into the backprojectors, so they are not timed by the tuning. Results do not depend on it, up to the
+ * order of FP32 atomic sums. RLN_ERR_ARG for other values. */
 int rln_estep_set_wsum_bands(rln_estep *e, int n_bands);
 /* Work-item shape of the fine pass (index into the shapes below), or -1 (the default) for the tuning's choice; the
  * tuning then times only the other parameters. Results do not depend on it, up to the order of FP32 partial sums.
