@@ -11,7 +11,7 @@ Headline (the learned proposal on this data): HEALPix order 3 global search.
     timed on the first --plain-particles particles (particles are independent, so particles/s carries over);
   * proposal: the pose-proposal network (64x64 input, 6 conv x 64 channels, 192 x 24 bins) trained on
     --train-samples projections of the reference with CTF and the model's noise, its top-16 bins seed the coarse
-    search (exhaustive fallback below top-1 probability 0.2), coarse cross term in split-BF16 on MFMA. Timed
+    search (exhaustive fallback below top-1 probability 0.2), split precision setting. Timed
     on all particles; the step includes the network's inference.
   Reported beside it: the miss rate (particles whose max-likelihood pose differs from the exhaustive search's)
   and the FSC between the two paths' backprojections, both over the plain subset; training time (untimed).
@@ -37,7 +37,6 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_TFLOPS = 157.3   # MI355X published FP32 peak
-PEAK_BF16_TFLOPS = 2500.0  # MI355X published dense BF16 MFMA peak
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 
 
@@ -232,7 +231,7 @@ def uneven_leg(args, n, steps, warmup):
     out = {"metric": "E-step particles/s, box 192 uneven-SNR batched fine pass", "value": round(n * steps / el, 2),
            "unit": "particles/s", "n_gpus": 1, "steps": steps, "warmup": warmup,
            "ms_per_step": round(1000 * el / steps, 2), "higher_is_better": True, "scaling": "weak",
-           "vs_baseline": None, "dtype": "bf16x3+f32", "data": "synthetic",
+           "vs_baseline": None, "dtype": "f32", "data": "synthetic",
            "config": {"workload": f"box{box} order3 global, order4 fine, {n} particles, SNR log-U[0.01,0.3]",
                       "coarse_size": coarse, "global_batch": n, "parallelism": "1 GPU"},
            "significant_coarse_poses_per_particle": {"min": int(fe.min()), "median": int(np.median(fe)),
@@ -864,8 +863,8 @@ def main():
                      for i in range(0, len(res), max(1, len(res) // 500))])
 
     # roofline of the dominant kernel of the reported path, on the algorithmic work of the E-step's cost model:
-    #   coarse diff2: F = 4 P_c N_pose FLOP (the cross term Re sum conj(X_t) CTF P, 2 FMA per complex pixel)
-    #     against FP32 peak (plain) or BF16 MFMA peak / 3 (split-BF16: hi*hi + hi*lo + lo*hi);
+    #   coarse diff2: the cross term Re sum conj(X_t) CTF P contracted over x and then y for a lattice of M positive
+    #     shifts, 8 M + 4 (2 M + 1)^2 / s FLOP per pixel and orientation, against FP32 peak;
     #   fine diff2: B_proj = 8 P N_or bytes, the complex-FP32 projections of the N_or fine orientations (8 per fine
     #     job) at the fine image size P = s (s/2 + 1), against HBM peak;
     #   weighted sums / backprojection: B_proj of the backprojected orientations plus the read-modify-write of
@@ -873,15 +872,15 @@ def main():
     # The fine pass actually gathers one 64-byte corner block of the packed reference per sampled pixel and
     # orientation; that request rate is reported beside the roofline (gather_requests).
     stage = max(("fine_diff2", "coarse_diff2", "wsum_backproject"), key=lambda k: timings[k])
-    split = is_prop or head == "local_split"
     P_f = counters["fine_pixels"]
     gather = None
     if stage == "coarse_diff2":
-        work = 4.0 * counters["coarse_poses"] * counters["coarse_pixels"]
-        bound, unit = "mfma", "TFLOP/s"
-        peak = PEAK_BF16_TFLOPS / 3.0 if split else PEAK_FP32_TFLOPS
+        M = int(cfg_g.offset_range / cfg_g.offset_step + 1e-6)
+        per = 8.0 * M + 4.0 * (2 * M + 1) ** 2 / cfg_g.coarse_size
+        work = per * counters["coarse_poses"] / ra.sampling_counts(cfg_g)[2] * counters["coarse_pixels"]
+        bound, unit, peak = "mfma", "TFLOP/s", PEAK_FP32_TFLOPS
         achieved = work / (timings[stage] * 1e-3) / 1e12
-        alg = {"flop_per_step": work, "formula": "4 * P_c * N_pose"}
+        alg = {"flop_per_step": work, "formula": "(8 M + 4 (2 M + 1)^2 / s) * P_c * N_pose / N_trans", "M": M}
     else:
         if stage == "fine_diff2":
             n_or = 8 * counters["fine_jobs"]
@@ -951,7 +950,7 @@ def main():
         "metric": "E-step particles/s, box 256 refine: plain FP32 vs proposal+split-BF16",
         "value": round(R["value"], 3), "unit": "particles/s", "n_gpus": 1, "steps": R["steps"],
         "warmup": R["warmup"], "ms_per_step": round(R["ms"], 2), "higher_is_better": True, "scaling": "weak",
-        "vs_baseline": None, "dtype": "bf16x3+f32" if split else "f32", "data": "synthetic",
+        "vs_baseline": None, "dtype": "bf16 (proposal network) + f32" if is_prop else "f32", "data": "synthetic",
         "config": {"workload": (f"refine box{box} order{order} "
                                 f"{'global search seeded by the pose proposal' if is_prop else 'local search'}"
                                 f" {n} particles"),
