@@ -321,6 +321,12 @@ int rln_coarse_image_size(int ori_size, double pixel_size, int healpix_order, do
                           int current_size);
 /* Number of directions (C1), psi angles and translations of the coarse grid. */
 int rln_sampling_counts(const rln_estep_config *cfg, int *n_dir, int *n_psi, int *n_trans);
+/* How rln_estep_run cuts n particles into chunks of at most max_particles (rln_estep_set_pool), for the largest coarse
+ * layout of the configuration: starts[0 .. n_chunks] (room for n + 1), chunk c holding particles starts[c] up to
+ * starts[c + 1]. set_offsets: [n + 1] as in rln_estep_set_orientation_sets, or null. A chunk's coarse intermediates stay
+ * within 24 GB and its orientations below 2^31 (one particle always fits). */
+int rln_estep_chunk_plan(const rln_estep_config *cfg, int n, const int *set_offsets, int max_particles, int *starts,
+                         int *n_chunks);
 /* Coarse grid: rot/tilt per direction (degrees), psi per psi index, translations (Angstrom). */
 int rln_sampling_grid(const rln_estep_config *cfg, double *rot, double *tilt, double *psi,
                       double *trans_x, double *trans_y);

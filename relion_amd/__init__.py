@@ -169,6 +169,7 @@ _SIGNATURES = {
     "rln_estep_last_counters": (C.c_int, [_vp, C.POINTER(C.c_longlong), C.c_int, _ip]),
     "rln_coarse_image_size": (C.c_int, [C.c_int, C.c_double, C.c_int, C.c_double, C.c_int]),
     "rln_sampling_counts": (C.c_int, [C.POINTER(EstepConfig), _ip, _ip, _ip]),
+    "rln_estep_chunk_plan": (C.c_int, [C.POINTER(EstepConfig), C.c_int, _ip, C.c_int, _ip, _ip]),
     "rln_sampling_grid": (C.c_int, [C.POINTER(EstepConfig), _dp, _dp, _dp, _dp, _dp]),
     "rln_sampling_local": (C.c_int, [C.POINTER(EstepConfig), C.c_double, C.c_double, C.c_double, _ip, _dp, C.c_int,
                                      _ip, _ip, _dp, C.c_int, _ip]),
@@ -306,6 +307,17 @@ def sampling_counts(cfg):
     nd, npsi, nt = C.c_int(), C.c_int(), C.c_int()
     _check(lib.rln_sampling_counts(C.byref(cfg), C.byref(nd), C.byref(npsi), C.byref(nt)))
     return nd.value, npsi.value, nt.value
+
+
+def chunk_plan(cfg, n, set_offsets=None, pool=16384):
+    """First particle of every chunk that a run of n particles is cut into, then n."""
+    starts, chunks = np.zeros(n + 1, np.int32), C.c_int()
+    off = None if set_offsets is None else np.ascontiguousarray(set_offsets, np.int32)
+    if off is not None and off.size != n + 1:
+        raise ValueError(f"set_offsets has {off.size} entries for {n} particles")
+    _check(lib.rln_estep_chunk_plan(C.byref(cfg), n, None if off is None else _ptr(off, C.c_int), pool,
+                                    _ptr(starts, C.c_int), C.byref(chunks)))
+    return starts[:chunks.value + 1].copy()
 
 
 def sampling_grid(cfg):

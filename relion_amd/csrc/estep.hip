@@ -698,8 +698,8 @@ enum PackedArray {
 // set_off/set_og (optional): explicit coarse orientation lists of the chunk's particles (global grid indices
 // idir * n_psi + ipsi, offsets relative to set_off[0]); an empty list means the exhaustive grid.
 // Two passes: sizes per particle, then every particle fills its own slices (OpenMP over particles).
-static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, ChunkHost &h,
-                             const int *set_off = nullptr, const int *set_og = nullptr) {
+static int build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, ChunkHost &h,
+                            const int *set_off = nullptr, const int *set_og = nullptr) {
     const rln_estep_config &cfg = e.cfg;
     const int K = e.K, NT = e.NT;
     // the lists of an earlier chunk are overwritten in place (no new allocation); every element of every list
@@ -731,7 +731,6 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
     auto full_grid = [&](int b) { return !cfg.local_search && n_set(b) == 0; };
     bool any_full = false;
     for (int b = 0; b < B && !any_full; ++b) any_full = full_grid(b);
-    const int n_grid = K * n_dir * n_psi;
     // pass 1: sizes
     for (int b = 0; b < B; ++b) {
         int nd, np;
@@ -747,8 +746,11 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
         }
         h.nd[b] = nd;
         h.np[b] = np;
+        if ((long long)K * nd * np > INT_MAX)
+            RLN_FAIL(RLN_ERR_MEMORY, "%d x %d x %d orientations of one particle", K, nd, np);
         h.or_cnt[b] = K * nd * np;
     }
+    const int n_grid = any_full ? K * n_dir * n_psi : 0;
     long long tot_or = any_full ? n_grid : 0, d2 = 0, tot_oc = 0, total = 0;
     for (int b = 0; b < B; ++b) total += (long long)h.or_cnt[b] * NT;
     const long long seg = rlnk::choose_segment(total);
@@ -771,6 +773,10 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
     }
     h.total_entries = d2;
     h.total_oc = tot_oc;
+    // the offsets above are 32-bit; plan_chunks bounds a chunk by its estimate, local searches can exceed theirs
+    if (tot_oc > INT_MAX || tot_or > INT_MAX)
+        RLN_FAIL(RLN_ERR_MEMORY, "%lld orientations in a chunk of %d particles: at most %d", std::max(tot_oc, tot_or), B,
+                 INT_MAX);
     // Tile placement. Global searches enumerate the same grid for every particle: the coarse tiles are ordered by
     // orientation block first, so that blocks running together read the same projection rows (L2 hits) instead
     // of each particle streaming the whole grid from HBM. Tiles of particles searched over the whole grid (all of
@@ -934,6 +940,7 @@ static void build_chunk_host(Engine &e, int B, const rln_particle_meta *meta, Ch
         h.meta_d[2 * cB + b] = h.prior_off[b];
     }
     for (int b = 0; b < B; ++b) h.meta_d[4 * (size_t)cB + b] = meta[b].highres_Xi2 / 2.;
+    return RLN_OK;
 }
 
 // Host array `which` (PackedArray) of a chunk's upload: address and bytes.
@@ -2245,34 +2252,15 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
     const bool have_sets = !set_off.empty();
     if (have_sets && (int)set_off.size() != n + 1)
         RLN_FAIL(RLN_ERR_ARG, "orientation lists were set for %d particles, run has %d", (int)set_off.size() - 1, n);
-    // chunk boundaries from a device-memory budget for the coarse intermediates (5 bytes per coarse pose: diff2 and
-    // mask; the weights are stored only with the intermediates kept, in one chunk), with per-particle pose counts: the explicit list, the whole grid, or a fraction
-    // of it for local searches
     const size_t Pf = e->igf.P;
-    const double fixed = 12.0 * e->Kc + 20.0 * Pf + 128.0 * 1024;
-    const double budget = 24.0e9;
-    std::vector<int> starts;
-    {
-        // the first chunk holds at most a quarter of the pool and at most 1,024 particles: its lists are built
-        // before any device work of the run, the later chunks' while the device runs the chunk before
-        const int first_pool = std::max(1, std::min(e->max_pool / 4, 1024));
-        double used = 0.;
-        int cnt = 0;
-        for (int i = 0; i < n; ++i) {
-            long long orients = e->cfg.local_search ? std::max(1, e->n_or / 8) : e->n_or;
-            if (have_sets && set_off[i + 1] > set_off[i]) orients = set_off[i + 1] - set_off[i];
-            const double need = 5.0 * (double)e->K * (double)orients * e->NT + fixed;
-            const int pool = starts.size() == 1 ? first_pool : e->max_pool;
-            if (cnt == 0 || (!e->keep && (used + need > budget || cnt >= pool))) {
-                starts.push_back(i);
-                used = 0.;
-                cnt = 0;
-            }
-            used += need;
-            ++cnt;
-        }
-        starts.push_back(n);
-    }
+    rln::ChunkCosts cost;
+    cost.K = e->K;
+    cost.NT = e->NT;
+    cost.orients = e->cfg.local_search ? std::max(1, e->n_or / 8) : e->n_or;
+    cost.fixed = rln::chunk_fixed_bytes(e->Kc, (long long)Pf);
+    cost.max_pool = e->max_pool;
+    cost.single = e->keep;
+    const std::vector<int> starts = rln::plan_chunks(cost, n, have_sets ? set_off.data() : nullptr);
     for (size_t c = 0; c + 1 < starts.size(); ++c) e->cap_B = std::max(e->cap_B, starts[c + 1] - starts[c]);
     // chunk c runs on the device while a second host thread builds the lists of chunk c + 1
     using clk = std::chrono::steady_clock;
@@ -2284,7 +2272,7 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
     const int n_chunks = (int)starts.size() - 1;
     if (n_chunks > 0) {
         const clk::time_point t0 = clk::now();
-        rln::build_chunk_host(*e, starts[1] - starts[0], meta, *pcur, so(0), sg(0));
+        RLN_TRY(rln::build_chunk_host(*e, starts[1] - starts[0], meta, *pcur, so(0), sg(0)));
         e->host_ms[1] = std::chrono::duration<double, std::milli>(clk::now() - t0).count();
         e->host_ms[0] += e->host_ms[1];
     }
@@ -2297,8 +2285,9 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
             // chunk c + 1 packs into the staging buffer of chunk c - 1, whose copies ended with that chunk
             builder = std::thread([&, i1, B1, c] {
                 try {
-                    rln::build_chunk_host(*e, B1, meta + i1, *pnxt, so(i1), sg(i1));
-                    if (rln::pack_chunk_host(*e, *pnxt, e->h_stage[(c + 1) & 1]) != RLN_OK) next_ok = false;
+                    if (rln::build_chunk_host(*e, B1, meta + i1, *pnxt, so(i1), sg(i1)) != RLN_OK ||
+                        rln::pack_chunk_host(*e, *pnxt, e->h_stage[(c + 1) & 1]) != RLN_OK)
+                        next_ok = false;
                 } catch (...) {
                     next_ok = false;
                 }

@@ -2,6 +2,7 @@
 #include "sampling.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 namespace rln {
@@ -351,6 +352,42 @@ void local_priors_batch(const PoseGrid &g, const rln_estep_config &cfg, const rl
                        out[i].dir_prior, out[i].psi_idx, out[i].psi_prior);
 }
 
+double chunk_fixed_bytes(long long coarse_slots, long long fine_pixels) {
+    return 12. * (double)coarse_slots + 20. * (double)fine_pixels + 128. * 1024;
+}
+
+// A budget for the coarse intermediates: per coarse pose diff2 and mask (5 bytes; the weights are stored only with the
+// intermediates kept, in one chunk), per orientation its significant count (4 bytes). At one translation a pose is an
+// orientation, and the budget alone would let the orientations of a chunk pass 2^31, beyond their 32-bit offsets.
+std::vector<int> plan_chunks(const ChunkCosts &c, int n, const int *set_off) {
+    const double budget = 24.0e9;
+    const double max_orients = (double)INT_MAX;
+    // the first chunk holds at most a quarter of the pool and at most 1,024 particles: its lists are built before any
+    // device work of the run, the later chunks' while the device runs the chunk before
+    const int first_pool = std::max(1, std::min(c.max_pool / 4, 1024));
+    const double grid = (double)c.K * (double)c.orients;  // the shared block of exhaustive particles beside the lists
+    std::vector<int> starts;
+    double used = 0., total = 0.;
+    int cnt = 0;
+    for (int i = 0; i < n; ++i) {
+        const bool list = set_off && set_off[i + 1] > set_off[i];
+        const double o = (double)c.K * (double)(list ? set_off[i + 1] - set_off[i] : c.orients);
+        const double need = o * (5. * c.NT + 4.) + c.fixed;
+        const int pool = starts.size() == 1 ? first_pool : c.max_pool;
+        const bool full = used + need > budget || cnt >= pool || total + o + (set_off ? grid : 0.) > max_orients;
+        if (cnt == 0 || (!c.single && full)) {
+            starts.push_back(i);
+            used = total = 0.;
+            cnt = 0;
+        }
+        used += need;
+        total += o;
+        ++cnt;
+    }
+    starts.push_back(n);
+    return starts;
+}
+
 }  // namespace rln
 
 // ------------------------------------------------------------------------------------------------
@@ -379,6 +416,25 @@ extern "C" int rln_sampling_counts(const rln_estep_config *cfg, int *n_dir, int 
     *n_dir = g.n_dir;
     *n_psi = g.n_psi;
     *n_trans = g.n_trans;
+    return RLN_OK;
+}
+
+extern "C" int rln_estep_chunk_plan(const rln_estep_config *cfg, int n, const int *set_offsets, int max_particles,
+                                    int *starts, int *n_chunks) {
+    rln::PoseGrid g;
+    if (!cfg || n < 0 || max_particles < 1 || !starts || !n_chunks || !g.build(*cfg))
+        RLN_FAIL(RLN_ERR_ARG, "rln_estep_chunk_plan: invalid argument");
+    const long long sc = cfg->coarse_size, sf = cfg->current_size;
+    rln::ChunkCosts c;
+    c.K = cfg->nr_classes;
+    c.NT = g.n_trans;
+    c.orients = (long long)g.n_dir * g.n_psi;
+    if (cfg->local_search) c.orients = std::max(1LL, c.orients / 8);
+    c.fixed = rln::chunk_fixed_bytes((sc / 2 + 1) * 16 * ((sc / 2 + 8) / 8), sf * (sf / 2 + 1));
+    c.max_pool = max_particles;
+    const std::vector<int> s = rln::plan_chunks(c, n, set_offsets);
+    std::copy(s.begin(), s.end(), starts);
+    *n_chunks = (int)s.size() - 1;
     return RLN_OK;
 }
 

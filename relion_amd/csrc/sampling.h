@@ -41,6 +41,20 @@ struct LocalSet {
 void local_priors_batch(const PoseGrid &g, const rln_estep_config &cfg, const rln_particle_meta *meta, int n,
                         std::vector<LocalSet> &out);
 
+// What bounds a chunk of rln_estep_run: the device memory of the coarse intermediates, the pool, and the 32-bit offsets
+// of the per-orientation state.
+struct ChunkCosts {
+    int K = 1, NT = 1;
+    long long orients = 1;  // orientations searched per class and particle (an estimate for local searches)
+    double fixed = 0.;      // bytes per particle whatever its poses (chunk_fixed_bytes)
+    int max_pool = 1;
+    bool single = false;    // one chunk whatever its size
+};
+double chunk_fixed_bytes(long long coarse_slots, long long fine_pixels);
+// First particle of every chunk, then n. set_off (optional): explicit orientation lists, [n + 1] offsets from set_off[0];
+// an empty list stands for the exhaustive grid.
+std::vector<int> plan_chunks(const ChunkCosts &c, int n, const int *set_off);
+
 // HEALPix NEST primitives (Gorski et al. 2005), as in src/Healpix_2.15a/healpix_base.cc.
 void hp_nest2xyf(int order, long long pix, int &ix, int &iy, int &face);
 long long hp_xyf2nest(int order, int ix, int iy, int face);
