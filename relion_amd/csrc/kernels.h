@@ -997,6 +997,7 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
 // 4 5.5, 8 6.5. Finding the bin in the last block of a particle instead of a launch of its own needs device-wide fences,
 // which made the first pass wait on the caches for 16 ms.
 // --------------------------------------------------------------------------------------------------
+constexpr double kWholeTail = 1. - 1e-9;  // fractions from which the weights below the threshold may hold nothing
 constexpr int kExpBins = 1088;    // binary exponents of the weights (a weight is below 2^64: the prior's mean is 1)
 constexpr int kGather = 4096;     // candidates sorted exactly
 constexpr int kSegBatch = 4;      // diff2 values a thread has in flight
@@ -1097,6 +1098,8 @@ __global__ void __launch_bounds__(kBlock) k_wpart_init(WPart *__restrict__ part,
 //   - the weights below x = (1 - f) sum / n together hold less than the (1 - f) tail, so the threshold is at least x and
 //     its bin's lower edge at least x / 2: weights below (1 - f) s / (4 n) are left out of the histogram;
 //   - weights below 2^-64 s / n, all together, do not change the FP64 sum: they are not formed.
+// Neither holds where the tail is lost in the rounding of the sums (kWholeTail): every positive weight can then be the
+// threshold, and all of them are formed and counted.
 __global__ void __launch_bounds__(kBlock) k_wseg_exp(CoarseWeightArgs a) {
     __shared__ double red[kBlock / 64];
     __shared__ unsigned int c[kExpBins];
@@ -1113,7 +1116,8 @@ __global__ void __launch_bounds__(kBlock) k_wseg_exp(CoarseWeightArgs a) {
     const double mind = (double)__uint_as_float(a.part[b].mn_bits);
     if (threadIdx.x == 0) s_seen = atomicAdd(&a.part[b].seen, 0ULL);
     __syncthreads();
-    const double n = (double)a.n_entries[b], tail = (1. - a.adaptive_fraction) / (4. * n);
+    const bool bounded = a.adaptive_fraction < kWholeTail;
+    const double n = (double)a.n_entries[b], tail = bounded ? (1. - a.adaptive_fraction) / (4. * n) : 0.;
     double sum = 0., seen = 0., hist_min = 0., cut = 1e300;
     for (SegCursor<kBlock> k(sg.begin, a.NT); k.e < sg.end;) {
         float v[kSegBatch];
@@ -1124,7 +1128,7 @@ __global__ void __launch_bounds__(kBlock) k_wseg_exp(CoarseWeightArgs a) {
         if (s > seen) {  // rare: the bounds follow the largest weight
             seen = s;
             hist_min = tail * s;
-            if (!a.weight) cut = log(a.prior_max / s * n) + 44.4;  // 2^-64 = exp(-44.36)
+            if (bounded && !a.weight) cut = log(a.prior_max / s * n) + 44.4;  // 2^-64 = exp(-44.36)
         }
 #pragma unroll
         for (int u = 0; u < kSegBatch; ++u, k.next()) {
@@ -1215,7 +1219,8 @@ __global__ void __launch_bounds__(kWBlock) k_wsel_pick(CoarseWeightArgs a) {
     }
     if (tid == 0) {
         s_p = a.part[b];
-        s_p.target = a.adaptive_fraction * s_p.sum;
+        // the whole sum is never exceeded: every positive weight is significant, whatever the sums' rounding
+        s_p.target = a.adaptive_fraction < 1. ? a.adaptive_fraction * s_p.sum : INFINITY;
         s_p.state = kSelRefine;
         if (!(s_p.sum > 0.)) {
             s_p.status = -6;  // zero or NaN sum (src/ml_optimiser.cpp:8054-8104)
@@ -1320,8 +1325,10 @@ __global__ void __launch_bounds__(kBlock) k_wsel_final(CoarseWeightArgs a) {
         }
         return;
     }
-    const bool all = state == kSelAll;
+    // a list that does not hold every entry from the crossing bin up (the histogram counted fewer) selects nothing: the
+    // particle goes by the mask, from the bin's lower edge up
     const int ncand = p.ncand, nc = min(ncand, kGather);
+    const bool all = state == kSelAll && ncand <= kGather;
     const double above_sum = all ? 0. : p.above_sum;
     if (tid == 0) s_above = 0;
     // sort size: the next power of two holding the candidates (uniform over the block), padded with -1 below every
@@ -1388,12 +1395,12 @@ __global__ void __launch_bounds__(kBlock) k_wsel_final(CoarseWeightArgs a) {
     } else {
         // all 64 bits fixed and more than kGather equal elements: the bin is one value
         thr = __longlong_as_double((long long)p.prefix);
-        long long m = (long long)floor((p.target - p.above_sum) / thr) + 1;
-        if (m < 1) m = 1;
+        const long long m = (long long)fmax(1., fmin(floor((p.target - p.above_sum) / thr) + 1., (double)ncand));
         nr_sign = p.above_cnt + m;
     }
     if (!all) {
         if (tid == 0) {
+            p.state = kSelBin;
             p.thr = thr;
             p.nr_sign = nr_sign;
             a.njobs[b] = 0;

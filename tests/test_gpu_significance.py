@@ -73,3 +73,26 @@ def test_selection_is_its_definition(kind):
             assert np.allclose(res[f], res2[f], rtol=1e-12, atol=0.0)
         else:
             assert np.array_equal(res[f], res2[f]), f
+
+
+@pytest.mark.parametrize("order,range_px,snr", [(1, 1.0, 0.3), (1, 2.5, 0.3), (2, 3.0, 0.3), (1, 2.5, 0.003)])
+def test_whole_fraction_keeps_every_positive_weight(order, range_px, snr):
+    """adaptive_fraction 1: the descending sum never exceeds the whole sum, so every pose of positive weight (up to 700
+    above the minimum) is significant, whatever the blocks saw first. One, three and many segments of 4,096 poses; few
+    and more than 4,096 poses of positive weight; with the intermediates kept and without."""
+    p = make_problem(box=32, px=4.0, order=order, offset_range_px=range_px, offset_step_px=1, n=3, snr=snr, nr_blobs=20,
+                     seed=21, fraction=1.0)
+    print(f"[whole] order {order} range {range_px} snr {snr}", flush=True)
+    es, res, _, _, _ = run_gpu(p)
+    for ip in range(3):
+        _, w, m, _ = es.coarse(ip)
+        pos = w[w > 0]
+        assert res["nr_significant"][ip] == pos.size
+        assert res["coarse_significant_weight"][ip] == pos.min()
+        assert np.array_equal(m.astype(bool), w > 0)
+        assert np.array_equal(np.unique(es.fine(ip)[0] >> 5), np.flatnonzero(w > 0))
+    for _ in range(3):
+        _, res2, _, _, _ = run_gpu(p, keep=False)
+        for f in ("coarse_significant_weight", "nr_significant", "coarse_min_diff2", "nr_fine_evaluated",
+                  "best_ihidden_over"):
+            assert np.array_equal(res[f], res2[f]), f
