@@ -50,9 +50,13 @@ enum {
     RLN_ERR_MEMORY = -7          /* device allocation failed */
 };
 
-/* Precision of the squared-difference (diff2) kernels. Both run the coarse cross term Re(P conj(CTF*s*X_t)) on the
- * FP32 matrix units with FP32 accumulation, the particle's own power in FP64; RLN_PREC_SPLIT_BF16 allows BF16 hi+lo
- * products for it, which the FP32 contraction is at least as fast as. */
+/* Precision of the coarse squared differences, formed as the particle's power plus the projection's minus twice their
+ * cross term; the projections, images and the stored diff2 are FP32 in both.
+ *   RLN_PREC_PLAIN_FP32: FP64 operands, products and sums on the FP64 matrix units, so that the difference of the large
+ *     terms keeps the accuracy of summed FP32 differences whatever the signal's power.
+ *   RLN_PREC_SPLIT_BF16: FP32 products and sums on the FP32 matrix units (at least as accurate as the BF16 hi+lo products
+ *     that the setting allows, and faster), the particle's power in FP64. The absolute error of diff2 follows the power
+ *     of the projection, about 1e-7 of it. */
 enum {
     RLN_PREC_PLAIN_FP32 = 0,
     RLN_PREC_SPLIT_BF16 = 1
@@ -381,6 +385,9 @@ double rln_ctf_value(double defU, double defV, double defAngle, double voltage, 
 /* Self-test of the MFMA lane layout the split-BF16 kernels rely on: D(16x16) = A(16x32) * B(32x16), row-major
  * float inputs rounded to BF16, one v_mfma_f32_16x16x32_bf16 on `device`. No counterpart in the reference. */
 int rln_selftest_mfma_bf16(int device, const float *A, const float *B, float *D);
+/* The same for the coarse contraction: D(16x16) = A(16x4) * B(4x16) by one v_mfma_f64_16x16x4_f64 (fp64) or
+ * v_mfma_f32_16x16x4_f32, inputs rounded to that type. */
+int rln_selftest_mfma_lattice(int device, int fp64, const double *A, const double *B, double *D);
 
 const char *rln_last_error(void);
 

@@ -179,6 +179,7 @@ _SIGNATURES = {
                                       _fp, _fp, C.POINTER(ParticleMeta), _dp, _dp]),
     "rln_ctf_value": (C.c_double, [C.c_double] * 11),
     "rln_selftest_mfma_bf16": (C.c_int, [C.c_int, _fp, _fp, _fp]),
+    "rln_selftest_mfma_lattice": (C.c_int, [C.c_int, C.c_int, _dp, _dp, _dp]),
     "rln_sampling_ang2pix": (C.c_int, [C.c_int, C.c_double, C.c_double, C.POINTER(C.c_longlong)]),
     # learned pose proposal (include/rln_proposal.h)
     "rln_proposal_create": (C.c_int, [C.c_int, C.POINTER(ProposalConfig), C.POINTER(_vp)]),
@@ -345,6 +346,16 @@ def ang2pix(order, rot, tilt):
     out = C.c_longlong()
     _check(lib.rln_sampling_ang2pix(order, float(rot), float(tilt), C.byref(out)))
     return out.value
+
+
+def selftest_mfma_lattice(A, B, fp64, device=0):
+    a, b = np.ascontiguousarray(A, np.float64), np.ascontiguousarray(B, np.float64)
+    if a.shape != (16, 4) or b.shape != (4, 16):
+        raise ValueError(f"A {a.shape}, B {b.shape}: expected (16, 4) and (4, 16)")
+    d = np.zeros((16, 16))
+    _check(lib.rln_selftest_mfma_lattice(device, int(fp64), _ptr(a, C.c_double), _ptr(b, C.c_double),
+                                         _ptr(d, C.c_double)))
+    return d
 
 
 def selftest_mfma_bf16(A, B, device=0):

@@ -400,18 +400,24 @@ static int lattice_columns(Engine &e) {
     return upload(e.d_tile_of, tile_of, e.stream);
 }
 
-// Pixel layout of the coarse contraction and its phase tables (kernels.h), from the coarse sqrt(Minvsigma2 / 2).
+// Whether the coarse contraction runs in FP64 (kernels.h, Lattice).
+static bool fp64_coarse(const Engine &e) { return e.cfg.precision == RLN_PREC_PLAIN_FP32; }
+
+// Pixel layout of the coarse contraction and its phase tables (kernels.h), from the coarse sqrt(Minvsigma2 / 2). T: the
+// arithmetic of the contraction.
+template <typename T>
 static int coarse_layout(Engine &e, const std::vector<float> &qc) {
     const int s = e.igc.s, xs = e.igc.xs, m = e.mshift;
     const double N = e.cfg.ori_size, px = e.cfg.pixel_size;
     std::vector<int2> grp, steps;
-    std::vector<float> ytab;
+    typedef typename rlnk::Lattice<T>::Pair Pair;
+    std::vector<T> ytab;
     e.n_xsteps = 0;
     // cos and -sin of 2 pi k shift / N, the phase reduced in turns before the trigonometry
     auto phase = [&](double k, double shift) {
         double turns = -k * shift / N;
         turns -= std::nearbyint(turns);
-        return make_float2((float)cos(2. * kPi * turns), (float)sin(2. * kPi * turns));
+        return std::make_pair((T)cos(2. * kPi * turns), (T)sin(2. * kPi * turns));
     };
     for (int y = 0; y <= s / 2; ++y) {
         const bool minus = y > 0 && s - y >= xs;
@@ -425,8 +431,8 @@ static int coarse_layout(Engine &e, const std::vector<float> &qc) {
             grp.push_back(make_int2(minus ? s - y : -1, 8 * j));
             steps.push_back(make_int2(64 * j, (minus ? rlnk::kStepMinus : 0) | (j + 1 == n ? rlnk::kStepEnd : 0)));
         }
-        for (int k = 0; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).x);
-        for (int k = 1; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).y);
+        for (int k = 0; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).first);
+        for (int k = 1; k <= m; ++k) ytab.push_back(phase(y, e.tr_uy[m + k] / px).second);
         e.n_xsteps = std::max(e.n_xsteps, n);
     }
     if (steps.size() & 1) {
@@ -435,17 +441,17 @@ static int coarse_layout(Engine &e, const std::vector<float> &qc) {
     }
     e.n_steps = (int)steps.size();
     e.Kc = 8 * (int)grp.size();
-    std::vector<float2> xtab((size_t)e.col_tiles * e.n_xsteps * 64);
+    std::vector<Pair> xtab((size_t)e.col_tiles * e.n_xsteps * 64);
     for (int ct = 0; ct < e.col_tiles; ++ct)
         for (int j = 0; j < e.n_xsteps; ++j)
             for (int l = 0; l < 64; ++l) {
                 const int n = l & 15, x = 8 * j + 2 * (l >> 4), k = rlnk::kColShift * ct + (n & 7) + 1;
-                float2 v = make_float2(0.f, 0.f);
+                Pair v{0, 0};
                 if (k <= m) {
-                    const float2 p0 = phase(x, e.tr_ux[m + k] / px), p1 = phase(x + 1, e.tr_ux[m + k] / px);
-                    v = n < 8 ? make_float2(p0.x, p1.x) : make_float2(p0.y, p1.y);
+                    const auto p0 = phase(x, e.tr_ux[m + k] / px), p1 = phase(x + 1, e.tr_ux[m + k] / px);
+                    v = n < 8 ? Pair{p0.first, p1.first} : Pair{p0.second, p1.second};
                 } else if (n == 7 && ct == e.col_tiles - 1) {
-                    v = make_float2(1.f, 1.f);  // tx = 0
+                    v = Pair{1, 1};  // tx = 0
                 }
                 xtab[((size_t)ct * e.n_xsteps + j) * 64 + l] = v;
             }
@@ -605,7 +611,7 @@ static int engine_model_tables(Engine &e) {
     std::vector<float> qc, qf, mw;
     q_of(e.sc, qc, nullptr);
     q_of(e.sf, qf, &mw);
-    RLN_TRY(coarse_layout(e, qc));
+    RLN_TRY(fp64_coarse(e) ? coarse_layout<double>(e, qc) : coarse_layout<float>(e, qc));
     RLN_TRY(upload(e.d_q_c, qc, e.stream));
     RLN_TRY(upload(e.d_q_f, qf, e.stream));
     // fine pixels gathered per fine orientation: non-zero Minvsigma2 inside the projection radius
@@ -1325,22 +1331,38 @@ static int run_fine_stage(Engine &e, const FineLaunch &L0) {
     return RLN_OK;
 }
 
+// The particle rows of a chunk in the contraction's layout.
+template <typename T>
+static int prep_coarse(Engine &e, int B, const float2 *dX, const float *dC, const float *d_scale) {
+    const size_t nc = (size_t)B * e.Kc;
+    RLN_TRY(e.d_wc.ensure(nc * 2 * sizeof(T)));
+    RLN_TRY(e.d_ctf2.ensure(nc * sizeof(T)));
+    RLN_TRY(e.d_ynorm.ensure(sizeof(double) * B));
+    HIP_TRY(hipMemsetAsync(e.d_ynorm.ptr, 0, sizeof(double) * B, e.stream));
+    hipLaunchKernelGGL(rlnk::k_prep_coarse<T>, dim3((std::max(e.Kc, e.igc.P) + rlnk::kBlock - 1) / rlnk::kBlock, B),
+                       dim3(rlnk::kBlock), 0, e.stream, dX, dC, d_scale, e.sf, e.igf.P, e.igc,
+                       e.d_q_c.as<const float>(), e.d_grp.as<const int2>(), e.Kc, e.cfg.do_ctf_correction,
+                       e.d_wc.as<typename rlnk::Lattice<T>::Pair>(), e.d_ctf2.as<T>(), e.d_ynorm.as<double>());
+    return launch_check("k_prep_coarse");
+}
+
+template <typename T>
 static int launch_coarse(Engine &e, unsigned n_tiles, const float *xi2, const long long *d2off) {
-    rlnk::CoarseArgs a{};
+    rlnk::CoarseArgs<T> a{};
     a.tiles = e.d_tiles.as<const rlnk::CoarseTile>();
     a.or_off = e.d_or_off.as<const int>();
     a.or_cnt = e.d_or_cnt.as<const int>();
     a.or_proj = e.d_or_proj.as<const int>();
     a.pf = e.d_pf.as<const float2>();
     a.zero_row = e.d_zero_row.as<const float2>();
-    a.w = e.d_wc.as<const float2>();
-    a.ctf2 = e.d_ctf2.as<const float>();
+    a.w = e.d_wc.as<const typename rlnk::Lattice<T>::Pair>();
+    a.ctf2 = e.d_ctf2.as<const T>();
     a.ynorm = e.d_ynorm.as<const double>();
     a.xi2half = xi2;
     a.d2_off = d2off;
     a.steps = e.d_steps.as<const int2>();
-    a.ytab = e.d_ytab.as<const float>();
-    a.xtab = e.d_xtab.as<const float2>();
+    a.ytab = e.d_ytab.as<const T>();
+    a.xtab = e.d_xtab.as<const typename rlnk::Lattice<T>::Pair>();
     a.cols = e.d_cols.as<const rlnk::CoarseColumn>();
     a.tile_of = e.col_tiles > 1 ? e.d_tile_of.as<const int>() : nullptr;
     a.n_steps = e.n_steps;
@@ -1350,11 +1372,12 @@ static int launch_coarse(Engine &e, unsigned n_tiles, const float *xi2, const lo
     a.diff2 = e.d_diff2.as<float>();
     a.part = e.d_wpart.as<rlnk::WPart>();
     const dim3 grid(n_tiles, e.col_tiles);
-    const size_t lds = sizeof(float2) * 64 * e.n_xsteps;
+    const size_t lds = 2 * sizeof(T) * 64 * e.n_xsteps;
+    void (*kernel)(rlnk::CoarseArgs<T>) = nullptr;
     switch (e.mshift) {
-#define RLN_COARSE_CASE(M)                                                                               \
-    case M:                                                                                              \
-        hipLaunchKernelGGL(rlnk::k_coarse_lattice<M>, grid, dim3(rlnk::kBlock), lds, e.stream, a);       \
+#define RLN_COARSE_CASE(M)                        \
+    case M:                                       \
+        kernel = rlnk::k_coarse_lattice<T, M>;    \
         break;
         RLN_COARSE_CASE(0) RLN_COARSE_CASE(1) RLN_COARSE_CASE(2) RLN_COARSE_CASE(3) RLN_COARSE_CASE(4)
         RLN_COARSE_CASE(5) RLN_COARSE_CASE(6) RLN_COARSE_CASE(7) RLN_COARSE_CASE(8) RLN_COARSE_CASE(9)
@@ -1362,6 +1385,11 @@ static int launch_coarse(Engine &e, unsigned n_tiles, const float *xi2, const lo
         default:
             RLN_FAIL(RLN_ERR_ARG, "translation lattice of %d shifts on an axis", 2 * e.mshift + 1);
     }
+    // beyond 64 KB with the static part (FP64, coarse sizes above 638) the kernel has to ask for its shared memory
+    if (lds > 32 * 1024)
+        HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)lds));
+    hipLaunchKernelGGL(kernel, grid, dim3(rlnk::kBlock), lds, e.stream, a);
     return launch_check("k_coarse_lattice");
 }
 
@@ -1430,16 +1458,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     const double *d_xi2d = d_old + 4 * cB;  // highres_Xi2 / 2 in FP64
 
     // coarse: particle rows in the contraction's layout
-    const size_t nc = (size_t)B * e.Kc;
-    RLN_TRY(e.d_wc.ensure(nc * sizeof(float2)));
-    RLN_TRY(e.d_ctf2.ensure(nc * sizeof(float)));
-    RLN_TRY(e.d_ynorm.ensure(sizeof(double) * B));
-    HIP_TRY(hipMemsetAsync(e.d_ynorm.ptr, 0, sizeof(double) * B, st));
-    hipLaunchKernelGGL(rlnk::k_prep_coarse, dim3((std::max(e.Kc, (int)Pc) + rlnk::kBlock - 1) / rlnk::kBlock, B),
-                       dim3(rlnk::kBlock), 0, st, dX, dC, d_scale, e.sf, (int)Pf, e.igc, e.d_q_c.as<const float>(),
-                       e.d_grp.as<const int2>(), e.Kc, cfg.do_ctf_correction, e.d_wc.as<float2>(),
-                       e.d_ctf2.as<float>(), e.d_ynorm.as<double>());
-    RLN_TRY(launch_check("k_prep_coarse"));
+    const bool f64 = fp64_coarse(e);
+    RLN_TRY(f64 ? prep_coarse<double>(e, B, dX, dC, d_scale) : prep_coarse<float>(e, B, dX, dC, d_scale));
     HIP_TRY(hipEventRecord(e.ev[kStCoarse], st));
     RLN_TRY(e.d_diff2.ensure(sizeof(float) * std::max<long long>(1, h.total_entries)));
     if (e.keep) RLN_TRY(e.d_weight.ensure(sizeof(double) * std::max<long long>(1, h.total_entries)));
@@ -1448,7 +1468,11 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     const unsigned gB = (unsigned)((B + rlnk::kBlock - 1) / rlnk::kBlock);
     RLN_TRY(e.d_wpart.ensure(sizeof(rlnk::WPart) * B));
     hipLaunchKernelGGL(rlnk::k_wpart_init, dim3(gB), dim3(rlnk::kBlock), 0, st, e.d_wpart.as<rlnk::WPart>(), B);
-    if (!h.tiles.empty()) RLN_TRY(launch_coarse(e, (unsigned)h.tiles.size(), d_xi2, d_d2off.as<const long long>()));
+    if (!h.tiles.empty()) {
+        const unsigned nt = (unsigned)h.tiles.size();
+        const long long *off = d_d2off.as<const long long>();
+        RLN_TRY(f64 ? launch_coarse<double>(e, nt, d_xi2, off) : launch_coarse<float>(e, nt, d_xi2, off));
+    }
     HIP_TRY(hipEventRecord(e.ev[kStCoarseW], st));
     RLN_TRY(e.d_stats_c.ensure(sizeof(rlnk::PassStats) * B));
     // coarse weights over segments of the poses (multi-block per particle)
@@ -2257,7 +2281,7 @@ extern "C" int rln_estep_run(rln_estep *e, int n, const float *fimg, const float
     cost.K = e->K;
     cost.NT = e->NT;
     cost.orients = e->cfg.local_search ? std::max(1, e->n_or / 8) : e->n_or;
-    cost.fixed = rln::chunk_fixed_bytes(e->Kc, (long long)Pf);
+    cost.fixed = rln::chunk_fixed_bytes(e->cfg, e->Kc, (long long)Pf);
     cost.max_pool = e->max_pool;
     cost.single = e->keep;
     const std::vector<int> starts = rln::plan_chunks(cost, n, have_sets ? set_off.data() : nullptr);
@@ -2333,6 +2357,31 @@ extern "C" int rln_selftest_mfma_bf16(int device, const float *A, const float *B
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpy(D, dD, sizeof(float) * 16 * 16, hipMemcpyDeviceToHost));
     return RLN_OK;
+}
+
+template <typename T>
+static int selftest_lattice(const double *A, const double *B, double *D) {
+    std::vector<T> ab(128), d(256);
+    std::copy(A, A + 64, ab.begin());
+    std::copy(B, B + 64, ab.begin() + 64);
+    rln::DevBuf buf;
+    RLN_TRY(buf.ensure(sizeof(T) * (128 + 256)));
+    T *dev = buf.as<T>();
+    HIP_TRY(hipMemcpy(dev, ab.data(), sizeof(T) * 128, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(rlnk::k_selftest_lattice<T>, dim3(1), dim3(64), 0, 0, dev, dev + 64, dev + 128);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpy(d.data(), dev + 128, sizeof(T) * 256, hipMemcpyDeviceToHost));
+    std::copy(d.begin(), d.end(), D);
+    return RLN_OK;
+}
+
+extern "C" int rln_selftest_mfma_lattice(int device, int fp64, const double *A, const double *B, double *D) {
+    if (!A || !B || !D) RLN_FAIL(RLN_ERR_ARG, "null argument");
+    int n = 0;
+    HIP_TRY(hipGetDeviceCount(&n));
+    if (device < 0 || device >= n) RLN_FAIL(RLN_ERR_ARG, "no HIP device %d", device);
+    HIP_TRY(hipSetDevice(device));
+    return fp64 ? selftest_lattice<double>(A, B, D) : selftest_lattice<float>(A, B, D);
 }
 
 extern "C" int rln_estep_keep_intermediates(rln_estep *e, int keep) {

@@ -222,6 +222,56 @@ __global__ void k_selftest_mfma(const float *__restrict__ A, const float *__rest
 // even. grp holds (row, x0) of every 8 slots (row -1: zeros). Kc = 16 * steps complex slots per projection.
 // --------------------------------------------------------------------------------------------------
 
+// Arithmetic of the contraction, by the precision setting.
+//   double (RLN_PREC_PLAIN_FP32): the difference of the three sums loses what they have in common, so with FP32 sums the
+//     error of diff2 follows the signal's power, where sums of squared FP32 differences follow diff2 itself. With FP64
+//     operands, products and sums the expansion is exact to FP64, and the FP32 projections, images and stored diff2 are
+//     what is left, as in the differences.
+//   float (RLN_PREC_SPLIT_BF16): FP32 products and sums, the particle's power in FP64.
+// The FP64 matrix product returns row g + 4 r in register r of lane group g, the FP32 one row 4 g + r (k_selftest_lattice).
+typedef double doublex4_t __attribute__((ext_vector_type(4)));
+// Tables read at wave-uniform addresses, in the constant address space: scalar loads, which do not queue behind the
+// projection values in flight.
+typedef const __attribute__((address_space(4))) float *UniformF;
+typedef const __attribute__((address_space(4))) double *UniformD;
+typedef const __attribute__((address_space(4))) int *UniformI;
+template <typename T>
+struct Lattice;
+template <>
+struct Lattice<float> {
+    typedef float2 Pair;
+    typedef floatx4_t Acc;
+    typedef UniformF Uniform;
+    static __device__ __forceinline__ Acc mfma(float a, float b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
+    static __device__ __forceinline__ int reg(int row) { return row & 3; }
+    static __device__ __forceinline__ int group(int row) { return row >> 2; }
+};
+template <>
+struct Lattice<double> {
+    typedef double2 Pair;
+    typedef doublex4_t Acc;
+    typedef UniformD Uniform;
+    static __device__ __forceinline__ Acc mfma(double a, double b, Acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int g, int r) { return g + 4 * r; }
+    static __device__ __forceinline__ int reg(int row) { return row >> 2; }
+    static __device__ __forceinline__ int group(int row) { return row & 3; }
+};
+
+// D (16 x 16, row-major) = A (16 x 4) B (4 x 16) by one matrix instruction of the contraction: lane l supplies row or
+// column l % 16 at k = l / 16 and receives its four rows of column l % 16.
+template <typename T>
+__global__ void k_selftest_lattice(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ D) {
+    const int l = threadIdx.x, n = l & 15, g = l >> 4;
+    typename Lattice<T>::Acc acc = {0, 0, 0, 0};
+    acc = Lattice<T>::mfma(A[n * 4 + g], B[g * 16 + n], acc);
+    for (int r = 0; r < 4; ++r) D[Lattice<T>::row(g, r) * 16 + n] = acc[r];
+}
+
 // Projections of every coarse orientation of every class in that layout: FP32 complex pf [K*n_or][Kc].
 // grid (K*n_or, ceil(Kc/256)).
 __global__ void __launch_bounds__(kBlock) k_project_grid(const float4 *const *__restrict__ vols, VolGeom vg,
@@ -242,16 +292,17 @@ __global__ void __launch_bounds__(kBlock) k_project_grid(const float4 *const *__
 }
 
 // Particle side in that layout: w[b][slot] = c_p q_p X(p), ctf2[b][slot] = c_p^2, and ynorm[b] = sum_p |q_p X(p)|^2
-// over all pixels (FP64). grid (ceil(max(Kc, P)/256), B).
+// over all pixels (summed in FP64). grid (ceil(max(Kc, P)/256), B).
+template <typename T>
 __global__ void __launch_bounds__(kBlock) k_prep_coarse(const float2 *__restrict__ fimg, const float *__restrict__ fctf,
                                                         const float *__restrict__ scale, int sf, int Pf, ImgGeom ig,
                                                         const float *__restrict__ q, const int2 *__restrict__ grp,
-                                                        int Kc, int do_ctf, float2 *__restrict__ w,
-                                                        float *__restrict__ ctf2, double *__restrict__ ynorm) {
+                                                        int Kc, int do_ctf, typename Lattice<T>::Pair *__restrict__ w,
+                                                        T *__restrict__ ctf2, double *__restrict__ ynorm) {
     __shared__ double red[kBlock / 64];
     const int idx = blockIdx.x * kBlock + threadIdx.x;
     const int b = blockIdx.y;
-    const float sc = scale[b];
+    const T sc = scale[b];
     auto src_of = [&](int i, int x) {
         const int y = (i < ig.xs) ? i : i - ig.s;
         const int isrc = (y < 0) ? y + sf : y;
@@ -260,25 +311,27 @@ __global__ void __launch_bounds__(kBlock) k_prep_coarse(const float2 *__restrict
     if (idx < Kc) {
         const int2 gr = grp[idx >> 3];
         const int x = gr.y + (idx & 7), i = gr.x;
-        float2 v = make_float2(0.f, 0.f);
-        float c2 = 0.f;
+        typename Lattice<T>::Pair v;
+        v.x = v.y = 0;
+        T c2 = 0;
         if (i >= 0 && x < ig.xs) {
             const size_t src = src_of(i, x);
-            const float qp = q[i * ig.xs + x];
-            const float c = qp * (do_ctf ? fctf[src] : 1.f) * sc;
+            const T qp = q[i * ig.xs + x];
+            const T c = qp * (T)(do_ctf ? fctf[src] : 1.f) * sc;
             const float2 X = fimg[src];
-            v = make_float2(c * qp * X.x, c * qp * X.y);
+            v.x = c * qp * (T)X.x;
+            v.y = c * qp * (T)X.y;
             c2 = c * c;
         }
         w[(size_t)b * Kc + idx] = v;
         ctf2[(size_t)b * Kc + idx] = c2;
     }
-    float yn = 0.f;
+    T yn = 0;
     if (idx < ig.P) {
         const int i = idx / ig.xs, x = idx - i * ig.xs;
-        const float qp = q[idx];
+        const T qp = q[idx];
         const float2 X = fimg[src_of(i, x)];
-        yn = qp * qp * (X.x * X.x + X.y * X.y);
+        yn = qp * qp * ((T)X.x * (T)X.x + (T)X.y * (T)X.y);
     }
     double s = yn;
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
@@ -323,19 +376,21 @@ constexpr int kColShift = 8;
 constexpr int kStepMinus = 1, kStepEnd = 2;  // the step has a row -y; it is the last of its row pair
 constexpr int kStepChunk = 64;               // steps whose particle rows are staged in LDS at a time (even)
 
+template <typename T>
 struct CoarseArgs {
+    typedef typename Lattice<T>::Pair Pair;
     const CoarseTile *tiles;
     const int *or_off, *or_cnt, *or_proj;
     const float2 *pf;         // projections [K*n_or][Kc]
     const float2 *zero_row;   // [Kc] zeros
-    const float2 *w;          // [b][Kc]
-    const float *ctf2;        // [b][Kc]
+    const Pair *w;            // [b][Kc]
+    const T *ctf2;            // [b][Kc]
     const double *ynorm;
     const float *xi2half;
     const long long *d2_off;
     const int2 *steps;        // [n_steps] (offset of the step's x phases in xtab, flags: kStepMinus | kStepEnd)
-    const float *ytab;        // per row pair: cos(2 pi y ty / N) for ty = 0 .. M, -sin for ty = 1 .. M
-    const float2 *xtab;       // [column tile][step of a row][lane]: the two x phases of the lane's column
+    const T *ytab;            // per row pair: cos(2 pi y ty / N) for ty = 0 .. M, -sin for ty = 1 .. M
+    const Pair *xtab;         // [column tile][step of a row][lane]: the two x phases of the lane's column
     const CoarseColumn *cols; // [column tile][16], then the tx = 0 column of M == 8
     const int *tile_of;       // column tile of each translation, null with one tile
     int n_steps, n_xsteps;    // n_steps even
@@ -344,45 +399,51 @@ struct CoarseArgs {
     WPart *part;
 };
 
-// Tables read at wave-uniform addresses, in the constant address space: scalar loads, which do not queue behind the
-// projection values in flight.
-typedef const __attribute__((address_space(4))) float *UniformF;
-typedef const __attribute__((address_space(4))) int *UniformI;
-
 // Value of the lane 8 further in its row of 16 lanes.
 __device__ __forceinline__ float dpp_ror8(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
 }
+__device__ __forceinline__ double dpp_ror8(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x128, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x128, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
 
 // One block per tile of 64 orientations of one particle, 16 per wave, all translations of one column tile; M: number
-// of positive shifts of the lattice. Each lane loads its row's projection values (lane l: orientation l % 16, x pairs
-// 2 (l / 16) of every 8) and forms A in registers, so that the operands of the x contraction
-// (v_mfma_f32_16x16x4_f32: lane l supplies row or column l % 16 at k = l / 16 and receives rows 4 (l / 16) .. + 3 of
-// column l % 16) go from memory to the matrix units through registers alone; the column operand is the same for every
-// row, particle and orientation. The particle's rows, shared by the block, are staged in LDS: read from memory by every
-// wave they took more of the vector memory path than the projections (busy 81% of the time). The steps alternate
-// between two register sets, the next step's loads in flight. The results leave through LDS so that whole rows are
-// stored. Bound by the FP32 matrix rate and the vector instructions that form A, about evenly.
+// of positive shifts of the lattice; T: the arithmetic (Lattice). Each lane loads its row's projection values (lane l:
+// orientation l % 16, x pairs 2 (l / 16) of every 8) and forms A in registers, so that the operands of the x contraction
+// (16x16x4 products: lane l supplies row or column l % 16 at k = l / 16) go from memory to the matrix units through
+// registers alone; the column operand is the same for every row, particle and orientation. The particle's rows, shared by
+// the block, are staged in LDS: read from memory by every wave they took more of the vector memory path than the
+// projections (busy 81% of the time). The steps alternate between two register sets, the next step's loads in flight. The
+// results leave through LDS so that whole rows are stored. Bound by the matrix rate and the vector instructions that form
+// A, about evenly.
 // The lattice form needs 4 (2 M) + 4 (2 M + 1)^2 / s flops per pixel and orientation where the direct cross term needs
 // 4 NT (113 translations, coarse size 54: 57 against 452), which is why FP32 matrix products here are faster than BF16
-// hi+lo products of the direct form, and much faster than direct squared differences on the vector units.
-// Measured (box 128, coarse size 54, 36,864 orientations x 113 translations): 101 particles 5.4 ms (81 ms with direct
-// FP32 squared differences, 7.3 ms without the staged rows), 151 particles and 4 classes 31.9 ms (63.6 ms with BF16
-// hi+lo products of the direct cross term): 79 G poses/s. Reading all LDS operands of a step at once and running the
-// missing row -y on zeros instead of a branch costs 16 registers, one wave per SIMD and 4 to 10% of the time.
+// hi+lo products of the direct form, and FP64 ones, at half the FP32 matrix rate and with twice the registers, much faster
+// than direct FP32 squared differences on the vector units.
+// Measured (box 128, coarse size 54, 36,864 orientations x 113 translations): 101 particles in FP64 9.2 ms (81 ms with
+// direct FP32 squared differences; 5.5 ms with FP32 sums, whose error is 1e-7 of the signal's power), 151 particles and 4
+// classes in FP32 30.5 ms (63.6 ms with BF16 hi+lo products of the direct cross term): 82 G poses/s. In FP32, reading all
+// LDS operands of a step at once and running the missing row -y on zeros instead of a branch costs 16 registers, one wave
+// per SIMD and 4 to 10% of the time.
 // grid (tiles, column tiles), dynamic LDS: xtab of the column tile.
-template <int M>
-__global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
+template <typename T, int M>
+__global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs<T> a) {
+    typedef Lattice<T> L;
+    typedef typename L::Pair Pair;
     constexpr bool kZero = M == kColShift;  // the tx = 0 column has no lane: summed beside the others
     constexpr int kY = 2 * M + 1;
     __shared__ union {
         struct {
-            float4 w[8 * kStepChunk];
-            float2 c[8 * kStepChunk];
+            Pair w[16 * kStepChunk];
+            Pair c[8 * kStepChunk];
         } in;
         float out[kBlock / 64][4][256];
     } lds;
-    extern __shared__ float2 s_x[];
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    Pair *s_x = reinterpret_cast<Pair *>(s_dyn);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform, and so is what follows from it
     const int n = lane & 15, g = lane >> 4;
@@ -394,93 +455,77 @@ __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
     const int og = n < n_rows ? a.or_proj[a.or_off[b] + o0 + n] : -1;
     for (int i = tid; i < a.n_xsteps * 64; i += kBlock) s_x[i] = a.xtab[(size_t)blockIdx.y * a.n_xsteps * 64 + i];
     const float4 *pr = reinterpret_cast<const float4 *>(og >= 0 ? a.pf + (size_t)og * a.Kc : a.zero_row) + g;
-    const float4 *wr = reinterpret_cast<const float4 *>(a.w + (size_t)b * a.Kc);
-    const float2 *cr = reinterpret_cast<const float2 *>(a.ctf2 + (size_t)b * a.Kc);
-    const float sgn = n < 8 ? 1.f : -1.f;
-    float cc[M + 1][4], cs[M + 1][4];  // cos and sin parts per |ty| of this lane's 4 rows (cs[0] unused)
-    float zc[M + 1], zs[M + 1];        // the tx = 0 column, this lane's share of row n
+    const Pair *wr = a.w + (size_t)b * a.Kc;
+    const Pair *cr = reinterpret_cast<const Pair *>(a.ctf2 + (size_t)b * a.Kc);
+    const T sgn = n < 8 ? 1 : -1;
+    T cc[M + 1][4], cs[M + 1][4];  // cos and sin parts per |ty| of this lane's 4 rows (cs[0] unused)
+    T zc[M + 1], zs[M + 1];        // the tx = 0 column, this lane's share of row n
 #pragma unroll
     for (int k = 0; k <= M; ++k) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) cc[k][r] = cs[k][r] = 0.f;
-        zc[k] = zs[k] = 0.f;
+        for (int r = 0; r < 4; ++r) cc[k][r] = cs[k][r] = 0;
+        zc[k] = zs[k] = 0;
     }
-    float an = 0.f;  // this lane's share of sum_p c_p^2 |P_o(p)|^2 of row n
-    floatx4_t da = {0.f, 0.f, 0.f, 0.f}, db = da, ea = da, eb = da;
-    float zpa = 0.f, zpb = 0.f, zma = 0.f, zmb = 0.f;
-    UniformF yt = (UniformF)a.ytab;
+    T an = 0;  // this lane's share of sum_p c_p^2 |P_o(p)|^2 of row n
+    typename L::Acc da = {0, 0, 0, 0}, db = da, ea = da, eb = da;
+    T zpa = 0, zpb = 0, zma = 0, zmb = 0;
+    typename L::Uniform yt = (typename L::Uniform)a.ytab;
     UniformI steps = (UniformI)a.steps;
-    auto norm = [&](const float4 &p, const float2 &c2) {
-        an = fmaf(p.x * p.x + p.y * p.y, c2.x, an);
-        an = fmaf(p.z * p.z + p.w * p.w, c2.y, an);
+    // two complex slots of one row: A = P conj(w), its products with the lane's x phases, the row's norm
+    auto half = [&](const float4 &p, int slot, const Pair &x, typename L::Acc &sa, typename L::Acc &sb, T &za, T &zb) {
+        const Pair w0 = lds.in.w[2 * slot], w1 = lds.in.w[2 * slot + 1], c2 = lds.in.c[slot];
+        const T p0 = p.x, p1 = p.y, p2 = p.z, p3 = p.w;
+        const T a0 = p0 * w0.x + p1 * w0.y, b0 = p1 * w0.x - p0 * w0.y;
+        const T a1 = p2 * w1.x + p3 * w1.y, b1 = p3 * w1.x - p2 * w1.y;
+        sa = L::mfma(a0, x.x, sa);
+        sb = L::mfma(b0, x.x, sb);
+        sa = L::mfma(a1, x.y, sa);
+        sb = L::mfma(b1, x.y, sb);
+        an = fma_t(p0 * p0 + p1 * p1, c2.x, an);
+        an = fma_t(p2 * p2 + p3 * p3, c2.y, an);
+        if (kZero) {
+            za += a0 + a1;
+            zb += b0 + b1;
+        }
     };
-    // one step: 4 float4 of complex pairs of row y (pp) and of row -y (pm); st within the staged chunk
+    // one step: a float4 (two complex slots) of row y (pp) and of row -y (pm) per lane; st within the staged chunk
     auto step = [&](const float4 &pp, const float4 &pm, int st, int xoff, int flags) {
-        const float2 x = s_x[xoff + lane];
-        {
-            const float4 w = lds.in.w[8 * st + g];
-            // A = P conj(w)
-            const float a0 = pp.x * w.x + pp.y * w.y, b0 = pp.y * w.x - pp.x * w.y;
-            const float a1 = pp.z * w.z + pp.w * w.w, b1 = pp.w * w.z - pp.z * w.w;
-            da = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, x.x, da, 0, 0, 0);
-            db = __builtin_amdgcn_mfma_f32_16x16x4f32(b0, x.x, db, 0, 0, 0);
-            da = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, x.y, da, 0, 0, 0);
-            db = __builtin_amdgcn_mfma_f32_16x16x4f32(b1, x.y, db, 0, 0, 0);
-            norm(pp, lds.in.c[8 * st + g]);
-            if (kZero) {
-                zpa += a0 + a1;
-                zpb += b0 + b1;
-            }
-        }
-        if (flags & kStepMinus) {
-            const float4 w = lds.in.w[8 * st + 4 + g];
-            const float a0 = pm.x * w.x + pm.y * w.y, b0 = pm.y * w.x - pm.x * w.y;
-            const float a1 = pm.z * w.z + pm.w * w.w, b1 = pm.w * w.z - pm.z * w.w;
-            ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, x.x, ea, 0, 0, 0);
-            eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b0, x.x, eb, 0, 0, 0);
-            ea = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, x.y, ea, 0, 0, 0);
-            eb = __builtin_amdgcn_mfma_f32_16x16x4f32(b1, x.y, eb, 0, 0, 0);
-            norm(pm, lds.in.c[8 * st + 4 + g]);
-            if (kZero) {
-                zma += a0 + a1;
-                zmb += b0 + b1;
-            }
-        }
+        const Pair x = s_x[xoff + lane];
+        half(pp, 8 * st + g, x, da, db, zpa, zpb);
+        if (flags & kStepMinus) half(pm, 8 * st + 4 + g, x, ea, eb, zma, zmb);
         if (!(flags & kStepEnd)) return;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             // cos lanes (+tx): U = Sa + Sb', V = Tb - Ta'; sin lanes (-tx): U = Sa' - Sb, V = Tb' + Ta, primes from
             // the partner lane, S and T the sum and difference of rows y and -y
-            const float su = n < 8 ? da[r] + ea[r] : db[r] + eb[r];
-            const float sv = n < 8 ? db[r] - eb[r] : da[r] - ea[r];
-            const float U = fmaf(sgn, su, dpp_ror8(su)), V = fmaf(-sgn, dpp_ror8(sv), sv);
-            cc[0][r] = fmaf(yt[0], U, cc[0][r]);
+            const T su = n < 8 ? da[r] + ea[r] : db[r] + eb[r];
+            const T sv = n < 8 ? db[r] - eb[r] : da[r] - ea[r];
+            const T U = fma_t(sgn, su, dpp_ror8(su)), V = fma_t(-sgn, dpp_ror8(sv), sv);
+            cc[0][r] = fma_t(yt[0], U, cc[0][r]);
 #pragma unroll
             for (int m = 1; m <= M; ++m) {
-                cc[m][r] = fmaf(yt[m], U, cc[m][r]);
-                cs[m][r] = fmaf(yt[M + m], V, cs[m][r]);
+                cc[m][r] = fma_t(yt[m], U, cc[m][r]);
+                cs[m][r] = fma_t(yt[M + m], V, cs[m][r]);
             }
         }
         if (kZero) {
-            const float U = zpa + zma, V = zpb - zmb;
-            zc[0] = fmaf(yt[0], U, zc[0]);
+            const T U = zpa + zma, V = zpb - zmb;
+            zc[0] = fma_t(yt[0], U, zc[0]);
 #pragma unroll
             for (int m = 1; m <= M; ++m) {
-                zc[m] = fmaf(yt[m], U, zc[m]);
-                zs[m] = fmaf(yt[M + m], V, zs[m]);
+                zc[m] = fma_t(yt[m], U, zc[m]);
+                zs[m] = fma_t(yt[M + m], V, zs[m]);
             }
-            zpa = zpb = zma = zmb = 0.f;
+            zpa = zpb = zma = zmb = 0;
         }
-        da = db = ea = eb = floatx4_t{0.f, 0.f, 0.f, 0.f};
+        da = db = ea = eb = typename L::Acc{0, 0, 0, 0};
         yt += kY;
     };
     for (int s0 = 0; s0 < a.n_steps; s0 += kStepChunk) {
         const int ns = min(kStepChunk, a.n_steps - s0);
         __syncthreads();  // the previous chunk's rows were read (and s_x is written, first time)
-        for (int i = tid; i < 8 * ns; i += kBlock) {
-            lds.in.w[i] = wr[8 * s0 + i];
-            lds.in.c[i] = cr[8 * s0 + i];
-        }
+        for (int i = tid; i < 16 * ns; i += kBlock) lds.in.w[i] = wr[16 * s0 + i];
+        for (int i = tid; i < 8 * ns; i += kBlock) lds.in.c[i] = cr[8 * s0 + i];
         __syncthreads();
         if (n_rows == 0) continue;  // uniform over the wave
         const float4 *p = pr + 8 * s0;
@@ -512,16 +557,16 @@ __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
     if (kZero) zcol = a.cols[16 * gridDim.y];
     float *out = a.diff2 + a.d2_off[b];
     float mn = 3.0e38f;  // minimum of the non-negative values written, for the weights' exponent offset
-    auto value = [&](float norm2, float cross) {
-        const float v = (float)(base + (double)(norm2 - 2.f * cross));
+    auto value = [&](T norm2, T cross) {
+        const float v = (float)(base + (double)(norm2 - 2 * cross));
         return v < 0.f ? 0.f : v;  // rounding of a match without noise; NaN stays
     };
     float (*so)[256] = lds.out[wave];
     __syncthreads();  // the staged rows were read
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        // rows 4 g + r of the four lane groups; row n of the zero column's lanes is one of them when n % 4 == r
-        const float nr = __shfl(an, 4 * g + r);
+        // the rows of register r in the four lane groups; row n of the zero column's lanes may be one of them
+        const T nr = __shfl(an, L::row(g, r));
         __syncthreads();
 #pragma unroll
         for (int m = 0; m <= M; ++m) {
@@ -529,14 +574,14 @@ __global__ void __launch_bounds__(kBlock, 2) k_coarse_lattice(CoarseArgs a) {
                 so[g][col.t0 + m] = value(nr, cc[m][r] + cs[m][r]);
                 if (m > 0) so[g][col.t0 - m] = value(nr, cc[m][r] - cs[m][r]);
             }
-            if (kZero && g == 0 && (n & 3) == r && m <= zcol.half) {
-                so[n >> 2][zcol.t0 + m] = value(an, zc[m] + zs[m]);
-                if (m > 0) so[n >> 2][zcol.t0 - m] = value(an, zc[m] - zs[m]);
+            if (kZero && g == 0 && L::reg(n) == r && m <= zcol.half) {
+                so[L::group(n)][zcol.t0 + m] = value(an, zc[m] + zs[m]);
+                if (m > 0) so[L::group(n)][zcol.t0 - m] = value(an, zc[m] - zs[m]);
             }
         }
         __syncthreads();
         for (int gg = 0; gg < 4; ++gg) {
-            const int row = 4 * gg + r;
+            const int row = L::row(gg, r);
             if (row >= n_rows) break;
             const bool off = __shfl(og, row) < 0;  // orientation or class without prior: never evaluated
             for (int t = lane; t < a.NT; t += 64) {

@@ -352,8 +352,9 @@ void local_priors_batch(const PoseGrid &g, const rln_estep_config &cfg, const rl
                        out[i].dir_prior, out[i].psi_idx, out[i].psi_prior);
 }
 
-double chunk_fixed_bytes(long long coarse_slots, long long fine_pixels) {
-    return 12. * (double)coarse_slots + 20. * (double)fine_pixels + 128. * 1024;
+double chunk_fixed_bytes(const rln_estep_config &cfg, long long coarse_slots, long long fine_pixels) {
+    const double slot = cfg.precision == RLN_PREC_PLAIN_FP32 ? 24. : 12.;  // the coarse rows are FP64 or FP32
+    return slot * (double)coarse_slots + 20. * (double)fine_pixels + 128. * 1024;
 }
 
 // A budget for the coarse intermediates: per coarse pose diff2 and mask (5 bytes; the weights are stored only with the
@@ -430,7 +431,7 @@ extern "C" int rln_estep_chunk_plan(const rln_estep_config *cfg, int n, const in
     c.NT = g.n_trans;
     c.orients = (long long)g.n_dir * g.n_psi;
     if (cfg->local_search) c.orients = std::max(1LL, c.orients / 8);
-    c.fixed = rln::chunk_fixed_bytes((sc / 2 + 1) * 16 * ((sc / 2 + 8) / 8), sf * (sf / 2 + 1));
+    c.fixed = rln::chunk_fixed_bytes(*cfg, (sc / 2 + 1) * 16 * ((sc / 2 + 8) / 8), sf * (sf / 2 + 1));
     c.max_pool = max_particles;
     const std::vector<int> s = rln::plan_chunks(c, n, set_offsets);
     std::copy(s.begin(), s.end(), starts);

@@ -50,7 +50,7 @@ struct ChunkCosts {
     int max_pool = 1;
     bool single = false;    // one chunk whatever its size
 };
-double chunk_fixed_bytes(long long coarse_slots, long long fine_pixels);
+double chunk_fixed_bytes(const rln_estep_config &cfg, long long coarse_slots, long long fine_pixels);
 // First particle of every chunk, then n. set_off (optional): explicit orientation lists, [n + 1] offsets from set_off[0];
 // an empty list stands for the exhaustive grid.
 std::vector<int> plan_chunks(const ChunkCosts &c, int n, const int *set_off);
