@@ -226,7 +226,7 @@ struct Engine {
     long long need_pairs = 0;
     int need_jobs = 0, need_small = 0, need_wide = 0;
     DevBuf d_plan, d_cp, d_items_s, d_items_w;
-    DevBuf d_wsegs, d_seg_first, d_wpart, d_hcnt, d_hsum, d_wcand, d_wcand_i, d_segbest, d_ocnt;  // coarse weights
+    DevBuf d_wsegs, d_seg_first, d_wpart, d_hcnt, d_hsum, d_refine, d_wcand, d_wcand_i, d_segbest, d_ocnt;  // coarse weights
     PinnedBuf h_stage[2];  // a chunk's lists packed for upload, alternating between consecutive chunks
     std::unique_ptr<ChunkHost> chunk_host[2];  // host lists of consecutive chunks, kept to reuse their memory
     rlnk::ChunkPtrs cp_host{};
@@ -1466,8 +1466,14 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     RLN_TRY(e.d_mask.ensure(std::max<long long>(1, h.total_entries)));
     // per-particle selection state; the coarse kernel folds the minimum diff2 into it as it writes
     const unsigned gB = (unsigned)((B + rlnk::kBlock - 1) / rlnk::kBlock);
+    const unsigned nseg = (unsigned)h.segs.size();
     RLN_TRY(e.d_wpart.ensure(sizeof(rlnk::WPart) * B));
-    hipLaunchKernelGGL(rlnk::k_wpart_init, dim3(gB), dim3(rlnk::kBlock), 0, st, e.d_wpart.as<rlnk::WPart>(), B);
+    RLN_TRY(e.d_hcnt.ensure(sizeof(unsigned int) * rlnk::kExpBins * B));
+    RLN_TRY(e.d_hsum.ensure(sizeof(double) * rlnk::kExpBins * B));
+    RLN_TRY(e.d_refine.ensure(sizeof(int) * rlnk::refine_ints(B, nseg)));
+    hipLaunchKernelGGL(rlnk::k_wpart_init, dim3(std::max(gB, 4u * std::min<unsigned>(B, 4 * e.n_cu))), dim3(rlnk::kBlock), 0,
+                       st, e.d_wpart.as<rlnk::WPart>(), B, e.d_hcnt.as<unsigned int>(), e.d_hsum.as<double>(),
+                       e.d_refine.as<int>());
     if (!h.tiles.empty()) {
         const unsigned nt = (unsigned)h.tiles.size();
         const long long *off = d_d2off.as<const long long>();
@@ -1477,18 +1483,13 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
     RLN_TRY(e.d_stats_c.ensure(sizeof(rlnk::PassStats) * B));
     // coarse weights over segments of the poses (multi-block per particle)
     {
-        const unsigned nseg = (unsigned)h.segs.size();
         RLN_TRY(upload_packed(e.d_wsegs, h, kPkSegs, st));
         RLN_TRY(upload_packed(e.d_seg_first, h, kPkSegFirst, st));
-        RLN_TRY(e.d_hcnt.ensure(sizeof(unsigned int) * rlnk::kExpBins * B));
-        RLN_TRY(e.d_hsum.ensure(sizeof(double) * rlnk::kExpBins * B));
         RLN_TRY(e.d_wcand.ensure(sizeof(double) * rlnk::kGather * B));
         RLN_TRY(e.d_wcand_i.ensure(sizeof(int) * rlnk::kGather * B));
         RLN_TRY(e.d_segbest.ensure(sizeof(rlnk::WSegBest) * nseg));
         RLN_TRY(e.d_ocnt.ensure(sizeof(int) * std::max<long long>(1, h.total_oc)));
         RLN_TRY(ensure_fine_capacity(e));
-        HIP_TRY(hipMemsetAsync(e.d_hcnt.ptr, 0, sizeof(unsigned int) * rlnk::kExpBins * B, st));
-        HIP_TRY(hipMemsetAsync(e.d_hsum.ptr, 0, sizeof(double) * rlnk::kExpBins * B, st));
         rlnk::CoarseWeightArgs wa{};
         wa.segs = e.d_wsegs.as<const rlnk::WSeg>();
         wa.seg_first = e.d_seg_first.as<const int>();
@@ -1508,6 +1509,8 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         wa.part = e.d_wpart.as<rlnk::WPart>();
         wa.hcnt = e.d_hcnt.as<unsigned int>();
         wa.hsum = e.d_hsum.as<double>();
+        wa.refine = e.d_refine.as<int>();
+        wa.n_seg = (int)nseg;
         wa.cand_w = e.d_wcand.as<double>();
         wa.cand_i = e.d_wcand_i.as<int>();
         wa.weight = e.keep ? e.d_weight.as<double>() : nullptr;
@@ -1521,10 +1524,16 @@ static int run_chunk(Engine &e, int B, const float *fimg, const float *fimgn, co
         wa.B = B;
         const dim3 blk(rlnk::kBlock);
         hipLaunchKernelGGL(rlnk::k_wseg_exp, dim3(nseg), blk, 0, st, wa);
-        hipLaunchKernelGGL(rlnk::k_wsel_pick, dim3(B), dim3(rlnk::kWBlock), 0, st, wa);
+        hipLaunchKernelGGL(rlnk::k_wsel_pick<false>, dim3(B), blk, 0, st, wa, 0);
+        // refinement of broad posteriors; the listed particles and segments are known on the device only
+        static_assert(rlnk::kRefines == 2, "refinements launched here");
+        const dim3 g_part(std::min<unsigned>(B, 1024)), g_seg(std::min<unsigned>(nseg, 8 * e.n_cu));
+        hipLaunchKernelGGL(rlnk::k_wseg_refine, g_seg, blk, 0, st, wa, 0);
+        hipLaunchKernelGGL(rlnk::k_wsel_pick<false>, g_part, blk, 0, st, wa, 1);
+        hipLaunchKernelGGL(rlnk::k_wseg_refine, g_seg, blk, 0, st, wa, 1);
+        hipLaunchKernelGGL(rlnk::k_wsel_pick<true>, g_part, dim3(rlnk::kWBlock), 0, st, wa, 2);
         hipLaunchKernelGGL(rlnk::k_wseg_gather, dim3(nseg), blk, 0, st, wa);
         hipLaunchKernelGGL(rlnk::k_wsel_final, dim3(B), blk, 0, st, wa);
-        if (wa.maxsig > 0) hipLaunchKernelGGL(rlnk::k_wsel_maxsig, dim3(B), blk, 0, st, wa);
         hipLaunchKernelGGL(rlnk::k_wseg_mask, dim3(nseg), blk, 0, st, wa);
         hipLaunchKernelGGL(rlnk::k_wsel_stats, dim3((B + rlnk::kBlock / 64 - 1) / (rlnk::kBlock / 64)), blk, 0, st, wa);
         RLN_TRY(launch_check("coarse weights"));
@@ -2092,7 +2101,7 @@ extern "C" int rln_estep_destroy(rln_estep *e) {
                            &e->d_jobs, &e->d_job_order, &e->d_chunk_job, &e->d_chunk_first, &e->d_fdiff2, &e->d_fbase, &e->d_fweight,
                            &e->d_fine_n, &e->d_nent, &e->d_foff, &e->d_shell_acc, &e->d_part_acc, &e->d_pdfc_acc, &e->d_pdfd_acc,
                            &e->d_res, &e->d_plan, &e->d_cp, &e->d_items_s, &e->d_items_w, &e->d_wsegs, &e->d_seg_first,
-                           &e->d_wpart, &e->d_hcnt, &e->d_hsum, &e->d_wcand, &e->d_wcand_i, &e->d_segbest,
+                           &e->d_wpart, &e->d_hcnt, &e->d_hsum, &e->d_refine, &e->d_wcand, &e->d_wcand_i, &e->d_segbest,
                            &e->d_ocnt};
     rln::drop_fine_graphs(*e);
     for (rln::DevBuf *b : bufs) b->release();

@@ -1028,9 +1028,11 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
 // (an exhaustive search) is spread over the whole GPU. The weights are not stored (unless they are asked for): every
 // pass forms those it needs from the FP32 diff2, 4 bytes a pose, the same FP64 expression each time.
 //   k_wseg_exp     weights' sum and a histogram of their binary exponents
-//   k_wsel_pick    the bin where the descending cumulative sum crosses the target, and its further mantissa digits while
-//                  it holds more than the candidate list (one block per particle: the poses of such a flat posterior
-//                  cost far more in the fine pass)
+//   k_wsel_pick    the crossing bin: where the descending cumulative sum exceeds the target or the count reaches the cap
+//                  (maxsig), whichever comes first
+//   k_wseg_refine  particles whose crossing bin holds more than the candidate list: a histogram of its entries' next 10
+//                  mantissa bits, over the segments of a list that the pick made (nothing to do for sharp posteriors);
+//                  then the pick again. Twice; entries alike to 20 bits are told apart by the last pick itself
 //   k_wseg_gather  candidates: every entry from the crossing bin up when they fit the list (kSelAll), else the bin's
 //                  (kSelBin)
 //   k_wsel_final   exact threshold from the sorted candidates; for kSelAll also the significant poses in order, which
@@ -1040,11 +1042,15 @@ __global__ void __launch_bounds__(kWBlock) k_weights(WeightArgs a) {
 // 2.5e9 poses 20.0 -> 5.5 ms (20 GB: 3.7 TB/s), 4.2e8 poses 3.6 -> 1.1 ms, 2,048 particles of 35,000 poses 2.2 -> 0.66
 // ms, against stored FP64 weights with 8-bit digits in a launch each. Several diff2 values a thread in flight: 1 8.8 ms,
 // 4 5.5, 8 6.5. Finding the bin in the last block of a particle instead of a launch of its own needs device-wide fences,
-// which made the first pass wait on the caches for 16 ms.
+// which made the first pass wait on the caches for 16 ms. Refining in the pick's block instead of over the segments, and
+// the cap by a radix selection of its own in one block per particle, took 82 ms for 40 particles of 4.2e6 poses, broad
+// posteriors and a cap of 500 (20.8 ms with stored weights and every digit over the segments): now 1.6 ms.
 // --------------------------------------------------------------------------------------------------
 constexpr double kWholeTail = 1. - 1e-9;  // fractions from which the weights below the threshold may hold nothing
 constexpr int kExpBins = 1088;    // binary exponents of the weights (a weight is below 2^64: the prior's mean is 1)
 constexpr int kGather = 4096;     // candidates sorted exactly
+constexpr int kDigitBits = 10, kDigitBins = 1 << kDigitBits;  // mantissa bits per refinement (at most kExpBins bins)
+constexpr int kRefines = 2;       // refinements over the segments
 constexpr int kSegBatch = 4;      // diff2 values a thread has in flight
 constexpr int kSegMin = 4096, kSegMax = 32768;  // entries per segment (choose_segment)
 
@@ -1083,8 +1089,11 @@ struct CoarseWeightArgs {
     double adaptive_fraction;
     long long maxsig;            // <= 0: none
     WPart *part;
-    unsigned int *hcnt;          // [b][kExpBins], zero before k_wseg_exp
+    unsigned int *hcnt;          // [b][kExpBins] histogram: zero before k_wseg_exp, left zero for the next refinement
     double *hsum;
+    int *refine;                 // particles and segments to refine: counts [kRefines][2], then per refinement particles
+                                 // [B] and segments [n_seg]
+    int n_seg;
     double *cand_w;              // [b][kGather] candidate weights
     int *cand_i;                 // [b][kGather] their entries; then the significant entries of kSelAll in order
     double *weight;              // out, same indexing as diff2, or null
@@ -1130,8 +1139,25 @@ __device__ __forceinline__ double coarse_weight(float v, double mind, const doub
     return (diff > 700.) ? 0. : orp[o] * trp[t] * exp(-diff);
 }
 
-__global__ void __launch_bounds__(kBlock) k_wpart_init(WPart *__restrict__ part, int B) {
+// Lists of refinement r (0, 1) within CoarseWeightArgs::refine.
+__host__ __device__ __forceinline__ long long refine_ints(long long B, long long n_seg) {
+    return 2 * kRefines + kRefines * (B + n_seg);
+}
+__device__ __forceinline__ int *refine_count(const CoarseWeightArgs &a, int r) { return a.refine + 2 * r; }
+__device__ __forceinline__ int *refine_parts(const CoarseWeightArgs &a, int r) {
+    return a.refine + 2 * kRefines + (long long)r * (a.B + a.n_seg);
+}
+__device__ __forceinline__ int *refine_segs(const CoarseWeightArgs &a, int r) { return refine_parts(a, r) + a.B; }
+
+// Particle states, histograms and refinement counts of a chunk.
+__global__ void __launch_bounds__(kBlock) k_wpart_init(WPart *__restrict__ part, int B, unsigned int *__restrict__ hcnt,
+                                                       double *__restrict__ hsum, int *__restrict__ refine) {
     const int b = blockIdx.x * kBlock + threadIdx.x;
+    for (long long i = b; i < (long long)B * kExpBins; i += (long long)gridDim.x * kBlock) {
+        hcnt[i] = 0;
+        hsum[i] = 0.;
+    }
+    if (b < 2 * kRefines) refine[b] = 0;
     if (b >= B) return;
     WPart p{};
     p.mn_bits = 0x7f800000u;  // +inf
@@ -1205,10 +1231,12 @@ __global__ void __launch_bounds__(kBlock) k_wseg_exp(CoarseWeightArgs a) {
 }
 
 // The crossing bin of one particle among nb histogram bins (digit at `shift`) by wave 0: the bin where the descending
-// cumulative sum from above_sum exceeds the target, or (rounding: the total may not exceed it) the smallest bin present.
+// cumulative sum from above_sum exceeds the target or the count from above_cnt reaches the cap, or (rounding: the total
+// may not exceed the target) the smallest bin present.
 __device__ __forceinline__ void pick_bin(const CoarseWeightArgs &a, WPart &p, const unsigned int *c, const double *sm,
                                          int nb, int shift, unsigned long long digit_mask) {
     const int lane = threadIdx.x;
+    const long long cap = a.maxsig > 0 ? a.maxsig : 0x7fffffffffffffffLL;
     double acc = p.above_sum, low_sum = 0.;
     long long cnt = p.above_cnt, low_cnt = 0;
     int low = 0;
@@ -1229,7 +1257,7 @@ __device__ __forceinline__ void pick_bin(const CoarseWeightArgs &a, WPart &p, co
                 xc += yc;
             }
         }
-        const unsigned long long hit = __ballot(ck > 0 && acc + xs > p.target);
+        const unsigned long long hit = __ballot(ck > 0 && (acc + xs > p.target || cnt + xc >= cap));
         const int q = hit ? __ffsll((long long)hit) - 1 : 63 - __clzll((long long)present);
         low = k0 - q;
         low_sum = acc + __shfl(xs - s, q);
@@ -1249,73 +1277,153 @@ __device__ __forceinline__ void pick_bin(const CoarseWeightArgs &a, WPart &p, co
     p.state = low_cnt + in_low <= kGather ? kSelAll : (in_low <= kGather || shift == 0) ? kSelBin : kSelRefine;
 }
 
-// One block per particle: the crossing exponent bin, then the crossing bins of further digits of its mantissa while the
-// bin holds more than kGather entries.
-__global__ void __launch_bounds__(kWBlock) k_wsel_pick(CoarseWeightArgs a) {
+// Histogram of the next digit (nb bins at `shift`) of one particle's entries [begin, end) that match its prefix, by a
+// block of S threads, into LDS; for kMinMax also the smallest and largest of their bit patterns.
+template <int S, bool kMinMax>
+__device__ __forceinline__ void digit_histogram(const CoarseWeightArgs &a, int b, const WPart &p, long long begin,
+                                                long long end, int shift, int nb, unsigned int *c, double *sm,
+                                                unsigned long long *mm) {
+    const float *d2 = a.diff2 + a.d2_off[b];
+    const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
+    const double mind = (double)__uint_as_float(p.mn_bits);
+    unsigned long long lo = ~0ULL, hi = 0ULL;
+    for (SegCursor<S> k(begin, a.NT); k.e < end;) {
+        float v[kSegBatch];
+#pragma unroll
+        for (int u = 0; u < kSegBatch; ++u) v[u] = k.e + u * S < end ? d2[k.e + u * S] : -1.f;
+#pragma unroll
+        for (int u = 0; u < kSegBatch; ++u, k.next()) {
+            if (!(v[u] >= 0.f) || !((double)v[u] - mind <= p.dcut)) continue;
+            const double wt = coarse_weight(v[u], mind, orp, trp, k.o, k.t);
+            const unsigned long long key = (unsigned long long)__double_as_longlong(wt);
+            if (!(wt > 0.) || (key & p.mask) != p.prefix) continue;
+            const int bin = (int)((key >> shift) & (unsigned long long)(nb - 1));
+            atomicAdd(&c[bin], 1u);
+            atomicAdd(&sm[bin], wt);
+            if (kMinMax) {
+                lo = key < lo ? key : lo;
+                hi = key > hi ? key : hi;
+            }
+        }
+    }
+    if (kMinMax && hi) {
+        atomicMin(&mm[0], lo);
+        atomicMax(&mm[1], hi);
+    }
+}
+
+// Refinement r: the histogram of the crossing bins' next kDigitBits mantissa bits, over the listed segments.
+__global__ void __launch_bounds__(kBlock) k_wseg_refine(CoarseWeightArgs a, int r) {
+    __shared__ unsigned int c[kDigitBins];
+    __shared__ double sm[kDigitBins];
+    const int n = refine_count(a, r)[1];
+    const int *list = refine_segs(a, r);
+    for (int q = blockIdx.x; q < n; q += gridDim.x) {
+        const WSeg sg = a.segs[list[q]];
+        const WPart p = a.part[sg.b];
+        for (int k = threadIdx.x; k < kDigitBins; k += kBlock) {
+            c[k] = 0;
+            sm[k] = 0.;
+        }
+        __syncthreads();
+        digit_histogram<kBlock, false>(a, sg.b, p, sg.begin, sg.end, 52 - kDigitBits * (r + 1), kDigitBins, c, sm, nullptr);
+        __syncthreads();
+        for (int k = threadIdx.x; k < kDigitBins; k += kBlock)
+            if (c[k]) {
+                atomicAdd(&a.hcnt[(size_t)sg.b * kExpBins + k], c[k]);
+                atomicAdd(&a.hsum[(size_t)sg.b * kExpBins + k], sm[k]);
+            }
+        __syncthreads();  // the next segment clears the bins
+    }
+}
+
+// The crossing bin of every particle (level 0: of the exponents, grid B) or of the particles that were refined (level
+// 1, 2: of the refined digit, any grid). Particles whose bin still holds more than kGather entries are listed for the
+// next refinement; the last level goes on by itself, one block per particle, through the remaining 32 bits, and stops
+// after one pass where they are all alike.
+template <bool kLast>
+__global__ void __launch_bounds__(kLast ? kWBlock : kBlock) k_wsel_pick(CoarseWeightArgs a, int level) {
+    constexpr int S = kLast ? kWBlock : kBlock;
     __shared__ unsigned int c[kExpBins];
     __shared__ double sm[kExpBins];
     __shared__ WPart s_p;
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const unsigned int *hc = a.hcnt + (size_t)b * kExpBins;
-    const double *hs = a.hsum + (size_t)b * kExpBins;
-    for (int k = tid; k < kExpBins; k += kWBlock) {
-        c[k] = hc[k];
-        sm[k] = hs[k];
-    }
-    if (tid == 0) {
-        s_p = a.part[b];
-        // the whole sum is never exceeded: every positive weight is significant, whatever the sums' rounding
-        s_p.target = a.adaptive_fraction < 1. ? a.adaptive_fraction * s_p.sum : INFINITY;
-        s_p.state = kSelRefine;
-        if (!(s_p.sum > 0.)) {
-            s_p.status = -6;  // zero or NaN sum (src/ml_optimiser.cpp:8054-8104)
-            s_p.state = kSelNone;
+    __shared__ unsigned long long s_mm[2];
+    __shared__ int s_slot;
+    const int tid = threadIdx.x;
+    const int n = level == 0 ? a.B : refine_count(a, level - 1)[0];
+    const int nb0 = level == 0 ? kExpBins : kDigitBins;
+    int shift = 52 - kDigitBits * level;
+    for (int q = blockIdx.x; q < n; q += gridDim.x) {
+        const int b = level == 0 ? q : refine_parts(a, level - 1)[q];
+        unsigned int *hc = a.hcnt + (size_t)b * kExpBins;
+        double *hs = a.hsum + (size_t)b * kExpBins;
+        for (int k = tid; k < nb0; k += S) {
+            c[k] = hc[k];
+            sm[k] = hs[k];
         }
-    }
-    __syncthreads();
-    if (s_p.state != kSelNone) {
-        if (tid < 64) {
+        if (tid == 0) {
+            s_p = a.part[b];
+            if (level == 0) {
+                // the whole sum is never exceeded: every positive weight is significant, whatever the sums' rounding
+                s_p.target = a.adaptive_fraction < 1. ? a.adaptive_fraction * s_p.sum : INFINITY;
+                s_p.state = kSelRefine;
+                if (!(s_p.sum > 0.)) {
+                    s_p.status = -6;  // zero or NaN sum (src/ml_optimiser.cpp:8054-8104)
+                    s_p.state = kSelNone;
+                }
+            }
+        }
+        __syncthreads();
+        if (s_p.state == kSelRefine && tid < 64) {
             WPart p = s_p;
-            pick_bin(a, p, c, sm, kExpBins, 52, 0xfffULL << 52);
+            const unsigned long long digit = level == 0 ? 0xfffULL << 52 : (unsigned long long)(kDigitBins - 1) << shift;
+            pick_bin(a, p, c, sm, nb0, shift, digit);
             if (tid == 0) s_p = p;
         }
-        const float *d2 = a.diff2 + a.d2_off[b];
-        const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
-        const double mind = (double)__uint_as_float(a.part[b].mn_bits);
-        const long long n = a.n_entries[b];
-        int shift = 52;
-        for (int digit = 0; digit < 6; ++digit) {  // 9, 9, 9, 9, 8, 8 bits of the mantissa
-            __syncthreads();
-            if (s_p.state != kSelRefine) break;
-            const int bits = digit < 4 ? 9 : 8, nb = 1 << bits;
-            shift -= bits;
-            for (int k = tid; k < nb; k += kWBlock) {
-                c[k] = 0;
-                sm[k] = 0.;
+        __syncthreads();
+        if (kLast) {
+            for (int sh = shift - 8; sh >= 0; sh -= 8) {
+                if (s_p.state != kSelRefine) break;
+                const WPart p = s_p;
+                for (int k = tid; k < 256; k += S) {
+                    c[k] = 0;
+                    sm[k] = 0.;
+                }
+                if (tid == 0) {
+                    s_mm[0] = ~0ULL;
+                    s_mm[1] = 0ULL;
+                }
+                __syncthreads();
+                digit_histogram<S, true>(a, b, p, 0, a.n_entries[b], sh, 256, c, sm, s_mm);
+                __syncthreads();
+                if (tid < 64) {
+                    WPart w = p;
+                    pick_bin(a, w, c, sm, 256, sh, 255ULL << sh);
+                    if (s_mm[0] == s_mm[1] && w.state == kSelRefine) {  // one value: all of its bits are known
+                        w.prefix = s_mm[0];
+                        w.mask = ~0ULL;
+                        w.state = kSelBin;
+                    }
+                    if (tid == 0) s_p = w;
+                }
+                __syncthreads();
             }
-            const unsigned long long prefix = s_p.prefix, mask = s_p.mask;
-            const double dcut = s_p.dcut;
-            __syncthreads();
-            for (SegCursor<kWBlock> k(0, a.NT); k.e < n; k.next()) {
-                const float v = d2[k.e];
-                if (!((double)v - mind <= dcut)) continue;
-                const double wt = coarse_weight(v, mind, orp, trp, k.o, k.t);
-                const unsigned long long key = (unsigned long long)__double_as_longlong(wt);
-                if (!(wt > 0.) || (key & mask) != prefix) continue;
-                const int bin = (int)((key >> shift) & (unsigned long long)(nb - 1));
-                atomicAdd(&c[bin], 1u);
-                atomicAdd(&sm[bin], wt);
+        } else if (s_p.state == kSelRefine) {
+            const int s0 = a.seg_first[b], ns = a.seg_first[b + 1] - s0;
+            if (tid == 0) {
+                refine_parts(a, level)[atomicAdd(refine_count(a, level), 1)] = b;
+                s_slot = atomicAdd(refine_count(a, level) + 1, ns);
+            }
+            for (int k = tid; k < kDigitBins; k += S) {
+                hc[k] = 0;
+                hs[k] = 0.;
             }
             __syncthreads();
-            if (tid < 64) {
-                WPart p = s_p;
-                pick_bin(a, p, c, sm, nb, shift, (unsigned long long)(nb - 1) << shift);
-                if (tid == 0) s_p = p;
-            }
+            for (int i = tid; i < ns; i += S) refine_segs(a, level)[s_slot + i] = s0 + i;
         }
+        if (tid == 0) a.part[b] = s_p;
+        __syncthreads();
     }
-    __syncthreads();
-    if (tid == 0) a.part[b] = s_p;
 }
 
 // Candidates into the particle's list: all entries from the crossing bin up, or the crossing bin's weights.
@@ -1433,14 +1541,16 @@ __global__ void __launch_bounds__(kBlock) k_wsel_final(CoarseWeightArgs a) {
     long long nr_sign;
     if (ncand <= kGather && nc > 0) {
         // without a crossing (rounding) the smallest element, as the reference's loop ends
-        long long rank = s_rank;
-        if (all && a.maxsig > 0 && rank + 1 > a.maxsig) rank = a.maxsig - 1;
+        const long long above = all ? 0 : p.above_cnt;
+        const long long rank = a.maxsig > 0 ? min((long long)s_rank, a.maxsig - above - 1) : s_rank;
         thr = s_w[rank];
-        nr_sign = (all ? 0 : p.above_cnt) + rank + 1;
+        nr_sign = above + rank + 1;
     } else {
         // all 64 bits fixed and more than kGather equal elements: the bin is one value
         thr = __longlong_as_double((long long)p.prefix);
-        const long long m = (long long)fmax(1., fmin(floor((p.target - p.above_sum) / thr) + 1., (double)ncand));
+        double room = ncand;
+        if (a.maxsig > 0) room = fmin(room, (double)(a.maxsig - p.above_cnt));
+        const long long m = (long long)fmax(1., fmin(floor((p.target - p.above_sum) / thr) + 1., room));
         nr_sign = p.above_cnt + m;
     }
     if (!all) {
@@ -1500,60 +1610,6 @@ __global__ void __launch_bounds__(kBlock) k_wsel_final(CoarseWeightArgs a) {
         a.stats[b] = st;
         a.npairs[b] = na;
         a.njobs[b] = n_jobs;
-    }
-}
-
-// maxsig cap (src/ml_optimiser.cpp:8147-8157) of the particles whose candidates are only the crossing bin: the
-// maxsig-th largest weight becomes the threshold. One block per capped particle, radix selection by counts over the
-// particle's entries.
-__global__ void __launch_bounds__(kBlock) k_wsel_maxsig(CoarseWeightArgs a) {
-    __shared__ unsigned int hc[256];
-    __shared__ unsigned long long s_prefix, s_mask;
-    __shared__ long long s_cnt;
-    const int b = blockIdx.x, tid = threadIdx.x;
-    WPart &p = a.part[b];
-    if (p.state != kSelBin || a.maxsig <= 0 || p.nr_sign <= a.maxsig) return;
-    const long long n = a.n_entries[b];
-    const float *d2 = a.diff2 + a.d2_off[b];
-    const double *orp = a.or_prior + a.or_off[b], *trp = a.tr_prior + (size_t)b * a.NT;
-    const double mind = (double)__uint_as_float(p.mn_bits);
-    if (tid == 0) {
-        s_prefix = 0ULL;
-        s_mask = 0ULL;
-        s_cnt = 0;
-    }
-    __syncthreads();
-    for (int shift = 56; shift >= 0; shift -= 8) {
-        hc[tid] = 0;
-        __syncthreads();
-        const unsigned long long pre = s_prefix, msk = s_mask;
-        for (SegCursor<kBlock> k(0, a.NT); k.e < n; k.next()) {
-            const double v = coarse_weight(d2[k.e], mind, orp, trp, k.o, k.t);
-            if (!(v > 0.)) continue;
-            const unsigned long long key = (unsigned long long)__double_as_longlong(v);
-            if ((key & msk) != pre) continue;
-            atomicAdd(&hc[(int)((key >> shift) & 255ULL)], 1u);
-        }
-        __syncthreads();
-        if (tid == 0) {
-            long long cnt = s_cnt;
-            int bin = 0;
-            for (int k = 255; k >= 0; --k) {
-                if (cnt + (long long)hc[k] >= a.maxsig) {
-                    bin = k;
-                    break;
-                }
-                cnt += hc[k];
-            }
-            s_cnt = cnt;
-            s_prefix |= ((unsigned long long)bin << shift);
-            s_mask |= (255ULL << shift);
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        p.thr = __longlong_as_double((long long)s_prefix);
-        p.nr_sign = a.maxsig;
     }
 }
 

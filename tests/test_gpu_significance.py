@@ -4,7 +4,8 @@ the counts and the fine pass's poses follow from it. Exact except where a cumula
 rounding of a sum (1e-12 relative), which none of these inputs does.
 
 The cases reach each state of the selection: all candidates in one list; more significant poses than the list holds
-(4,096), found by one histogram or refined digit by digit; thousands of equal weights; the rank cap in both; several
+(4,096), found by one histogram or refined digit by digit, over several segments and down to weights that differ in their
+last bits only; thousands of equal weights; the rank cap in all of them, below and above the list's length; several
 segments per particle; weights spread over hundreds of binary orders by the priors.
 """
 import numpy as np
@@ -25,11 +26,19 @@ def _problem(kind):
         return make_problem(**dict(kw, snr=0.02, maxsig=3))
     if kind == "segments":  # 864 x 81 poses: several segments of 4,096
         return make_problem(**dict(kw, order=2, offset_range_px=5, n=2))
-    p = make_problem(**dict(kw, snr=1e-3, maxsig=5000 if kind == "broad_capped" else 0))
-    if kind in ("broad", "broad_capped"):  # a model noise far above the images, flat offset priors
+    caps = dict(broad_capped=5000, broad_capped_low=300, segments_broad_capped=9000, near_equal_capped=6000,
+                equal_capped=5000)
+    if kind.startswith("segments_broad"):
+        kw.update(order=2, offset_range_px=5, n=2)
+    p = make_problem(**dict(kw, snr=1e-3, maxsig=caps.get(kind, 0)))
+    if "broad" in kind:  # a model noise far above the images, flat offset priors
         p.sigma2_noise = 100.0 * p.sigma2_noise
         p.cfg.sigma2_offset = 1e6
-    if kind == "equal":  # no reference: every diff2 of a particle is the same and the weights are the priors
+    if kind.startswith("near_equal"):  # flat priors, diff2 spread over some 1e-6: the weights share more than 20 bits
+        p.sigma2_noise = 1e8 * p.sigma2_noise
+        p.pdf_direction = np.full_like(p.pdf_direction, 1.0 / p.pdf_direction.size)
+        p.cfg.sigma2_offset = 1e14
+    if kind.startswith("equal"):  # no reference: every diff2 of a particle is the same and the weights are the priors
         p.volumes = [np.zeros_like(v) for v in p.volumes]
         p.pdf_direction = np.full_like(p.pdf_direction, 1.0 / p.pdf_direction.size)
         p.cfg.sigma2_offset = 1e6
@@ -40,7 +49,9 @@ def _problem(kind):
     return p
 
 
-@pytest.mark.parametrize("kind", ["sharp", "sharp_capped", "segments", "broad", "broad_capped", "equal", "far_prior"])
+@pytest.mark.parametrize("kind", ["sharp", "sharp_capped", "segments", "broad", "broad_capped", "broad_capped_low",
+                                  "segments_broad", "segments_broad_capped", "near_equal", "near_equal_capped", "equal",
+                                  "equal_capped", "far_prior"])
 def test_selection_is_its_definition(kind):
     p = _problem(kind)
     es, res, _, _, _ = run_gpu(p)
@@ -64,7 +75,9 @@ def test_selection_is_its_definition(kind):
         assert np.array_equal(np.unique(es.fine(ip)[0] >> 5), np.flatnonzero(sig))
         assert res["nr_fine_evaluated"][ip] == 32 * sig.sum()
         biggest = max(biggest, int(sig.sum()))
-    assert (biggest > 4096) == (kind in ("broad", "broad_capped", "equal"))
+    assert (biggest > 4096) == (("broad" in kind or "equal" in kind) and kind != "broad_capped_low")
+    if kind.startswith("near_equal"):
+        assert 0 < pos[0] / pos[-1] - 1 < 2.0 ** -20 and np.unique(pos).size > 100
     # without the intermediates kept (weights and mask not stored): the same particles' results
     _, res2, _, _, _ = run_gpu(p, keep=False)
     for f in ("coarse_significant_weight", "nr_significant", "coarse_sum_weight", "coarse_min_diff2",
