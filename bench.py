@@ -7,8 +7,9 @@ step, oversampling 1, padding 2, adaptive_fraction 0.999, *particle diameter 200
 *current_size = box. Synthetic and seeded.
 
 Headline (the learned proposal on this data): HEALPix order 3 global search.
-  * plain: the exhaustive coarse search in plain FP32 (36,864 orientations x 197 translations per particle),
-    timed on the first --plain-particles particles (particles are independent, so particles/s carries over);
+  * plain: the exhaustive coarse search in the plain setting (36,864 orientations x 197 translations per particle),
+    timed after a warm-up step (its first step allocates) on the first --plain-particles particles (particles are
+    independent, so particles/s carries over);
   * proposal: the pose-proposal network (64x64 input, 6 conv x 64 channels, 192 x 24 bins) trained on
     --train-samples projections of the reference with CTF and the model's noise, its top-16 bins seed the coarse
     search (exhaustive fallback below top-1 probability 0.2), split precision setting. Timed
@@ -16,7 +17,7 @@ Headline (the learned proposal on this data): HEALPix order 3 global search.
   Reported beside it: the miss rate (particles whose max-likelihood pose differs from the exhaustive search's)
   and the FSC between the two paths' backprojections, both over the plain subset; training time (untimed).
 Secondary (precision variant): HEALPix order 3 local search (*sigma_ang 7.5 deg, *priors = true pose + 3 deg
-noise), plain FP32 vs split-BF16 coarse pass on all particles.
+noise), plain setting (coarse contraction in FP64) vs split setting (in FP32) on all particles.
 
 Also reported (extra block): image preparation (real-space particles -> masked/unmasked transforms, power
 spectra and CTF images) on --prep-particles device-resident particles.
@@ -37,6 +38,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_TFLOPS = 157.3   # MI355X published FP32 peak
+PEAK_FP64_TFLOPS = 78.6    # MI355X published FP64 peak
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 
 
@@ -186,7 +188,7 @@ def uneven(args):
 def uneven_leg(args, n, steps, warmup):
     """Box 192, 1.2 A, 100 blobs, n particles with per-particle SNR log-uniform in [0.01, 0.3]: the
     significant-pose counts of the fine pass spread over orders of magnitude. Global HEALPix order-3 coarse
-    search (split-BF16), order-4 fine pass (oversampling 1), offsets 6 px range 2 px step; the fine pass runs
+    search (split setting), order-4 fine pass (oversampling 1), offsets 6 px range 2 px step; the fine pass runs
     from device-side plans as persistent kernels in captured graphs with autotuned work units and grids."""
     import relion_amd as ra
     from relion_amd import hipmem
@@ -246,7 +248,7 @@ def classify_leg(args, n):
     """Classification: K = 4 classes of 128^3 blob maps (60 blobs each, 30% shared), 1.5 A pixels, n particles at
     SNR 0.05 with uniform class labels, HEALPix order 3 global search over all classes (4 x 36,864 orientations),
     offsets 6 px at 1 px steps (113 translations), particle diameter 180 A (coarse 40 px): 16.7 M coarse poses per
-    particle. One timed step each of the plain-FP32 and the split-BF16 coarse pass after one warm-up."""
+    particle. One timed step each of the plain and the split setting after one warm-up."""
     import relion_amd as ra
     from relion_amd import hipmem
     box, px, order, K = 128, 1.5, 3, 4
@@ -740,7 +742,7 @@ def main():
             res, _ = es_x.run(d_img.address, d_ctf.address, meta_plain, on_device=True)
             return res
 
-        runs["plain"] = timed("plain", plain_step, n_plain, 1, 0, es_x)
+        runs["plain"] = timed("plain", plain_step, n_plain, 1, 1, es_x)
         map_plain = bp.reconstruct(box, do_map=False, skip_gridding=True)
         es_x.close()
         res_x = runs["plain"]["out"]
@@ -864,7 +866,8 @@ def main():
 
     # roofline of the dominant kernel of the reported path, on the algorithmic work of the E-step's cost model:
     #   coarse diff2: the cross term Re sum conj(X_t) CTF P contracted over x and then y for a lattice of M positive
-    #     shifts, 8 M + 4 (2 M + 1)^2 / s FLOP per pixel and orientation, against FP32 peak;
+    #     shifts, 8 M + 4 (2 M + 1)^2 / s FLOP per pixel and orientation, against the peak of the setting's data
+    #     type (plain: FP64, split: FP32);
     #   fine diff2: B_proj = 8 P N_or bytes, the complex-FP32 projections of the N_or fine orientations (8 per fine
     #     job) at the fine image size P = s (s/2 + 1), against HBM peak;
     #   weighted sums / backprojection: B_proj of the backprojected orientations plus the read-modify-write of
@@ -878,7 +881,8 @@ def main():
         M = int(cfg_g.offset_range / cfg_g.offset_step + 1e-6)
         per = 8.0 * M + 4.0 * (2 * M + 1) ** 2 / cfg_g.coarse_size
         work = per * counters["coarse_poses"] / ra.sampling_counts(cfg_g)[2] * counters["coarse_pixels"]
-        bound, unit, peak = "mfma", "TFLOP/s", PEAK_FP32_TFLOPS
+        bound, unit = "mfma", "TFLOP/s"
+        peak = PEAK_FP64_TFLOPS if head.endswith("plain") else PEAK_FP32_TFLOPS
         achieved = work / (timings[stage] * 1e-3) / 1e12
         alg = {"flop_per_step": work, "formula": "(8 M + 4 (2 M + 1)^2 / s) * P_c * N_pose / N_trans", "M": M}
     else:
@@ -954,10 +958,10 @@ def main():
         "config": {"workload": (f"refine box{box} order{order} "
                                 f"{'global search seeded by the pose proposal' if is_prop else 'local search'}"
                                 f" {n} particles"),
-                   "path": {"proposal": "proposal top-16 + split-bf16 coarse + fp32 fine",
-                            "proposal_pipelined": "proposal top-16 + split-bf16 coarse + fp32 fine; the next batch's "
-                                                  "inference and orientation lists overlap this batch's E-step",
-                            "local_split": "split-bf16 coarse + fp32 fine"}.get(head, head),
+                   "path": {"proposal": "proposal top-16 + split setting (fp32 coarse) + fp32 fine",
+                            "proposal_pipelined": "proposal top-16 + split setting (fp32 coarse) + fp32 fine; the next "
+                                                  "batch's inference and orientation lists overlap this batch's E-step",
+                            "local_split": "split setting (fp32 coarse) + fp32 fine"}.get(head, head),
                    "global_batch": n, "coarse_size": coarse, "particle_diameter_A": diameter, "parallelism": "1 GPU"},
         "roofline": roofline, "cpu_baseline": cpu,
         "stages_ms": {k: round(v, 2) for k, v in timings.items()}, "counters": counters,
