@@ -163,6 +163,11 @@ int rln_projector_init_mdl_complex(rln_projector *p, const double *data);
 int rln_projector_compute_fourier_map(rln_projector *p, const float *vol, int on_device, int ori_size,
                                       int current_size, double padding_factor, int do_gridding, int min_ires,
                                       double *power_spectrum, double *data_out);
+/* The packed volume as it lies on the device, copied to out (*bytes of it; out null: only *bytes is set): bricks of
+ * 4 x 4 x 4 trilinear base voxels (x fastest, in a brick and of the bricks; ceil((dim - 1) / 4) bricks a side), 16 floats
+ * per base voxel: re, im of its corners (z, y, x), x fastest. What lies beyond the volume's last base voxel is undefined.
+ * No counterpart in the reference, whose volume is a texture. */
+int rln_projector_get_packed(rln_projector *p, float *out, long long *bytes);
 /* AccProjector::clear() (acc_projector.h:97) + destructor. */
 int rln_projector_destroy(rln_projector *p);
 
@@ -382,7 +387,7 @@ int rln_synth_particles(const rln_synth_spec *spec, int nr_classes, double share
 double rln_ctf_value(double defU, double defV, double defAngle, double voltage, double cs, double q0,
                      double bfactor, double scale, double phase_shift, double x, double y);
 
-/* Self-test of the MFMA lane layout the split-BF16 kernels rely on: D(16x16) = A(16x32) * B(32x16), row-major
+/* Self-test of the MFMA lane layout the pose proposal's kernels rely on: D(16x16) = A(16x32) * B(32x16), row-major
  * float inputs rounded to BF16, one v_mfma_f32_16x16x32_bf16 on `device`. No counterpart in the reference. */
 int rln_selftest_mfma_bf16(int device, const float *A, const float *B, float *D);
 /* The same for the coarse contraction: D(16x16) = A(16x4) * B(4x16) by one v_mfma_f64_16x16x4_f64 (fp64) or

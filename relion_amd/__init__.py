@@ -135,6 +135,7 @@ _SIGNATURES = {
     "rln_projector_set_mdl_dim": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_double, _ip]),
     "rln_projector_init_mdl": (C.c_int, [_vp, _fp, _fp]),
     "rln_projector_init_mdl_complex": (C.c_int, [_vp, _dp]),
+    "rln_projector_get_packed": (C.c_int, [_vp, _fp, C.POINTER(C.c_longlong)]),
     "rln_projector_destroy": (C.c_int, [_vp]),
     "rln_projector_compute_fourier_map": (C.c_int, [_vp, _vp, C.c_int, C.c_int, C.c_int, C.c_double, C.c_int, C.c_int,
                                                     _dp, _dp]),
@@ -487,6 +488,16 @@ class AccProjector:
         if data is None:
             return ps
         return ps, data[..., 0] + 1j * data[..., 1]
+
+    def packed(self):
+        """The packed volume on the device, float32 [nz][ny][nx] bricks of [4][4][4] base voxels of [2][2][2] corners of
+        (re, im), z slowest throughout."""
+        n = C.c_longlong()
+        _check(lib.rln_projector_get_packed(self._h, None, C.byref(n)))
+        out = np.zeros(n.value // 4, np.float32)
+        _check(lib.rln_projector_get_packed(self._h, _ptr(out, C.c_float), C.byref(n)))
+        nx, ny, nz = ((d + 2) // 4 for d in self.dims[:3])
+        return out.reshape(nz, ny, nx, 4, 4, 4, 2, 2, 2, 2)
 
     def clear(self):
         if self._h:

@@ -1935,6 +1935,16 @@ extern "C" int rln_projector_init_mdl_complex(rln_projector *p, const double *da
     return RLN_OK;
 }
 
+extern "C" int rln_projector_get_packed(rln_projector *p, float *out, long long *bytes) {
+    if (!p || !bytes) RLN_FAIL(RLN_ERR_ARG, "rln_projector_get_packed: null argument");
+    if (!p->data.ptr) RLN_FAIL(RLN_ERR_STATE, "projector not dimensioned");
+    *bytes = (long long)(4 * sizeof(float4) * p->bases());
+    if (!out) return RLN_OK;
+    HIP_TRY(hipSetDevice(p->device));
+    HIP_TRY(hipMemcpy(out, p->data.ptr, *bytes, hipMemcpyDeviceToHost));
+    return RLN_OK;
+}
+
 extern "C" int rln_projector_destroy(rln_projector *p) {
     if (!p) return RLN_OK;
     (void)hipSetDevice(p->device);

@@ -25,7 +25,7 @@ __device__ __forceinline__ bool brick_in_reach(const VolGeom &g, int bx, int by,
 // (an x pair of corners) each, so that the stores of a wave are 1 KB of consecutive memory; kPackBricks bricks of 64
 // base voxels per block, their loads in flight together. Bricks beyond squared radius reach2, where the plain volume
 // is zero, are not read: they are cleared if clear_far, else they hold zeros already.
-// Bound by the write of the packed volume: 2.3 GB of it in reach at box 256, 0.83 ms (a thread per base voxel, whose
+// Bound by the write of the packed volume: 2.3 GB of it in reach at box 256, 0.83 to 0.93 ms (a thread per base voxel, whose
 // 64-byte stores lie 64 bytes apart, and every brick written: 1.85 ms).
 constexpr int kPackBricks = 4;
 __global__ void __launch_bounds__(kBlock) k_pack_volume(const float2 *__restrict__ plain, VolGeom g, long long reach2,
@@ -187,7 +187,7 @@ __device__ __forceinline__ bf16x8_t load_bf16x8(const unsigned short *p) {
     return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(p));
 }
 
-// Lane layout of v_mfma_f32_16x16x32_bf16 (checked by k_selftest_mfma): lane l supplies row l%16 of
+// Lane layout of v_mfma_f32_16x16x32_bf16, which the pose proposal's kernels use: lane l supplies row l%16 of
 // A and column l%16 of B, each with the 8 consecutive k = 8*(l/16) .. 8*(l/16)+7; it receives D rows
 // 4*(l/16) .. 4*(l/16)+3 of column l%16.
 __global__ void k_selftest_mfma(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ D) {
@@ -213,7 +213,7 @@ __global__ void k_selftest_mfma(const float *__restrict__ A, const float *__rest
 // cy + i sy the y phase of ty,
 //   U(y,tx) = sum_x a cx + b sx,  V(y,tx) = sum_x b cx - a sx,  cross = sum_y cy U + sy V.
 // Opposite shifts share their sums (cos is even, sin odd): the x contraction is the real matrix product of the rows a
-// and b with the columns cos(tx), sin(tx), tx > 0, on the FP32 matrix units; rows y and -y are added and subtracted
+// and b with the columns cos(tx), sin(tx), tx > 0, on the matrix units; rows y and -y are added and subtracted
 // before the y contraction, which runs in registers on each lane's tx.
 //
 // Pixel layout of that contraction: per row pair (y, -y), y = 0 .. s/2, steps of 16 complex slots: 8 consecutive x of
@@ -2360,7 +2360,7 @@ struct ChunkResult {
 };
 
 // The chunk's results in one block of memory, so that they reach the host in one copy: [B] ChunkResult, then [B][K]
-// pdf_class sums, then the plan's header. (Ten separate copies of a chunk of 8 particles took 0.33 of 1.15 ms.)
+// pdf_class sums, the shell totals (k_shell_total) and the plan's header. (Ten separate copies of a chunk of 8 particles took 0.33 of 1.15 ms.)
 __global__ void __launch_bounds__(kBlock) k_pack_results(const FinePlan *__restrict__ plan, int B, int K,
                                                          const PassStats *__restrict__ sc,
                                                          const PassStats *__restrict__ sf,

@@ -11,7 +11,7 @@ both against the FP64 oracle with the parity suite's tolerances (tests/test_gpu_
 1e-5, identical best poses except near-ties, backprojection within 1e-4), on a few particles so that the oracle
 finishes in seconds;
   * the learned proposal on box-256 data (150-blob map, 1.0 A pixels, SNR 0.03, HEALPix order 3, offsets 4 px at
-    0.5 px steps): trained on projections of the reference, it seeds the split-BF16 search of 256 particles, which
+    0.5 px steps): trained on projections of the reference, it seeds the search (split setting) of 256 particles, which
     must keep the exhaustive search's best pose for at least 99% of them.
 """
 import numpy as np

@@ -6,7 +6,7 @@ At this size the pose-independent part of a fine diff2 (the noise power sum(|q X
 than the differences between poses that the weights exponentiate; the fine kernels therefore sum only the
 pose-dependent part in FP32 and add the rest in FP64, so that the weights, and the backprojection they scale,
 keep the oracle's relative values.
-A local search in plain FP32 and an exhaustive global search in split BF16 (7.26 M coarse poses per particle), on
+A local search in plain FP32 and an exhaustive global search in the split setting (7.26 M coarse poses per particle), on
 a few particles each so that the oracle finishes in seconds."""
 import pytest
 
@@ -29,7 +29,7 @@ def test_full_size_local_search_plain():
 
 def test_full_size_global_search_split_bf16():
     import relion_amd as ra
-    print("[fullsize] box 256 exhaustive global search, split BF16, 3 particles", flush=True)
+    print("[fullsize] box 256 exhaustive global search, split setting, 3 particles", flush=True)
     p = _headline(3)
     p.cfg.precision = ra.RLN_PREC_SPLIT_BF16
     check_run(p, debug=(0,), bp_tol=1e-4)

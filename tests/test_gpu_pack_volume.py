@@ -1,7 +1,7 @@
 """Packing of a prepared reference into the projector's bricks: only the bricks within the window's radius are written,
-so a projector that held other data, one whose far bricks are known to be clear, and one packed whole from the same
-values project the same reference. The E-step's FP32 and FP64 sums over poses are in a fixed order: results are equal
-but for the posterior's floating-point atomics (1e-5)."""
+the ones beyond are cleared when they may hold something else. The packed memory is compared with the plain volume it
+stands for, bit for bit, also after other data filled the projector; and the E-step's results of projectors that got there
+by different ways are equal but for the order of floating-point atomics (1e-5), the samples' bricks being within reach."""
 import numpy as np
 import pytest
 
@@ -43,4 +43,47 @@ def test_windowed_pack_projects_the_same_reference(box, current):
         assert np.array_equal(res["best_ihidden_over"], results[0]["best_ihidden_over"])
         assert np.allclose(res["dLL"], results[0]["dLL"], rtol=1e-5)
         assert np.allclose(res["pmax"], results[0]["pmax"], rtol=1e-5)
+    pr.clear()
+
+
+def _corners(plain):
+    """[z][y][x] base voxels of [2][2][2] corners (re, im) of a plain volume [Z][Y][X]."""
+    v = np.stack([plain.real, plain.imag], -1).astype(np.float32)
+    Z, Y, X = plain.shape
+    out = np.empty((Z - 1, Y - 1, X - 1, 2, 2, 2, 2), np.float32)
+    for dz in range(2):
+        for dy in range(2):
+            for dx in range(2):
+                out[..., dz, dy, dx, :] = v[dz:Z - 1 + dz, dy:Y - 1 + dy, dx:X - 1 + dx]
+    return out
+
+
+def _bases(pr):
+    p = pr.packed()
+    nz, ny, nx = p.shape[:3]
+    p = p.transpose(0, 3, 1, 4, 2, 5, 6, 7, 8, 9).reshape(4 * nz, 4 * ny, 4 * nx, 2, 2, 2, 2)
+    X, Y, Z = pr.dims[:3]
+    return p[:Z - 1, :Y - 1, :X - 1]
+
+
+@pytest.mark.parametrize("box,current,pad", [(32, 32, 2.0), (32, 18, 2.0), (40, 26, 2.0), (48, 48, 2.0), (36, 30, 1.5),
+                                             (60, 60, 1.0)])
+def test_packed_memory_is_the_plain_volume(box, current, pad):
+    print(f"[pack] box {box} current {current} pad {pad}", flush=True)
+    rng = np.random.default_rng(box)
+    pr = ra.AccProjector(0)
+    dims = ra.volume_dims(current, pad)
+    pr.setMdlDim(*dims, pad)
+    for step in ("new", "again", "noise", "window", "window again"):
+        if step == "noise":
+            shape = (dims[2], dims[1], dims[0])
+            data = rng.normal(size=shape) + 1j * rng.normal(size=shape)
+            pr.initMdl(data)
+        else:
+            vol = rng.normal(size=(box,) * 3).astype(np.float32)
+            _, data = pr.computeFourierTransformMap(vol, current, pad, return_data=True)
+            far = np.add.outer(np.add.outer(np.arange(-(dims[2] // 2), dims[2] // 2 + 1) ** 2,
+                                            np.arange(-(dims[1] // 2), dims[1] // 2 + 1) ** 2), np.arange(dims[0]) ** 2)
+            assert not data[far > (dims[0] - 2) ** 2].any()  # the window: radius xdim - 2
+        assert np.array_equal(_bases(pr), _corners(data)), step
     pr.clear()

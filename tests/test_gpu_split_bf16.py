@@ -1,9 +1,10 @@
-"""Split-BF16 MFMA coarse pass (RLN_PREC_SPLIT_BF16) against the FP64 oracle.
+"""The split precision setting (RLN_PREC_SPLIT_BF16), whose coarse cross term is an FP32 contraction where the plain
+setting's is FP64, against the FP64 oracle, and the lane layout of the BF16 matrix instruction of the pose proposal's
+kernels.
 
-Tolerances for this path (it trades the coarse cross term's precision for MFMA throughput):
-  * coarse diff2 within 1e-5 relative of the oracle, as the plain-FP32 path (measured 1.5e-6 to 3.7e-6 on these
-    cases; the box-256 exhaustive case of tests/test_gpu_fullsize.py holds the same 1e-5); the maximum is printed;
-  * the fine pass, weights and backprojection run in the same FP32/FP64 kernels as the plain path, so the
+Tolerances of the setting:
+  * coarse diff2 within 1e-5 relative of the oracle, as the plain setting; the maximum is printed;
+  * the fine pass, weights and backprojection run in the same FP32/FP64 kernels as with the plain setting, so the
     max-likelihood poses must agree with the oracle for >= 99% of particles (all but one in these small runs)
     and the backprojected data within 1e-4 norm-wise.
 """
@@ -52,7 +53,7 @@ def test_split_bf16_estep(kind):
         ok = d2o >= 0
         assert np.array_equal(d2g >= 0, ok)
         worst = max(worst, rel(d2g[ok], d2o[ok]).max())
-    print(f"split-BF16 coarse diff2 max rel err vs FP64 oracle ({kind}): {worst:.2e}")
+    print(f"split setting: coarse diff2 max rel err vs FP64 oracle ({kind}): {worst:.2e}")
     assert worst < 1e-5
     same = rg["best_ihidden_over"] == ro["best_ihidden_over"]
     assert len(same) - same.sum() <= max(1, int(0.01 * len(same)))
@@ -60,5 +61,5 @@ def test_split_bf16_estep(kind):
     for k in range(p.cfg.nr_classes):
         re, im, w = bpg[k]
         err = np.sqrt(((re - bpd[k][..., 0]) ** 2 + (im - bpd[k][..., 1]) ** 2).sum() / (bpd[k] ** 2).sum())
-        print(f"split-BF16 class {k}: BP data rel err {err:.2e}", flush=True)
+        print(f"split setting: class {k}: BP data rel err {err:.2e}", flush=True)
         assert err <= 1e-4
