@@ -423,9 +423,9 @@ __device__ __forceinline__ double fma_t(double a, double b, double c) { return f
 // 4 NT (113 translations, coarse size 54: 57 against 452), which is why FP32 matrix products here are faster than BF16
 // hi+lo products of the direct form, and FP64 ones, at half the FP32 matrix rate and with twice the registers, much faster
 // than direct FP32 squared differences on the vector units.
-// Measured (box 128, coarse size 54, 36,864 orientations x 113 translations): 101 particles in FP64 9.2 ms (81 ms with
+// Measured (box 128, coarse size 54, 36,864 orientations x 113 translations): 101 particles in FP64 9.3 to 10.3 ms (81 ms with
 // direct FP32 squared differences; 5.5 ms with FP32 sums, whose error is 1e-7 of the signal's power), 151 particles and 4
-// classes in FP32 30.5 ms (63.6 ms with BF16 hi+lo products of the direct cross term): 82 G poses/s. In FP32, reading all
+// classes in FP32 30.6 to 31.5 ms (63.6 ms with BF16 hi+lo products of the direct cross term): 81 G poses/s. In FP32, reading all
 // LDS operands of a step at once and running the missing row -y on zeros instead of a branch costs 16 registers, one wave
 // per SIMD and 4 to 10% of the time.
 // grid (tiles, column tiles), dynamic LDS: xtab of the column tile.
