@@ -58,6 +58,17 @@ def test_coarse_diff2_lattices(shifts, box, px, order, diameter, extra, precisio
     assert np.array_equal(rg["best_ihidden_over"], ro["best_ihidden_over"])
 
 
+def test_coarse_diff2_of_a_perfect_match_stays_evaluated():
+    """A noise-free particle at a grid pose: its diff2 is zero up to rounding and must not turn negative, which marks
+    poses that were never evaluated."""
+    p = make_problem(box=32, px=4.0, order=1, offset_range_px=2, offset_step_px=1, n=2, snr=1e9, nr_blobs=20, seed=5)
+    p.sigma2_noise = np.full(17, 1e-4 * float(np.mean(p.fimg.astype(np.float64) ** 2)))
+    es, _, _, _, _ = run_gpu(p)
+    for ip in range(2):
+        d2 = es.coarse(ip)[0]
+        assert (d2 >= 0).all()
+
+
 def _particles_at_grid_poses(shifts, ratio, n=2):
     """Projections of the reference at coarse poses, with noise of 1 / ratio of their mean power and that noise as the
     model's: the differences of the true poses hold only the noise."""
